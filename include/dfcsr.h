@@ -105,8 +105,9 @@ int dfcsr_beam_statistics(const double *x, const double *px, const double *y, co
 /* ---- a3: cloud-in-cell deposition ----------------------------------------
  * Replaces histogram_cic_2d (deposit.py:42-87): hist[i1][i2] += w*S1*S2 over
  * the four CIC corners with cell = (q - start) * (1/((end - start)/nbins)).
- * w == NULL means unit weights.  Sums are accumulated as 64-bit fixed point
- * (scale 2^k, k chosen from n * max|w|) so the result is bit-reproducible.
+ * w == NULL means unit weights; a weight that is not finite deposits
+ * nothing.  Sums are accumulated as two words of 64-bit fixed point (scale
+ * chosen from n and max|w|) so the result is bit-reproducible.
  * Optional outputs (NULL to skip): cell_index[2*p + {0,1}] = the particle's
  * lower cell (i1, i2) (floor, may lie off the grid); cell_count[i1][i2] =
  * number of particles whose lower cell is (i1, i2) on the grid. */

@@ -1,28 +1,28 @@
-// a3: cloud-in-cell deposition with two-word fixed-point atomics.
+// a3: cloud-in-cell deposition with two-word fixed-point sums.
 //
 // Replaces histogram_cic_2d (deposit.py:42-87) and the pair of calls in
 // DF_tracker.get_DF (deposit.py:172-182).  Cell indices use the reference's
 // FP64 expression cell = (q - start) * (1 / ((end - start) / nbins)),
 // i = floor(cell), S = 1 - (cell - i), evaluated without fused multiply-add
 // so they are bit-identical to the reference.  Each corner weight w*S1*S2 is
-// scaled by 2^k and split into a signed high word (multiples of 2^32) and an
-// unsigned low word (< 2^32, rounded); both are summed with 64-bit integer
-// atomics.  Integer addition is associative, so the grid is the same for
-// every launch order, and with k chosen from n * max|w| (n*max|w|*2^k < 2^94)
-// no word can overflow while the quantum 2^-k is ~1e-22 of the largest
-// weight: the sums are exact to far below float64 rounding.
+// split into two signed integers, its multiple of 2^-k and the remainder's
+// multiple of 2^-(k + d), and both are summed as 64-bit integers.  Integer
+// addition is associative, so the grid is the same for every launch order;
+// k and d are chosen from n and max|w| so that no word can overflow, and the
+// quantum 2^-(k + d) is 1e-22 or less of the largest weight (1e7 particles):
+// the sums are exact to far below float64 rounding.
 #include "common.h"
 
 namespace dfcsr {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kMaxBlocks = 2048;
+constexpr int kMaxBlocks = 512;
 
-// ws layout: [0] scale for grid A, [1] scale for grid B (doubles),
+// ws layout: [0..3] k and d of grid A, then of grid B (as doubles),
 //            [8 .. 8+kMaxBlocks) block max|w| partials,
-//            then per grid (A, B): nb1*nb2 int64 high words and nb1*nb2
-//            uint64 low words.
+//            then the words: per workgroup of the LDS form its tile's high
+//            and low words, or (direct form) per grid nb1*nb2 of each.
 constexpr int kHdr = 8 + kMaxBlocks;
 
 int nblocks_for(int64_t n) {
@@ -32,230 +32,413 @@ int nblocks_for(int64_t n) {
   return (int)b;
 }
 
+// max|w| over the finite weights (a weight that is not finite deposits
+// nothing).  Four loads in flight per thread: 80 MB in 13 us.
 __global__ __launch_bounds__(kThreads) void absmax_partial(const double *__restrict__ w, int64_t n,
                                                            double *__restrict__ part) {
   __shared__ double red[kThreads / 64];
   double m = 0.0;
-  int64_t stride = (int64_t)gridDim.x * kThreads;
-  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride)
-    m = fmax(m, fabs(w[i]));
+  const int64_t stride = (int64_t)gridDim.x * kThreads;
+  int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  for (; i + 3 * stride < n; i += 4 * stride) {
+    double v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = fabs(w[i + k * stride]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) m = v[k] < INFINITY ? fmax(m, v[k]) : m;
+  }
+  for (; i < n; i += stride) {
+    const double v = fabs(w[i]);
+    m = v < INFINITY ? fmax(m, v) : m;
+  }
   m = block_max(m, red);
   if (threadIdx.x == 0) part[blockIdx.x] = m;
 }
 
-// Picks 2^k with n*max|w|*2^k < 2^94: every scaled weight s has |s| < 2^94/n,
-// so n high words (|s|/2^32 each) stay below 2^62 and n low words (< 2^32
-// each, n < 2^31) below 2^63.  scale[0]: unit weights, scale[1]: w.
-__device__ double pick_scale(double bound) {
-  if (!(bound > 0.0) || !isfinite(bound)) return ldexp(1.0, 60);
-  int e;
-  frexp(bound, &e);   // bound < 2^e
-  int k = 94 - e;
-  if (k > 900) k = 900;
-  return ldexp(1.0, k);
+// Fixed-point format of one grid.  A weight v is s = v 2^k = hi + r with
+// hi = rint(s), |r| <= 1/2, and lo = rint(r 2^d).  n max|w| 2^k < 2^62 keeps
+// the sum of n high words in 63 bits, n 2^(d-1) < 2^61 that of the low ones;
+// |s| < 2^50 and d <= 50 let the conversions add 1.5 2^52 and read the
+// integer from the mantissa (4 operations a word, against about 15 for a
+// float64 -> int64 conversion).
+struct FxScale {
+  int k, d;
+  double up, up_lo;   // 2^k, 2^d
+};
+
+__device__ inline FxScale fx_scale(double max_w, int64_t n) {
+  FxScale f;
+  int e = 0, en = 0;
+  frexp((double)(n < 1 ? 1 : n), &en);   // n < 2^en
+  if (max_w > 0.0) frexp(max_w, &e);     // max|w| < 2^e
+  f.k = min(62 - e - en, 50 - e);
+  f.k = max_w > 0.0 ? min(f.k, 900) : 0;
+  f.d = min(62 - en, 50);
+  f.up = ldexp(1.0, f.k);
+  f.up_lo = ldexp(1.0, f.d);
+  return f;
 }
 
-__global__ void scale_final(const double *__restrict__ part, int nblk, int64_t n, int has_w,
-                            double *__restrict__ scale) {
-  __shared__ double red[kThreads / 64];
+struct FxWords {
+  long long hi, lo;
+};
+
+__device__ inline FxWords fx_words(double v, const FxScale &f) {
+#pragma clang fp contract(off)
+  constexpr double M = 0x1.8p52;
+  const double s = v * f.up;      // exact: a power of two
+  const double h = s + M;
+  const double r = s - (h - M);   // exact
+  const double l = r * f.up_lo + M;
+  FxWords w;
+  w.hi = __double_as_longlong(h) - __double_as_longlong(M);
+  w.lo = __double_as_longlong(l) - __double_as_longlong(M);
+  return w;
+}
+
+// (hi + lo 2^-d) 2^-k with one rounding: hi's halves are exact float64s.
+__device__ inline double fx_value(long long hi, long long lo, const FxScale &f) {
+  const double hh = (double)(hi >> 32) * 0x1p32, hl = (double)(hi & 0xffffffffll);
+  const double l = (double)lo * (1.0 / f.up_lo);
+  return (hh + (hl + l)) * (1.0 / f.up);
+}
+
+// Block reduction of the max|w| partials (0 without a weight).
+__device__ inline double max_weight(const double *part, int npart, double *red) {
   double m = 0.0;
-  if (has_w)
-    for (int b = threadIdx.x; b < nblk; b += blockDim.x) m = fmax(m, part[b]);
-  m = block_max(m, red);
-  if (threadIdx.x == 0) {
-    scale[0] = pick_scale((double)n);
-    scale[1] = pick_scale((double)n * m);
+  for (int b = threadIdx.x; b < npart; b += blockDim.x) m = fmax(m, part[b]);
+  return block_max(m, red);
+}
+
+__global__ __launch_bounds__(kThreads) void zero_i64(int64_t *__restrict__ a, int64_t n) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) a[i] = 0;
+}
+
+// Cell of one particle along an axis: floor index (or -8 when far off the
+// grid: only to fail the range tests) and the lower corner's weight.
+struct CicAxis {
+  int i;
+  double S;
+};
+
+__device__ inline CicAxis cic_axis(double q, double start, double inv, int nb) {
+#pragma clang fp contract(off)
+  const double c = (q - start) * inv;
+  const double f = floor(c);
+  CicAxis a;
+  a.i = (f > -4.0 && f < (double)nb + 4.0) ? (int)f : -8;
+  a.S = 1.0 - (c - f);
+  return a;
+}
+
+// A weight that is not finite deposits nothing.
+__device__ inline double fx_weight(double w) { return fabs(w) < INFINITY ? w : 0.0; }
+
+// ---- particles' cells (parity outputs) --------------------------------------
+// cell_index[2 p + {0, 1}] = floor of the exact cell coordinates, saturated
+// to int32; cell_count += 1 at the lower cell when it lies on the grid.
+__global__ __launch_bounds__(kThreads) void cic_cells_kernel(
+    const double *__restrict__ q1, const double *__restrict__ q2, int64_t n, int nb1,
+    double start1, double inv1, int nb2, double start2, double inv2,
+    int32_t *__restrict__ cell_index, int32_t *__restrict__ cell_count) {
+#pragma clang fp contract(off)
+  const int64_t stride = (int64_t)gridDim.x * kThreads;
+  for (int64_t p = (int64_t)blockIdx.x * kThreads + threadIdx.x; p < n; p += stride) {
+    const double f1 = floor((q1[p] - start1) * inv1), f2 = floor((q2[p] - start2) * inv2);
+    if (cell_index) {
+      const double g1 = fmin(fmax(f1, -2147483648.0), 2147483647.0);
+      const double g2 = fmin(fmax(f2, -2147483648.0), 2147483647.0);
+      cell_index[2 * p] = isnan(f1) ? INT32_MIN : (int32_t)g1;
+      cell_index[2 * p + 1] = isnan(f2) ? INT32_MIN : (int32_t)g2;
+    }
+    if (cell_count && f1 >= 0.0 && f1 < (double)nb1 && f2 >= 0.0 && f2 < (double)nb2)
+      atomicAdd(cell_count + (int64_t)f1 * nb2 + (int64_t)f2, 1);
   }
 }
 
-__global__ __launch_bounds__(kThreads) void zero_i64(int64_t *__restrict__ a, int64_t n,
-                                                     int32_t *__restrict__ c, int64_t nc) {
-  int64_t stride = (int64_t)gridDim.x * blockDim.x;
+__global__ __launch_bounds__(kThreads) void zero_i32(int32_t *__restrict__ a, int64_t n) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) a[i] = 0;
-  if (c)
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nc; i += stride) c[i] = 0;
 }
 
-// acc[0..ncell) high words, acc[ncell..2 ncell) low words
-__device__ inline void fx_add(int64_t *acc, int64_t cell, int64_t ncell, double v, double scale) {
-  const double s = v * scale;                   // exact: scale is a power of two
-  const double h = floor(s * 0x1p-32);
-  const double l = s - h * 0x1p32;              // in [0, 2^32]
-  const long long hi = (long long)h;
-  const unsigned long long lo = (unsigned long long)rint(l);
-  if (hi != 0) atomicAdd(reinterpret_cast<unsigned long long *>(acc + cell), (unsigned long long)hi);
-  if (lo != 0) atomicAdd(reinterpret_cast<unsigned long long *>(acc + ncell + cell), lo);
-}
-
-// One pass over the particles.  Grid A: weights wA (unit weights when wA is
-// null) at scale[sA].  Grid B (only when wB is non-null): weights wB at
-// scale[1].
+// ---- direct form: global atomics ---------------------------------------------
+// For grids whose row tiles do not suit LDS (tile_plan).  blockIdx.y: the
+// grid (0: weights wA, 1: weights wB; null: unit weights).
 __global__ __launch_bounds__(kThreads) void cic_kernel(
     const double *__restrict__ q1, const double *__restrict__ q2,
     const double *__restrict__ wA, const double *__restrict__ wB, int64_t n, int nb1,
-    double start1, double inv1, int nb2, double start2, double inv2,
-    const double *__restrict__ scale, int sA, int64_t *__restrict__ accA,
-    int64_t *__restrict__ accB, int32_t *__restrict__ cell_index,
-    int32_t *__restrict__ cell_count) {
+    double start1, double inv1, int nb2, double start2, double inv2, double *__restrict__ hdr,
+    int npart, int64_t *__restrict__ acc) {
 #pragma clang fp contract(off)
-  const double scA = scale[sA], scB = scale[1];
-  int64_t stride = (int64_t)gridDim.x * kThreads;
-  for (int64_t p = (int64_t)blockIdx.x * kThreads + threadIdx.x; p < n; p += stride) {
-    double c1 = (q1[p] - start1) * inv1;
-    double c2 = (q2[p] - start2) * inv2;
-    double f1 = floor(c1), f2 = floor(c2);
-    double S1 = 1.0 - (c1 - f1);
-    double S2 = 1.0 - (c2 - f2);
-    // Indices far off the grid only need to fail the range tests below.
-    int i1 = (f1 > -4.0 && f1 < (double)nb1 + 4.0) ? (int)f1 : -8;
-    int i2 = (f2 > -4.0 && f2 < (double)nb2 + 4.0) ? (int)f2 : -8;
-    if (cell_index) {
-      // floor() of the exact cell coordinate, saturated to int32
-      double g1 = fmin(fmax(f1, -2147483648.0), 2147483647.0);
-      double g2 = fmin(fmax(f2, -2147483648.0), 2147483647.0);
-      cell_index[2 * p] = isnan(f1) ? INT32_MIN : (int32_t)g1;
-      cell_index[2 * p + 1] = isnan(f2) ? INT32_MIN : (int32_t)g2;
-    }
-    bool a0 = (i1 >= 0) && (i1 < nb1), a1 = (i1 + 1 >= 0) && (i1 + 1 < nb1);
-    bool b0 = (i2 >= 0) && (i2 < nb2), b1 = (i2 + 1 >= 0) && (i2 + 1 < nb2);
-    if (cell_count && a0 && b0) atomicAdd(cell_count + (int64_t)i1 * nb2 + i2, 1);
-    double wa = wA ? wA[p] : 1.0;
-    // Corner weights in the reference's association: (w*S1)*S2.
-    double t00 = wa * S1 * S2, t01 = wa * S1 * (1.0 - S2);
-    double t10 = wa * (1.0 - S1) * S2, t11 = wa * (1.0 - S1) * (1.0 - S2);
-    const int64_t nc = (int64_t)nb1 * nb2;
-    const int64_t base = (int64_t)i1 * nb2 + i2;
-    if (a0 && b0) fx_add(accA, base, nc, t00, scA);
-    if (a0 && b1) fx_add(accA, base + 1, nc, t01, scA);
-    if (a1 && b0) fx_add(accA, base + nb2, nc, t10, scA);
-    if (a1 && b1) fx_add(accA, base + nb2 + 1, nc, t11, scA);
-    if (wB) {
-      double wb = wB[p];
-      double u00 = wb * S1 * S2, u01 = wb * S1 * (1.0 - S2);
-      double u10 = wb * (1.0 - S1) * S2, u11 = wb * (1.0 - S1) * (1.0 - S2);
-      if (a0 && b0) fx_add(accB, base, nc, u00, scB);
-      if (a0 && b1) fx_add(accB, base + 1, nc, u01, scB);
-      if (a1 && b0) fx_add(accB, base + nb2, nc, u10, scB);
-      if (a1 && b1) fx_add(accB, base + nb2 + 1, nc, u11, scB);
-    }
+  __shared__ double red[kThreads / 64];
+  const double *w = blockIdx.y ? wB : wA;
+  const FxScale f = fx_scale(w ? max_weight(hdr + 8, npart, red) : 1.0, n);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    hdr[2 * blockIdx.y] = f.k;
+    hdr[2 * blockIdx.y + 1] = f.d;
   }
-}
-
-// total = hi * 2^32 + lo, normalised so the low part is < 2^32, then one
-// rounding to float64 and an exact power-of-two rescale.
-// LDS-privatised form of cic_kernel for grids whose row tiles fit in LDS.
-// Workgroup (chunk c, tile y) takes particles [c*per, (c+1)*per) and the
-// grid rows [y*rows, y*rows + rows): it accumulates the same two-word
-// fixed-point words in LDS with 64-bit LDS atomics and adds its non-zero
-// cells to the global words once.  Integer sums: the grid is identical to
-// the direct form's, for every launch order.
-constexpr int kTileLdsBytes = 48 * 1024;
-
-__device__ inline void lds_fx_add(unsigned long long *hi, unsigned long long *lo, int cell,
-                                  double v, double scale) {
-  const double s = v * scale;
-  const double h = floor(s * 0x1p-32);
-  const double l = s - h * 0x1p32;
-  const long long hv = (long long)h;
-  const unsigned long long lv = (unsigned long long)rint(l);
-  if (hv != 0) atomicAdd(hi + cell, (unsigned long long)hv);
-  if (lv != 0) atomicAdd(lo + cell, lv);
-}
-
-__global__ __launch_bounds__(kThreads) void cic_tile_kernel(
-    const double *__restrict__ q1, const double *__restrict__ q2,
-    const double *__restrict__ wA, const double *__restrict__ wB, int64_t n, int64_t per,
-    int nb1, double start1, double inv1, int nb2, double start2, double inv2, int rows,
-    const double *__restrict__ scale, int sA, int64_t *__restrict__ accA,
-    int64_t *__restrict__ accB, int32_t *__restrict__ cell_index,
-    int32_t *__restrict__ cell_count) {
-#pragma clang fp contract(off)
-  extern __shared__ __align__(16) unsigned long long lds[];
-  const int r0 = blockIdx.y * rows;
-  const int r1 = min(r0 + rows, nb1);
-  const int tcells = (r1 - r0) * nb2;
-  const int ngrid = wB ? 2 : 1;
-  unsigned long long *hA = lds, *lA = lds + tcells;
-  unsigned long long *hB = lds + 2 * tcells, *lB = lds + 3 * tcells;
-  int *cnt = reinterpret_cast<int *>(lds + 2 * ngrid * tcells);
-  for (int e = threadIdx.x; e < 2 * ngrid * tcells; e += kThreads) lds[e] = 0ull;
-  if (cell_count)
-    for (int e = threadIdx.x; e < tcells; e += kThreads) cnt[e] = 0;
-  __syncthreads();
-  const double scA = scale[sA], scB = scale[1];
-  const int64_t p0 = (int64_t)blockIdx.x * per;
-  const int64_t p1 = min(p0 + per, n);
-  for (int64_t p = p0 + threadIdx.x; p < p1; p += kThreads) {
-    double c1 = (q1[p] - start1) * inv1;
-    double f1 = floor(c1);
-    // rows touched: f1 and f1 + 1; skip particles that miss this tile
-    const bool owner_low = (f1 >= (double)r0 && f1 < (double)r1) ||
-                           (blockIdx.y == 0 && !(f1 >= 0.0)) ||
-                           (r1 == nb1 && f1 >= (double)nb1);
-    const bool touches = f1 >= (double)(r0 - 1) && f1 < (double)r1;
-    if (!touches && !(owner_low && cell_index)) continue;
-    double c2 = (q2[p] - start2) * inv2;
-    double f2 = floor(c2);
-    double S1 = 1.0 - (c1 - f1);
-    double S2 = 1.0 - (c2 - f2);
-    int i1 = (f1 > -4.0 && f1 < (double)nb1 + 4.0) ? (int)f1 : -8;
-    int i2 = (f2 > -4.0 && f2 < (double)nb2 + 4.0) ? (int)f2 : -8;
-    if (cell_index && owner_low) {
-      double g1 = fmin(fmax(f1, -2147483648.0), 2147483647.0);
-      double g2 = fmin(fmax(f2, -2147483648.0), 2147483647.0);
-      cell_index[2 * p] = isnan(f1) ? INT32_MIN : (int32_t)g1;
-      cell_index[2 * p + 1] = isnan(f2) ? INT32_MIN : (int32_t)g2;
-    }
-    if (!touches) continue;
-    const bool a0 = (i1 >= r0) && (i1 < r1), a1 = (i1 + 1 >= r0) && (i1 + 1 < r1);
-    const bool b0 = (i2 >= 0) && (i2 < nb2), b1 = (i2 + 1 >= 0) && (i2 + 1 < nb2);
-    const int lrow = i1 - r0;   // may be -1 when only row i1+1 is in the tile
-    if (cell_count && a0 && b0) atomicAdd(cnt + lrow * nb2 + i2, 1);
-    const double wa = wA ? wA[p] : 1.0;
-    const double t00 = wa * S1 * S2, t01 = wa * S1 * (1.0 - S2);
-    const double t10 = wa * (1.0 - S1) * S2, t11 = wa * (1.0 - S1) * (1.0 - S2);
-    const int base = lrow * nb2 + i2;
-    if (a0 && b0) lds_fx_add(hA, lA, base, t00, scA);
-    if (a0 && b1) lds_fx_add(hA, lA, base + 1, t01, scA);
-    if (a1 && b0) lds_fx_add(hA, lA, base + nb2, t10, scA);
-    if (a1 && b1) lds_fx_add(hA, lA, base + nb2 + 1, t11, scA);
-    if (wB) {
-      const double wb = wB[p];
-      const double u00 = wb * S1 * S2, u01 = wb * S1 * (1.0 - S2);
-      const double u10 = wb * (1.0 - S1) * S2, u11 = wb * (1.0 - S1) * (1.0 - S2);
-      if (a0 && b0) lds_fx_add(hB, lB, base, u00, scB);
-      if (a0 && b1) lds_fx_add(hB, lB, base + 1, u01, scB);
-      if (a1 && b0) lds_fx_add(hB, lB, base + nb2, u10, scB);
-      if (a1 && b1) lds_fx_add(hB, lB, base + nb2 + 1, u11, scB);
-    }
-  }
-  __syncthreads();
   const int64_t nc = (int64_t)nb1 * nb2;
-  const int64_t g0 = (int64_t)r0 * nb2;
-  for (int e = threadIdx.x; e < tcells; e += kThreads) {
-    if (hA[e]) atomicAdd(reinterpret_cast<unsigned long long *>(accA + g0 + e), hA[e]);
-    if (lA[e]) atomicAdd(reinterpret_cast<unsigned long long *>(accA + nc + g0 + e), lA[e]);
-    if (wB) {
-      if (hB[e]) atomicAdd(reinterpret_cast<unsigned long long *>(accB + g0 + e), hB[e]);
-      if (lB[e]) atomicAdd(reinterpret_cast<unsigned long long *>(accB + nc + g0 + e), lB[e]);
+  unsigned long long *hi = reinterpret_cast<unsigned long long *>(acc) + blockIdx.y * 2 * nc;
+  unsigned long long *lo = hi + nc;
+  const int64_t stride = (int64_t)gridDim.x * kThreads;
+  for (int64_t p = (int64_t)blockIdx.x * kThreads + threadIdx.x; p < n; p += stride) {
+    const CicAxis A = cic_axis(q1[p], start1, inv1, nb1), B = cic_axis(q2[p], start2, inv2, nb2);
+    const double wa = w ? fx_weight(w[p]) : 1.0;
+    const bool a[2] = {A.i >= 0 && A.i < nb1, A.i + 1 >= 0 && A.i + 1 < nb1};
+    const bool b[2] = {B.i >= 0 && B.i < nb2, B.i + 1 >= 0 && B.i + 1 < nb2};
+    // Corner weights in the reference's association: (w*S1)*S2.
+    const double t0 = wa * A.S, t1 = wa * (1.0 - A.S);
+    const double t[4] = {t0 * B.S, t0 * (1.0 - B.S), t1 * B.S, t1 * (1.0 - B.S)};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      if (!(a[c >> 1] && b[c & 1])) continue;
+      const FxWords v = fx_words(t[c], f);
+      const int64_t cell = (int64_t)(A.i + (c >> 1)) * nb2 + B.i + (c & 1);
+      if (v.hi) atomicAdd(hi + cell, (unsigned long long)v.hi);
+      if (v.lo) atomicAdd(lo + cell, (unsigned long long)v.lo);
     }
-    if (cell_count && cnt[e]) atomicAdd(cell_count + g0 + e, cnt[e]);
   }
 }
 
 __global__ __launch_bounds__(kThreads) void fx_to_double(const int64_t *__restrict__ acc,
-                                                         const double *__restrict__ scale,
-                                                         int which, int64_t n,
-                                                         double *__restrict__ out) {
-  double inv = 1.0 / scale[which];
-  const uint64_t *lo_w = reinterpret_cast<const uint64_t *>(acc + n);
-  int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    uint64_t lo = lo_w[i];
-    int64_t hi = acc[i] + (int64_t)(lo >> 32);
-    double l = (double)(lo & 0xffffffffull);
-    out[i] = fma((double)hi, 0x1p32, l) * inv;
+                                                         const double *__restrict__ hdr, int64_t n,
+                                                         double *__restrict__ outA,
+                                                         double *__restrict__ outB) {
+  double *out = blockIdx.y ? outB : outA;
+  const int64_t *hi = acc + blockIdx.y * 2 * n, *lo = hi + n;
+  FxScale f;
+  f.up = ldexp(1.0, (int)hdr[2 * blockIdx.y]);
+  f.up_lo = ldexp(1.0, (int)hdr[2 * blockIdx.y + 1]);
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
+    out[i] = fx_value(hi[i], lo[i], f);
+}
+
+// ---- LDS form -----------------------------------------------------------------
+// A workgroup of 1024 threads owns one tile of one grid (density or vx) in
+// LDS, 16 bytes a cell, and a chunk of the particles; it adds the corners
+// that fall on its tile with 64-bit LDS atomics and stores the tile's words
+// once, without atomics, for tile_sum_kernel to add up.  Tiles: groups of G
+// rows dealt round the T tiles (row i in tile (i / G) % T), so a bunch whose
+// rows carry very different numbers of particles still loads the tiles alike.
+// Each grid has workgroups of its own: at 100 x 100 cells a whole grid is one
+// tile, every lane works on every particle, and a particle's cell (25 of
+// about 120 operations) is all that is computed twice.
+// Bound: LDS atomics (8 per particle and grid, spread over the banks).
+// kQueue (T > 2, where most of a wave's particles miss its tile): the wave
+// scans x alone and queues the hits in LDS; every 64 of them are deposited by
+// a full wave.
+// Measured (both grids, whole call): 1e7 particles on 100 x 100 112 us (544 us
+// with 48 KB row tiles, which left most lanes idle, and a flush by global
+// atomics), 128 x 128 180 us (801); 3e6 on 256 x 256 106 us (2157 us with 16
+// global atomics a particle, about 17 G atomics/s); 1e5 on 64 x 64 18 us (32).
+constexpr int kTileThreads = 1024;
+constexpr int kLdsBytes = 160 * 1024 - 256;   // a CU's LDS, less the static part
+constexpr int kQueueLen = 128;                                   // per wave
+constexpr int kQueueBytes = (kTileThreads / 64) * kQueueLen * 4;
+constexpr int kMaxTiles = 64;
+constexpr int kMaxWg = 256;                                      // one per CU
+constexpr int kMinPer = 4096;                                    // particles per workgroup
+
+struct TilePlan {
+  int T, G, rows;    // tiles, rows per group, rows per tile (T = 0: direct form)
+  int cells;         // rows * nb2
+  size_t lds;        // bytes
+};
+
+// Fewest tiles that fit; larger row groups first (a particle's two rows are
+// then in one tile more often).  Every tile scans all particles, so the gain
+// over the direct form falls with the number of tiles: 52 tiles (600 x 600)
+// take 1.6 ms at 1e7 particles and 33 us at 2e4, the direct form's atomics
+// 8.0 ms and 39 us; kMaxTiles keeps to that range.
+TilePlan tile_plan(int nb1, int nb2) {
+  TilePlan p = {0, 0, 0, 0, 0};
+  const int64_t map = (int64_t)(nb1 + 2) * 4 + 16;
+  for (int G = 4; G >= 1; G >>= 1) {
+    const int groups = (nb1 + G - 1) / G;
+    for (int T = 1; T <= kMaxTiles && T <= groups; ++T) {
+      const int64_t rows = (int64_t)((groups + T - 1) / T) * G;
+      const int64_t lds = rows * nb2 * 16 + map + (T > 2 ? kQueueBytes : 0);
+      if (lds > kLdsBytes) continue;
+      p.T = T;
+      p.G = G;
+      p.rows = (int)rows;
+      p.cells = (int)rows * nb2;
+      p.lds = (size_t)lds;
+      return p;
+    }
   }
+  return p;
+}
+
+// Chunks of the particles per tile and grid: at most kMaxWg workgroups.
+int tile_chunks(const TilePlan &t, int ngrid, int64_t n) {
+  int64_t c = kMaxWg / (t.T * ngrid);
+  const int64_t most = (n + kMinPer - 1) / kMinPer;
+  if (c > most) c = most;
+  return (int)(c < 1 ? 1 : c);
+}
+
+template <bool kQueue>
+__global__ __launch_bounds__(kTileThreads) void cic_tile_kernel(
+    const double *__restrict__ q1, const double *__restrict__ q2,
+    const double *__restrict__ wA, const double *__restrict__ wB, int64_t n, int64_t per,
+    int nb1, double start1, double inv1, int nb2, double start2, double inv2, int T, int G,
+    int cells, double *__restrict__ hdr, int npart, unsigned long long *__restrict__ words) {
+#pragma clang fp contract(off)
+  extern __shared__ __align__(16) unsigned long long lds[];
+  __shared__ double red[kTileThreads / 64];
+  unsigned long long *hi = lds, *lo = lds + cells;
+  // first cell of grid row i in the tile, at [i + 1]; -1 when the row is in
+  // another tile or off the grid (i = -1 and nb1)
+  int *rowmap = reinterpret_cast<int *>(lds + 2 * (size_t)cells);
+  const int grid = blockIdx.y / T, tile = blockIdx.y - grid * T;
+  const double *w = grid ? wB : wA;
+  for (int e = threadIdx.x; e < 2 * cells; e += kTileThreads) lds[e] = 0ull;
+  for (int i = (int)threadIdx.x - 1; i <= nb1; i += kTileThreads) {
+    const int g = i / G;
+    rowmap[i + 1] = (i >= 0 && i < nb1 && g % T == tile) ? ((g / T) * G + (i - g * G)) * nb2 : -1;
+  }
+  const FxScale f = fx_scale(w ? max_weight(hdr + 8, npart, red) : 1.0, n);
+  if (blockIdx.x == 0 && tile == 0 && threadIdx.x == 0) {
+    hdr[2 * grid] = f.k;
+    hdr[2 * grid + 1] = f.d;
+  }
+  __syncthreads();
+
+  const auto add = [&](int cell, double t) {
+    const FxWords v = fx_words(t, f);
+    atomicAdd(hi + cell, (unsigned long long)v.hi);
+    atomicAdd(lo + cell, (unsigned long long)v.lo);
+  };
+  const auto deposit = [&](double x, double z, double wt) {
+    const CicAxis A = cic_axis(x, start1, inv1, nb1), B = cic_axis(z, start2, inv2, nb2);
+    if (A.i < -1 || A.i >= nb1) return;
+    const int ra = rowmap[A.i + 1], rb = rowmap[A.i + 2];
+    const bool b0 = B.i >= 0 && B.i < nb2, b1 = B.i + 1 >= 0 && B.i + 1 < nb2;
+    // Corner weights in the reference's association: (w*S1)*S2.
+    const double t0 = wt * A.S, t1 = wt * (1.0 - A.S);
+    if (ra >= 0) {
+      if (b0) add(ra + B.i, t0 * B.S);
+      if (b1) add(ra + B.i + 1, t0 * (1.0 - B.S));
+    }
+    if (rb >= 0) {
+      if (b0) add(rb + B.i, t1 * B.S);
+      if (b1) add(rb + B.i + 1, t1 * (1.0 - B.S));
+    }
+  };
+  const int64_t p0 = (int64_t)blockIdx.x * per, p1 = min(p0 + per, n);
+  if (!kQueue) {
+    int64_t p = p0 + threadIdx.x;
+    double x = 0.0, z = 0.0, wt = 1.0;
+    if (p < p1) {
+      x = q1[p];
+      z = q2[p];
+      if (w) wt = w[p];
+    }
+    while (p < p1) {   // the next particle's loads in flight over this one's sums
+      const int64_t pn = p + kTileThreads;
+      double xn = 0.0, zn = 0.0, wn = 1.0;
+      if (pn < p1) {
+        xn = q1[pn];
+        zn = q2[pn];
+        if (w) wn = w[pn];
+      }
+      deposit(x, z, fx_weight(wt));
+      p = pn;
+      x = xn;
+      z = zn;
+      wt = wn;
+    }
+  } else {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int *queue = rowmap + nb1 + 2 + wave * kQueueLen;
+    int count = 0;   // wave-uniform
+    const auto drain = [&](int take) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      if (lane < take) {
+        const int64_t p = p0 + queue[count - take + lane];
+        deposit(q1[p], q2[p], w ? fx_weight(w[p]) : 1.0);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      count -= take;
+    };
+    // kScan groups of 64 particles a time, the next kScan in flight
+    constexpr int kScan = 4;
+    const auto load = [&](int64_t b, double (&x)[kScan]) {
+#pragma unroll
+      for (int k = 0; k < kScan; ++k) {
+        const int64_t p = b + k * 64 + lane;
+        x[k] = p < p1 ? q1[p] : NAN;   // misses every tile
+      }
+    };
+    double x[kScan], xn[kScan];
+    int64_t b = p0 + wave * (64 * kScan);
+    load(b, x);
+    while (b < p1) {
+      const int64_t bn = b + kTileThreads * kScan;
+      load(bn, xn);
+#pragma unroll
+      for (int k = 0; k < kScan; ++k) {
+        const double c = floor((x[k] - start1) * inv1);
+        bool hit = c >= -1.0 && c < (double)nb1;
+        if (hit) {
+          const int i = (int)c;
+          hit = rowmap[i + 1] >= 0 || rowmap[i + 2] >= 0;
+        }
+        const unsigned long long m = __ballot(hit);
+        if (hit)
+          queue[count + __popcll(m & ((1ull << lane) - 1ull))] = (int)(b + k * 64 + lane - p0);
+        count += __popcll(m);
+        if (count >= 64) drain(64);
+        x[k] = xn[k];
+      }
+      b = bn;
+    }
+    if (count) drain(count);
+  }
+  __syncthreads();
+  unsigned long long *out = words + ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 2 * cells;
+  for (int e = threadIdx.x; e < 2 * cells; e += kTileThreads) out[e] = lds[e];
+}
+
+// Adds the chunks' words of each cell and converts the sums: 64 cells per
+// workgroup, its four waves each a quarter of the chunks.
+__global__ __launch_bounds__(kThreads) void tile_sum_kernel(
+    const unsigned long long *__restrict__ words, const double *__restrict__ hdr, int chunks,
+    int nb1, int nb2, int T, int G, int cells, double *__restrict__ outA,
+    double *__restrict__ outB) {
+  __shared__ unsigned long long part[2][kThreads];
+  const int grid = blockIdx.y / T, tile = blockIdx.y - grid * T;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int cell = blockIdx.x * 64 + lane;
+  const unsigned long long *base = words + (int64_t)blockIdx.y * chunks * 2 * cells;
+  unsigned long long h = 0, l = 0;
+  if (cell < cells) {
+    const int c1 = (wave + 1) * chunks / 4;
+#pragma unroll 8
+    for (int c = wave * chunks / 4; c < c1; ++c) {
+      h += base[(int64_t)c * 2 * cells + cell];
+      l += base[(int64_t)c * 2 * cells + cells + cell];
+    }
+  }
+  part[0][threadIdx.x] = h;
+  part[1][threadIdx.x] = l;
+  __syncthreads();
+  if (wave || cell >= cells) return;
+#pragma unroll
+  for (int k = 1; k < 4; ++k) {
+    h += part[0][k * 64 + lane];
+    l += part[1][k * 64 + lane];
+  }
+  const int lr = cell / nb2, col = cell - lr * nb2;
+  const int row = ((lr / G) * T + tile) * G + lr % G;
+  if (row >= nb1) return;
+  FxScale f;
+  f.up = ldexp(1.0, (int)hdr[2 * grid]);
+  f.up_lo = ldexp(1.0, (int)hdr[2 * grid + 1]);
+  (grid ? outB : outA)[(int64_t)row * nb2 + col] = fx_value((long long)h, (long long)l, f);
 }
 
 int grid_for(int64_t n) {
@@ -282,47 +465,40 @@ int deposit_impl(const char *who, const double *q1, const double *q2, const doub
     return set_error(DFCSR_ENOWS, "%s: workspace too small", who);
   hipStream_t s = as_stream(stream);
   double *hdr = static_cast<double *>(ws);
-  int64_t ncell = (int64_t)nb1 * nb2;
-  int64_t *accA = reinterpret_cast<int64_t *>(hdr + kHdr);
-  int64_t *accB = accA + 2 * ncell;
+  const int64_t ncell = (int64_t)nb1 * nb2;
   // bins: inv_spacing = 1 / ((end - start) / nbins), deposit.py:55-58
-  double inv1 = 1.0 / ((e1 - s1) / (double)nb1);
-  double inv2 = 1.0 / ((e2 - s2) / (double)nb2);
-  int nb = nblocks_for(n);
+  const double inv1 = 1.0 / ((e1 - s1) / (double)nb1);
+  const double inv2 = 1.0 / ((e2 - s2) / (double)nb2);
+  const int nb = nblocks_for(n);
+  const int ngrid = outB ? 2 : 1;
+  if (cell_count)
+    hipLaunchKernelGGL(zero_i32, dim3(grid_for(ncell)), dim3(kThreads), 0, s, cell_count, ncell);
+  if ((cell_index || cell_count) && n > 0)
+    hipLaunchKernelGGL(cic_cells_kernel, dim3(grid_for(n)), dim3(kThreads), 0, s, q1, q2, n, nb1,
+                       s1, inv1, nb2, s2, inv2, cell_index, cell_count);
   const double *wmax = wB ? wB : wA;   // the non-unit weight, if any
   if (wmax) hipLaunchKernelGGL(absmax_partial, dim3(nb), dim3(kThreads), 0, s, wmax, n, hdr + 8);
-  hipLaunchKernelGGL(scale_final, dim3(1), dim3(kThreads), 0, s, (const double *)(hdr + 8), nb,
-                     n, wmax ? 1 : 0, hdr);
-  hipLaunchKernelGGL(zero_i64, dim3(grid_for(4 * ncell)), dim3(kThreads), 0, s, accA, 4 * ncell,
-                     cell_count, cell_count ? ncell : 0);
-  // A lone weighted deposit (wA) uses the weighted scale[1] for grid A.
-  int sA = wA ? 1 : 0;
-  // LDS tiles: 2 words per cell per grid (+ an int count) must fit kTileLdsBytes
-  const int ngrid = wB ? 2 : 1;
-  const int per_cell = 16 * ngrid + (cell_count ? 4 : 0);
-  const int rows = (int)(kTileLdsBytes / per_cell) / nb2;
-  const int ntile = rows > 0 ? (nb1 + rows - 1) / rows : 0;
-  if (rows >= 4 && ntile <= 16 && n > 0) {
-    // enough particles per workgroup that the flush stays small
-    int64_t chunks = (n + 16383) / 16384;
-    if (chunks < 1) chunks = 1;
-    if (chunks * ntile < 512) chunks = (512 + ntile - 1) / ntile;
-    int64_t per = (n + chunks - 1) / chunks;
-    chunks = (n + per - 1) / per;
-    const size_t lds = (size_t)rows * nb2 * per_cell + 16;
-    hipLaunchKernelGGL(cic_tile_kernel, dim3((unsigned)chunks, ntile), dim3(kThreads), lds, s, q1,
-                       q2, wA, wB, n, per, nb1, s1, inv1, nb2, s2, inv2, rows,
-                       (const double *)hdr, sA, accA, accB, cell_index, cell_count);
+  const TilePlan t = tile_plan(nb1, nb2);
+  if (t.T) {
+    int chunks = tile_chunks(t, ngrid, n);
+    const int64_t per = n > 0 ? (n + chunks - 1) / chunks : 1;
+    auto kernel = t.T > 2 ? cic_tile_kernel<true> : cic_tile_kernel<false>;
+    unsigned long long *words = reinterpret_cast<unsigned long long *>(hdr + kHdr);
+    hipLaunchKernelGGL(kernel, dim3(chunks, t.T * ngrid), dim3(kTileThreads), t.lds, s, q1, q2, wA,
+                       wB, n, per, nb1, s1, inv1, nb2, s2, inv2, t.T, t.G, t.cells, hdr, nb,
+                       words);
+    hipLaunchKernelGGL(tile_sum_kernel, dim3((t.cells + 63) / 64, t.T * ngrid), dim3(kThreads), 0,
+                       s, (const unsigned long long *)words, (const double *)hdr, chunks, nb1,
+                       nb2, t.T, t.G, t.cells, outA, outB);
   } else {
-    hipLaunchKernelGGL(cic_kernel, dim3(grid_for(n)), dim3(kThreads), 0, s, q1, q2, wA, wB, n,
-                       nb1, s1, inv1, nb2, s2, inv2, (const double *)hdr, sA, accA, accB,
-                       cell_index, cell_count);
+    int64_t *acc = reinterpret_cast<int64_t *>(hdr + kHdr);
+    hipLaunchKernelGGL(zero_i64, dim3(grid_for(2 * ngrid * ncell)), dim3(kThreads), 0, s, acc,
+                       2 * ngrid * ncell);
+    hipLaunchKernelGGL(cic_kernel, dim3(grid_for(n), ngrid), dim3(kThreads), 0, s, q1, q2, wA, wB,
+                       n, nb1, s1, inv1, nb2, s2, inv2, hdr, nb, acc);
+    hipLaunchKernelGGL(fx_to_double, dim3(grid_for(ncell), ngrid), dim3(kThreads), 0, s,
+                       (const int64_t *)acc, (const double *)hdr, ncell, outA, outB);
   }
-  hipLaunchKernelGGL(fx_to_double, dim3(grid_for(ncell)), dim3(kThreads), 0, s,
-                     (const int64_t *)accA, (const double *)hdr, sA, ncell, outA);
-  if (outB)   // zero-filled when there are no particles
-    hipLaunchKernelGGL(fx_to_double, dim3(grid_for(ncell)), dim3(kThreads), 0, s,
-                       (const int64_t *)accB, (const double *)hdr, 1, ncell, outB);
   DFCSR_LAUNCH_CHECK(who);
   return DFCSR_OK;
 }
@@ -334,7 +510,18 @@ using namespace dfcsr;
 
 extern "C" int64_t dfcsr_histogram_workspace_bytes(int nbins_1, int nbins_2) {
   if (nbins_1 < 1 || nbins_2 < 1) return 0;
-  return (int64_t)kHdr * 8 + 4 * (int64_t)nbins_1 * nbins_2 * 8;
+  // the tiles' words of every workgroup (LDS form), or both grids' (direct)
+  const TilePlan t = tile_plan(nbins_1, nbins_2);
+  int64_t words = 4 * (int64_t)nbins_1 * nbins_2;
+  if (t.T) {
+    words = 0;
+    for (int g = 1; g <= 2; ++g) {
+      const int64_t w =
+          (int64_t)tile_chunks(t, g, (int64_t)1 << 31) * t.T * g * 2 * (int64_t)t.cells;
+      words = w > words ? w : words;
+    }
+  }
+  return ((int64_t)kHdr + words) * 8;
 }
 
 extern "C" int dfcsr_histogram_cic_2d(const double *q1, const double *q2, const double *w,

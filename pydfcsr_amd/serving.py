@@ -97,7 +97,8 @@ def request_footprint(config: dict, steps: int, precision: str = "mixed") -> int
     hist = slots * grid * (grid * rec + (grid + 1) * cell)
     raw = slots * 5 * nb * nb * 8
     particles = n * 8 * (6 * 2 + 4)           # coordinates, tracking temporary, scratch
-    deposit = 4 * nb * nb * 8 * 2 + 3 * nb * nb * 8
+    # the deposition's words: at most 256 workgroups' 160 KB tiles, or both grids'
+    deposit = max(4 * nb * nb * 8, 256 * 160 * 1024) + 4 * nb * nb * 8 + 3 * nb * nb * 8
     comp = config.get("CSR_computation") or {}
     mesh = int(comp.get("xbins", 20)) * int(comp.get("zbins", 30)) * 8 * 4
     return int(hist + raw + particles + deposit + mesh + (64 << 20))
