@@ -212,7 +212,11 @@ int dfcsr_regrid(const double *src, int64_t src_slot_stride, const DfcsrRegridJo
  * z pair (z, z + 1) a lookup reads is interpolate3D's (clamped at the last
  * z) everywhere.  With them the near-region phases of
  * a wake read cells (FP64 wakes: cells, mixed: cells32), whose neighbouring
- * z lie in neighbouring cells; results are identical with or without them.
+ * z lie in neighbouring cells.  Off the chirp branch a mesh of 17 or more x
+ * bins is then integrated by z lines, from these rings alone: the results
+ * differ from the phases' by rounding (float64 sums in another order; FP64
+ * also interpolates along x first).  Otherwise they are identical with or
+ * without them.
  * One plane must span at most 4 GiB (the wakes address cells within a plane
  * with 32-bit offsets).
  * dcells32 (optional, with cells32) holds the float32 time differences of
@@ -221,7 +225,7 @@ int dfcsr_regrid(const double *src, int64_t src_slot_stride, const DfcsrRegridJo
  * newest slice (dfcsr_cells32_tdiff fills it).  A mixed-precision wake reads
  * the cell-major rings only when both are present: the time lerp
  * v0 + td (v1 - v0) then takes v1 - v0 from dcells32, the same float32
- * value, so the results are those of the float32 rings. */
+ * value: every float32 operation is that of the float32 rings. */
 typedef struct {
   const double *data;    /* [Xi][Zi][cap][DFCSR_HIST_REC64] or NULL */
   const float *data32;   /* [Xi][cap][DFCSR_HIST_CHUNKS32][Zi][4] or NULL */
@@ -325,8 +329,10 @@ int dfcsr_csr_integrand(const DfcsrHistory *hist, const DfcsrLattice *lat, doubl
  * accumulation; FP64 retardation geometry and final sum; needs an FP32
  * ring; vx at the observer comes from the FP64 ring when present, else
  * from an FP32 ring).  The workspace holds per-phase partial sums (a phase is one
- * integration region and one chunk of its x' rows): its size depends on the
- * mesh and integration bins and the chirp branch of p. */
+ * integration region and one chunk of its x' rows), observer data and, by z
+ * lines, their column tables: its size depends on the mesh and integration
+ * bins and the chirp branch of p.  A smaller workspace that holds the phases
+ * is accepted (the wake then goes by phases). */
 int64_t dfcsr_wake_workspace_bytes(const DfcsrWakeParams *p);
 int dfcsr_wake_mesh(const DfcsrHistory *hist, const DfcsrLattice *lat, const DfcsrWakeParams *p,
                     int precision, double *xmesh, double *zmesh, double *dE_dct, double *x_kick,
@@ -336,8 +342,8 @@ int dfcsr_wake_mesh(const DfcsrHistory *hist, const DfcsrLattice *lat, const Dfc
  * allocate (code under HIP graph capture, serving loops, harnesses that
  * forbid hipMalloc).  No counterpart in the reference.  The partial sums and
  * observer data live in a static device array of DFCSR_WAKE_SCRATCH_BYTES
- * per GPU, held until the process ends; a mesh whose workspace
- * (dfcsr_wake_workspace_bytes) exceeds it is rejected with DFCSR_ERANGE
+ * per GPU, held until the process ends; a mesh whose workspace by phases
+ * exceeds it is rejected with DFCSR_ERANGE
  * (32 MiB: up to a 128 x 128 mesh on either branch at 200 x 200
  * integration).  Calls on one GPU share that array: calls that overlap on
  * one GPU (concurrent streams or threads) race.  Calls no allocating
@@ -373,6 +379,8 @@ typedef struct {
   int64_t partial_bytes;  /* partial-sum buffer the launch needs */
   int32_t precision;      /* the precision the tasks were checked for; the
                              launch must use the same */
+  int32_t forms;          /* the kernel forms the tasks take; a captured launch
+                             is for batches of the same */
 } DfcsrWakeBatch;
 int64_t dfcsr_wake_task_table_bytes(int k);
 int dfcsr_wake_tasks_pack(int k, const DfcsrHistory *hist, const DfcsrLattice *lat,

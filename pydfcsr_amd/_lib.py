@@ -74,7 +74,8 @@ class Element(ctypes.Structure):
 
 class WakeBatch(ctypes.Structure):
     _fields_ = [("tasks", c_i32), ("blocks_far", c_i32), ("blocks_near", c_i32),
-                ("observers", c_i32), ("partial_bytes", c_i64), ("precision", c_i32)]
+                ("observers", c_i32), ("partial_bytes", c_i64), ("precision", c_i32),
+                ("forms", c_i32)]
 
 
 class WakeParams(ctypes.Structure):

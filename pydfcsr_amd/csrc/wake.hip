@@ -27,6 +27,7 @@
 // sweep the same z line together, each taking groups of 16 neighbouring
 // workgroups.
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "csr_point.h"
@@ -442,7 +443,26 @@ struct PhasePlan {
   bool obs_major;           // region 0 observer-major (mesh observers)
   int W, S, nob, q;         // observer-major: lanes per observer block, column blocks
                             // per wave, observer blocks per z line, workgroups per block
+  bool line;                // the near regions by z lines (line_block)
+  int obg, nog, ng;         // line: observer blocks per workgroup, groups of them per z
+                            // line, row groups per region
 };
+
+// Doubles of one mesh point's observer data, and (line form) of a z line's
+// axes and of one of its near-region columns.
+constexpr int kObsStride = 48, kObsLine = 16;
+constexpr int kLineHead = 24, kColFp64 = 12, kColMixed = 18;
+
+// Workgroups of a line-form near launch (of 256 threads; half as many of 512):
+// the more, the better the rows near the bunch spread over the chip.  128 x
+// 128 float64 near regions: 1728 us with 3072 or 4096, 1920 with 2048.
+constexpr int kLineWgTarget = 4096;
+
+// Doubles per mesh point of a wake by phases: partial sums and observer data.
+__host__ __device__ inline int64_t point_doubles(const PhasePlan &pl) {
+  const int sums = pl.obs_major ? 4 * pl.S * pl.q : pl.ch0;
+  return (int64_t)(sums + (pl.nreg - 1) * pl.ch1) * 2 + kObsStride;
+}
 
 // Waves of an observer-major region-0 launch wanted per simulation: about
 // 2048 workgroups of 4 waves, 8 per CU, at most 32 per (z line, observer
@@ -451,7 +471,9 @@ struct PhasePlan {
 // chicane (64 x 64) gains from 16 to 32 per block (FP64 6.29 -> 5.97 ms).
 constexpr int kFarWaveTarget = 8192;
 
-__host__ __device__ inline PhasePlan make_plan(const DfcsrWakeParams &P) {
+// cstride: doubles per column of the line form, 0 when the history lacks the
+// rings it reads (line_stride).
+__host__ __device__ inline PhasePlan make_plan(const DfcsrWakeParams &P, int cstride) {
   PhasePlan pl;
   pl.nreg = (fabs(P.slope0) <= 1) ? 3 : 4;   // the branch test of make_regions
   pl.rows0 = 2 * P.Nx;
@@ -476,12 +498,47 @@ __host__ __device__ inline PhasePlan make_plan(const DfcsrWakeParams &P) {
     q = q > 32 ? 32 : q;
     q = q > qmax ? (qmax < 1 ? 1 : qmax) : q;
     pl.q = q;
-    pl.nA = 4 * pl.S * q;
+    pl.nA = q;
   } else {
     pl.W = pl.S = pl.nob = pl.q = 0;
     pl.nA = pl.ch0;
   }
+  // By z lines: off the chirp branch (all observers of a line then share rows
+  // and columns), a quarter wave of observers or more.
+  pl.line = false;
+  pl.obg = pl.nog = pl.ng = 0;
+  if (cstride && pl.obs_major && pl.nreg == 3 && pl.S <= 2) {
+    pl.line = true;
+    pl.obg = pl.nob == 1 ? 1 : (pl.nob == 2 ? 2 : 4);
+    pl.nog = (pl.nob + pl.obg - 1) / pl.obg;
+    const int64_t lines = (int64_t)P.mesh_zbins * pl.nog * 2;
+    const int64_t target = pl.S == 1 ? kLineWgTarget : kLineWgTarget / 2;
+    const int64_t most = (P.Nx + 2 * pl.S - 1) / (2 * pl.S);   // two passes of rows or more
+    int64_t ng = (target + lines - 1) / lines;
+    ng = ng > most ? most : ng;
+    // row groups that leave the workspace at the size of the phases', unless
+    // that would halve them
+    const int64_t M = (int64_t)P.mesh_xbins * P.mesh_zbins;
+    const int64_t room = (point_doubles(pl) - kObsLine - 2 * pl.nA) * M -
+                         (int64_t)P.mesh_zbins * (kLineHead + 2 * (int64_t)P.Nz * cstride);
+    const int64_t fit = room / (4 * M);
+    pl.ng = (int)(fit < ng && 2 * fit >= ng ? fit : ng);
+    pl.nB = 2 * pl.ng;
+  }
   return pl;
+}
+
+// Doubles of a line-form wake's workspace.
+__host__ __device__ inline int64_t line_doubles(const PhasePlan &pl, const DfcsrWakeParams &P,
+                                                int cstride) {
+  return (int64_t)P.mesh_xbins * P.mesh_zbins * (2 * (pl.nA + pl.nB) + kObsLine) +
+         (int64_t)P.mesh_zbins * (kLineHead + 2 * (int64_t)P.Nz * cstride);
+}
+
+// Workgroups of the near launch of one simulation.
+__host__ __device__ inline int64_t near_blocks(const PhasePlan &pl, const DfcsrWakeParams &P) {
+  return pl.line ? (int64_t)P.mesh_zbins * pl.nog * pl.nB
+                 : (int64_t)P.mesh_xbins * P.mesh_zbins * pl.nB;
 }
 
 // Workgroups of the region-0 launch of one simulation.
@@ -513,19 +570,20 @@ struct WakeTask {
   double *dE, *xk;        // outputs [M]
   double *xmesh, *zmesh;  // optional outputs [M] (NULL: not written)
   int64_t part;           // first of its M * (nA + nB) * 2 partial sums
-  int64_t obs;            // first of its M * kObsStride observer values
-  int M, nA, nB;
+  int64_t obs;            // first of its M * ostride observer values
+  int64_t line;           // (line form) first of its z lines' axes and columns
+  int M, nA, nB, ostride;
+  int cstride;            // doubles per column of the line form (0: not in line form)
   int blockA0, blockB0, obs0;   // first workgroup / observer in a batched launch
 };
 
 // Observer data of one mesh point, computed once by wake_observer_kernel
-// and read by every phase of that point (kObsStride doubles):
+// and read by every phase of that point (kObsStride doubles; in the line form
+// the first kObsLine, the axes once per z line -- line_column):
 //   [0] s, [1] x, [2..7] lattice X0, Y0, n_x, n_y, tau_x, tau_y at s,
 //   [8] vx at the observer, [9] 1 if s lies outside the lattice table (its
 //   lookups are 0 there), [16 + 4 r] x' axis of region r (a, b, step, n),
 //   [32 + 4 r] s' axis of region r.
-constexpr int kObsStride = 48;
-
 __device__ inline void store_axis(double *o, const LinAxis &a) {
   o[0] = a.a;
   o[1] = a.b;
@@ -570,11 +628,32 @@ __device__ inline void observer_point(const WakeTask &T, int i, double *__restri
   od[7] = o.L.ty;
   od[8] = o.vx;
   od[9] = trunc_index((s - T.L.min_s) * (1.0 / T.L.ds), T.L.ns).ok ? 0.0 : 1.0;
+  if (T.line) return;   // the axes are stored once per z line (line_column)
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     store_axis(od + 16 + 4 * r, rg.xa[r]);
     store_axis(od + 32 + 4 * r, rg.sa[r]);
   }
+}
+
+// Observer data of mesh point i.
+__host__ __device__ inline int64_t obs_at(const WakeTask &T, int i) {
+  return T.obs + (int64_t)i * T.ostride;
+}
+
+// Line form: axes and near-region column tables of z line zl.  [4 r], r < 3:
+// x' axis of region r; [12 + 4 r] its s' axis; then per column of region 1,
+// then of region 2, cstride doubles (LineColumn).
+__host__ __device__ inline int64_t line_at(const WakeTask &T, int zl) {
+  return T.line + (int64_t)zl * (kLineHead + 2 * (int64_t)T.P.Nz * T.cstride);
+}
+
+// x' (r in region 0 .. 2) and s' axes of region r for mesh point i.
+__device__ inline const double *xaxis_at(const WakeTask &T, const double *ws, int i, int r) {
+  return T.line ? ws + line_at(T, i % T.P.mesh_zbins) + 4 * r : ws + obs_at(T, i) + 16 + 4 * r;
+}
+__device__ inline const double *saxis_at(const WakeTask &T, const double *ws, int i, int r) {
+  return T.line ? ws + line_at(T, i % T.P.mesh_zbins) + 12 + 4 * r : ws + obs_at(T, i) + 32 + 4 * r;
 }
 
 // Integrates phase ph of the mesh point whose observer data is od; every
@@ -591,7 +670,7 @@ __device__ void wake_phase(const WakeTask &T, const double *__restrict__ od, int
   const HistAxes A = make_axes(H);
   const double inv_ds = 1.0 / L.ds;
   int r, j0, j1;
-  phase_rows(make_plan(T.P), ph, r, j0, j1);
+  phase_rows(make_plan(T.P, 0), ph, r, j0, j1);
   const LinAxis xa = load_axis(od + 16 + 4 * r);
   const LinAxis sa = load_axis(od + 32 + 4 * r);
   // (all branches below are uniform over the workgroup)
@@ -748,8 +827,7 @@ __device__ inline void run_phase_block(const WakeTask &T, int l, double *__restr
   ph = kNear ? T.nA + q : q;
   __shared__ RowTable rt;
   double sz, sx;
-  wake_phase<kMixed, kTI, kCells, kNear>(T, partials + T.obs + (int64_t)i * kObsStride, ph, red,
-                                         rt, sz, sx);
+  wake_phase<kMixed, kTI, kCells, kNear>(T, partials + obs_at(T, i), ph, red, rt, sz, sx);
   if (threadIdx.x == 0) {
     double *p = partials + T.part + ((int64_t)i * (T.nA + T.nB) + ph) * 2;
     p[0] = sz;
@@ -760,9 +838,9 @@ __device__ inline void run_phase_block(const WakeTask &T, int l, double *__restr
 // Workgroup l of a task's observer-major region-0 launch: z line, block of
 // observers, group of column blocks (see PhasePlan).  Lane (sub, ol) of wave
 // w integrates, for observer ol of the block, column block (4 g + w) S + sub
-// over every row of region 0 inside the history, and writes that partial sum
-// (NaN where the reference's integrand is 0/0 over the region, as
-// wake_phase).  Summation: per column over the rows in order, weighted sums
+// over every row of region 0 inside the history; the workgroup's 4 S column
+// blocks are added in order into one partial sum per observer (NaN where the
+// reference's integrand is 0/0 over the region, as wake_phase).  Summation: per column over the rows in order, weighted sums
 // over the block's columns in order.  kSkip: lookups the history's span
 // table shows to gather zero density and gradients are skipped (an integrand
 // of exactly 0, as in the near regions); every entry is read from the table
@@ -772,7 +850,7 @@ __device__ void far_obs_block(const WakeTask &T, int l, double *__restrict__ par
                               RowTable &rt) {
   const DfcsrHistory &H = T.H;
   const DfcsrLattice &L = T.L;
-  const PhasePlan pl = make_plan(T.P);
+  const PhasePlan pl = make_plan(T.P, T.cstride);
   const int xb = T.P.mesh_xbins, zb = T.P.mesh_zbins;
   const int per_line = pl.nob * pl.q;
   const int zl = l / per_line, rem = l - zl * per_line;
@@ -784,18 +862,20 @@ __device__ void far_obs_block(const WakeTask &T, int l, double *__restrict__ par
   const int i = (valid ? ix : ob * pl.W) * zb + zl;   // padding lanes follow the block's first
   const int cb = (4 * g + wave) * pl.S + sub;
   const int Nz = T.P.Nz;
-  const int k0 = (int)((int64_t)cb * Nz / pl.nA), k1 = (int)((int64_t)(cb + 1) * Nz / pl.nA);
-  const double *__restrict__ od = partials + T.obs + (int64_t)i * kObsStride;
+  const int ncb = 4 * pl.S * pl.q;
+  const int k0 = (int)((int64_t)cb * Nz / ncb), k1 = (int)((int64_t)(cb + 1) * Nz / ncb);
+  const double *__restrict__ od = partials + obs_at(T, i);
   const double t = T.P.t;
   const HistAxes A = make_axes(H);
   const double inv_ds = 1.0 / L.ds;
   // the z line's x' rows (the same for every observer of the line) and this
   // observer's s' columns (the same too, off the chirp branch)
-  const LinAxis xa = load_axis(partials + T.obs + (int64_t)(ob * pl.W * zb + zl) * kObsStride + 16);
-  const LinAxis sa = load_axis(od + 32);
-  double *out = partials + T.part + ((int64_t)i * (pl.nA + pl.nB) + cb) * 2;
+  const LinAxis xa = load_axis(xaxis_at(T, partials, ob * pl.W * zb + zl, 0));
+  const LinAxis sa = load_axis(saxis_at(T, partials, i, 0));
+  double *out = partials + T.part + ((int64_t)i * (pl.nA + pl.nB) + g) * 2;
+  const bool writer = wave == 0 && sub == 0 && valid;
   if (xa.n < 2 || sa.n < 2) {   // trapz over a single sample (uniform)
-    if (valid) out[0] = out[1] = 0.0;
+    if (writer) out[0] = out[1] = 0.0;
     return;
   }
   bool nan_region = false;
@@ -902,10 +982,18 @@ __device__ void far_obs_block(const WakeTask &T, int l, double *__restrict__ par
     for (int d = 32; d >= 1; d >>= 1) c += __shfl_xor(c, d, 64);
     if (lane == 0 && c) atomicAdd(T.P.points_evaluated, c);
   }
-  if (valid) {
-    out[0] = nan_region ? NAN : acc_z;
-    out[1] = nan_region ? NAN : acc_x;
+  __shared__ double sums[2][kThreads];
+  sums[0][threadIdx.x] = acc_z;
+  sums[1][threadIdx.x] = acc_x;
+  __syncthreads();
+  if (!writer) return;
+  double tz = 0.0, tx = 0.0;
+  for (int b = ol; b < kThreads; b += pl.W) {   // waves in order, column blocks in order
+    tz += sums[0][b];
+    tx += sums[1][b];
   }
+  out[0] = nan_region ? NAN : tz;
+  out[1] = nan_region ? NAN : tx;
 }
 
 // The FP32 ring a mixed launch reads: region 0 (many retarded planes per
@@ -959,6 +1047,8 @@ __host__ __device__ inline bool far_skip(const DfcsrHistory &H, const PhasePlan 
   return H.zspan != nullptr && pl.nreg == 4;
 }
 
+#include "wake_line.h"
+
 // Last task whose first index (workgroup or observer) is <= b.
 template <typename F>
 __device__ inline int find_task(const WakeTask *__restrict__ tasks, int ntask, int b, F first) {
@@ -981,9 +1071,10 @@ __global__ __launch_bounds__(kThreads, kMixed && kNear ? 4 : DFCSR_WAKE_MINBLOCK
                           [](const WakeTask &T) { return kNear ? T.blockB0 : T.blockA0; });
   const WakeTask &T = tasks[j];
   const int l = b - (kNear ? T.blockB0 : T.blockA0);
+  if (T.cstride) return;   // the line form's launch runs it
   if (!kNear && T.P.observers == nullptr) {   // observer-major region 0
     __shared__ RowTable rt;
-    const bool skip = far_skip(T.H, make_plan(T.P));   // per task, as dfcsr_wake_mesh
+    const bool skip = far_skip(T.H, make_plan(T.P, 0));   // per task, as dfcsr_wake_mesh
     if constexpr (kMixed) {
       const bool ti = mixed_reads_ti(T.H, false);
       if (ti && skip)
@@ -1017,32 +1108,79 @@ __global__ __launch_bounds__(kThreads, kMixed && kNear ? 4 : DFCSR_WAKE_MINBLOCK
   }
 }
 
+// Threads per mesh point of the observer launch: the first M of a task's
+// kObsThreads * M compute its observers, and (line form) all of them its z
+// lines' columns, of which there are several per mesh point.
+constexpr int kObsThreads = 8;
+
+__device__ inline void observer_data(const WakeTask &T, int i, double *__restrict__ partials) {
+  if (i < T.M) observer_point(T, i, partials + obs_at(T, i));
+  if (T.line)
+    for (int e = i; e < 2 * T.P.Nz * T.P.mesh_zbins; e += kObsThreads * T.M)
+      line_column(T, e, partials);
+}
+
 __global__ __launch_bounds__(kThreads) void wake_observer_kernel(WakeTask T,
                                                                  double *__restrict__ partials) {
   const int i = blockIdx.x * kThreads + threadIdx.x;
-  if (i < T.M) observer_point(T, i, partials + T.obs + (int64_t)i * kObsStride);
+  if (i < kObsThreads * T.M) observer_data(T, i, partials);
+}
+
+// The line form's workgroups of a batched launch (kNear or region 0): S as
+// the task's plan; workgroups of other tasks return.
+template <bool kMixed, bool kNear, int S>
+__global__ __launch_bounds__((kNear ? LineSize<S>::kThreads : kThreads), 4) void
+wake_line_batched_kernel(const WakeTask *__restrict__ tasks, int ntask,
+                         const double *__restrict__ lines, double *__restrict__ partials) {
+  const int b = blockIdx.x;
+  const int j = find_task(tasks, ntask, b,
+                          [](const WakeTask &T) { return kNear ? T.blockB0 : T.blockA0; });
+  const WakeTask &T = tasks[j];
+  if (!T.cstride) return;
+  const PhasePlan pl = make_plan(T.P, T.cstride);
+  if (pl.S != S) return;
+  if constexpr (kNear) {
+    __shared__ LineLds<kMixed, S> sh;
+    line_block<kMixed, S>(T, line_group(T, b - T.blockB0, (int)near_blocks(pl, T.P)), lines,
+                          partials, sh);
+  } else {
+    __shared__ FarLineLds<kMixed, S> sh;
+    far_line_block<kMixed, S>(T, line_group(T, b - T.blockA0, (int)far_blocks(pl, T.P)), partials,
+                              sh);
+  }
 }
 
 __global__ __launch_bounds__(kThreads) void wake_observer_batched_kernel(
     const WakeTask *__restrict__ tasks, int ntask, int nobs, double *__restrict__ partials) {
   const int g = blockIdx.x * kThreads + threadIdx.x;
-  if (g >= nobs) return;
-  const int j = find_task(tasks, ntask, g, [](const WakeTask &T) { return T.obs0; });
+  if (g >= kObsThreads * nobs) return;
+  const int j = find_task(tasks, ntask, g / kObsThreads, [](const WakeTask &T) { return T.obs0; });
   const WakeTask &T = tasks[j];
-  const int i = g - T.obs0;
-  observer_point(T, i, partials + T.obs + (int64_t)i * kObsStride);
+  observer_data(T, g - kObsThreads * T.obs0, partials);
 }
 
-// Sum of the phases of mesh point i in phase order; the reference's signs
-// and scaling (CSR.py:599-602).
-__device__ inline void finalize_point(const WakeTask &T, int i, const double *__restrict__ partials) {
+// Sum of the partial sums of mesh point i by kSumLanes lanes: lane j adds
+// every kSumLanes-th in order, a fixed tree adds the lanes; the reference's
+// signs and scaling (CSR.py:599-602).  One lane per mesh point took 38 us for
+// the 121 partial sums of a 32 x 32 mesh: 1024 serial chains of strided loads.
+constexpr int kSumLanes = 16;
+
+__device__ inline void finalize_point(const WakeTask &T, int i, int lane,
+                                      const double *__restrict__ partials) {
   const int nph = T.nA + T.nB;
-  const double *p = partials + T.part + (int64_t)i * nph * 2;
+  const double2 *p = reinterpret_cast<const double2 *>(partials + T.part) + (int64_t)i * nph;
   double sz = 0.0, sx = 0.0;
-  for (int ph = 0; ph < nph; ++ph) {
-    sz += p[2 * ph];
-    sx += p[2 * ph + 1];
+  for (int ph = lane; ph < nph; ph += kSumLanes) {
+    const double2 v = p[ph];
+    sz += v.x;
+    sx += v.y;
   }
+#pragma unroll
+  for (int d = kSumLanes / 2; d >= 1; d >>= 1) {
+    sz += __shfl_xor(sz, d, 64);
+    sx += __shfl_xor(sx, d, 64);
+  }
+  if (lane) return;
   T.dE[i] = -T.P.csr_scaling * sz;
   T.xk[i] = T.P.csr_scaling * sx;
   if (T.xmesh) {
@@ -1055,16 +1193,21 @@ __device__ inline void finalize_point(const WakeTask &T, int i, const double *__
 
 __global__ __launch_bounds__(kThreads) void wake_finalize_kernel(WakeTask T,
                                                                  const double *__restrict__ partials) {
-  const int i = blockIdx.x * kThreads + threadIdx.x;
-  if (i < T.M) finalize_point(T, i, partials);
+  const int g = blockIdx.x * kThreads + threadIdx.x, i = g / kSumLanes;
+  if (i < T.M) finalize_point(T, i, g % kSumLanes, partials);
 }
 
 __global__ __launch_bounds__(kThreads) void wake_finalize_batched_kernel(
     const WakeTask *__restrict__ tasks, int ntask, int nobs, const double *__restrict__ partials) {
-  const int g = blockIdx.x * kThreads + threadIdx.x;
-  if (g >= nobs) return;
-  const int j = find_task(tasks, ntask, g, [](const WakeTask &T) { return T.obs0; });
-  finalize_point(tasks[j], g - tasks[j].obs0, partials);
+  const int g = blockIdx.x * kThreads + threadIdx.x, i = g / kSumLanes;
+  if (i >= nobs) return;
+  const int j = find_task(tasks, ntask, i, [](const WakeTask &T) { return T.obs0; });
+  finalize_point(tasks[j], i - tasks[j].obs0, g % kSumLanes, partials);
+}
+
+// Workgroups of a launch of `per` threads per mesh point.
+unsigned point_grid(int M, int per) {
+  return (unsigned)(((int64_t)M * per + kThreads - 1) / kThreads);
 }
 
 int check_params(const DfcsrWakeParams *p, const char *who) {
@@ -1095,22 +1238,42 @@ int check_rings(const DfcsrHistory &H, int precision, const char *who) {
   return DFCSR_OK;
 }
 
+// Doubles per column of the line form of this precision, 0 when the history
+// lacks the cell-major rings it reads.
+int line_stride(const DfcsrHistory &H, int precision) {
+  if (precision == DFCSR_PREC_FP64) return H.cells ? kColFp64 : 0;
+  return mixed_cells(H) ? kColMixed : 0;
+}
+
 // check_params without setting the error message (for the size queries).
 bool params_ok(const DfcsrWakeParams &p) {
   return p.Nx >= 1 && p.Nz >= 1 && p.mesh_xbins >= 1 && p.mesh_zbins >= 1 &&
          (int64_t)p.mesh_xbins * p.mesh_zbins <= ((int64_t)1 << 24);
 }
 
-// Partial sums and observer data of one simulation, in doubles.
-int64_t partial_doubles(const DfcsrWakeParams &p) {
-  const PhasePlan pl = make_plan(p);
-  return (int64_t)p.mesh_xbins * p.mesh_zbins * ((pl.nA + pl.nB) * 2 + kObsStride);
+// Partial sums and observer data of one simulation, in doubles: by phases, and
+// the most any form takes (the precision is not known here).
+int64_t phase_doubles(const DfcsrWakeParams &p) {
+  return (int64_t)p.mesh_xbins * p.mesh_zbins * point_doubles(make_plan(p, 0));
 }
 
-// Fills a task; rejects launches whose workgroup counts overflow int.
+int64_t partial_doubles(const DfcsrWakeParams &p) {
+  int64_t n = phase_doubles(p);
+  for (int cs : {kColFp64, kColMixed}) {
+    const PhasePlan pl = make_plan(p, cs);
+    const int64_t m = pl.line ? line_doubles(pl, p, cs) : 0;
+    n = m > n ? m : n;
+  }
+  return n;
+}
+
+// Fills a task; rejects launches whose workgroup counts overflow int.  room:
+// doubles of workspace it may use; without room for the line form, by phases.
 int make_task(const DfcsrHistory &H, const DfcsrLattice &L, const DfcsrWakeParams &P,
-              double *dE, double *xk, double *xmesh, double *zmesh, WakeTask &T, const char *who) {
-  const PhasePlan pl = make_plan(P);
+              int precision, int64_t room, double *dE, double *xk, double *xmesh, double *zmesh,
+              WakeTask &T, const char *who) {
+  PhasePlan pl = make_plan(P, line_stride(H, precision));
+  if (pl.line && line_doubles(pl, P, line_stride(H, precision)) > room) pl = make_plan(P, 0);
   T.H = H;
   T.L = L;
   T.P = P;
@@ -1121,13 +1284,46 @@ int make_task(const DfcsrHistory &H, const DfcsrLattice &L, const DfcsrWakeParam
   T.M = P.mesh_xbins * P.mesh_zbins;
   T.part = 0;
   T.obs = (int64_t)T.M * (pl.nA + pl.nB) * 2;
+  T.ostride = pl.line ? kObsLine : kObsStride;
+  T.line = pl.line ? T.obs + (int64_t)T.M * kObsLine : 0;   // > 0 in line form
+  T.cstride = pl.line ? line_stride(H, precision) : 0;
   T.nA = pl.nA;
   T.nB = pl.nB;
   T.blockA0 = T.blockB0 = T.obs0 = 0;
-  if ((int64_t)T.M * (pl.nA + pl.nB) > ((int64_t)1 << 30) || far_blocks(pl, P) > ((int64_t)1 << 30))
-    return set_error(DFCSR_ERANGE, "%s: %d mesh points x %d phases is too many workgroups", who,
-                     T.M, pl.nA + pl.nB);
+  const int64_t phases = (point_doubles(pl) - kObsStride) / 2;
+  if ((int64_t)T.M * phases > ((int64_t)1 << 30) || far_blocks(pl, P) > ((int64_t)1 << 30))
+    return set_error(DFCSR_ERANGE, "%s: %d mesh points x %lld phases is too many workgroups", who,
+                     T.M, (long long)phases);
   return DFCSR_OK;
+}
+
+// The forms a batch's tasks take (DfcsrWakeBatch.forms): one launch each.
+enum { kFormPhases = 1, kFormLine1 = 2, kFormLine2 = 4 };
+
+template <bool kMixed>
+void launch_batched(const WakeTask *dt, int k, int forms, dim3 ga, dim3 gb, double *part,
+                    hipStream_t s) {
+  const double *lines = part;
+  if (forms & kFormPhases)
+    hipLaunchKernelGGL((wake_phase_batched_kernel<kMixed, false>), ga, dim3(kThreads), 0, s, dt, k,
+                       part);
+  if (forms & kFormLine1)
+    hipLaunchKernelGGL((wake_line_batched_kernel<kMixed, false, 1>), ga, dim3(kThreads), 0, s, dt,
+                       k, lines, part);
+  if (forms & kFormLine2)
+    hipLaunchKernelGGL((wake_line_batched_kernel<kMixed, false, 2>), ga, dim3(kThreads), 0, s, dt,
+                       k, lines, part);
+  if (forms & kFormPhases)
+    hipLaunchKernelGGL((wake_phase_batched_kernel<kMixed, true>), gb, dim3(kThreads), 0, s, dt, k,
+                       part);
+  if (forms & kFormLine1)
+    hipLaunchKernelGGL((wake_line_batched_kernel<kMixed, true, 1>), gb,
+                       dim3(LineSize<1>::kThreads), 0, s, dt,
+                       k, lines, part);
+  if (forms & kFormLine2)
+    hipLaunchKernelGGL((wake_line_batched_kernel<kMixed, true, 2>), gb,
+                       dim3(LineSize<2>::kThreads), 0, s, dt,
+                       k, lines, part);
 }
 
 constexpr int64_t kTableAlign = 256;
@@ -1161,17 +1357,29 @@ extern "C" int dfcsr_wake_mesh(const DfcsrHistory *hist, const DfcsrLattice *lat
   if (precision != DFCSR_PREC_FP64 && precision != DFCSR_PREC_MIXED)
     return set_error(DFCSR_EINVAL, "wake_mesh: unknown precision %d", precision);
   if ((rc = check_rings(*hist, precision, "wake_mesh"))) return rc;
-  if (!ws || ws_bytes < dfcsr_wake_workspace_bytes(p))
+  const int64_t least = phase_doubles(*p) * (int64_t)sizeof(double) + 256;
+  if (!ws || ws_bytes < least)
     return set_error(DFCSR_ENOWS, "wake_mesh: workspace of %lld bytes, %lld needed",
-                     (long long)ws_bytes, (long long)dfcsr_wake_workspace_bytes(p));
+                     (long long)ws_bytes, (long long)least);
   WakeTask T;
-  if ((rc = make_task(*hist, *lat, *p, dE_dct, x_kick, xmesh, zmesh, T, "wake_mesh"))) return rc;
+  if ((rc = make_task(*hist, *lat, *p, precision, ws_bytes / (int64_t)sizeof(double), dE_dct, x_kick, xmesh, zmesh, T, "wake_mesh")))
+    return rc;
   double *part = static_cast<double *>(ws);
   hipStream_t s = as_stream(stream);
-  const PhasePlan pl = make_plan(*p);
-  const dim3 ga((unsigned)far_blocks(pl, *p)), gb(T.M * T.nB), gf((T.M + kThreads - 1) / kThreads);
-  hipLaunchKernelGGL(wake_observer_kernel, gf, dim3(kThreads), 0, s, T, part);
-  if (precision == DFCSR_PREC_MIXED) {
+  const PhasePlan pl = make_plan(*p, T.cstride);
+  const dim3 ga((unsigned)far_blocks(pl, *p)), gb((unsigned)near_blocks(pl, *p));
+  const dim3 go(point_grid(T.M, pl.line ? kObsThreads : 1)), gf(point_grid(T.M, kSumLanes));
+  hipLaunchKernelGGL(wake_observer_kernel, go, dim3(kThreads), 0, s, T, part);
+  if (pl.line) {
+    const bool mixed = precision == DFCSR_PREC_MIXED;
+    auto far = mixed ? (pl.S == 1 ? wake_far_line_kernel<true, 1> : wake_far_line_kernel<true, 2>)
+                     : (pl.S == 1 ? wake_far_line_kernel<false, 1> : wake_far_line_kernel<false, 2>);
+    auto near = mixed ? (pl.S == 1 ? wake_line_kernel<true, 1> : wake_line_kernel<true, 2>)
+                      : (pl.S == 1 ? wake_line_kernel<false, 1> : wake_line_kernel<false, 2>);
+    hipLaunchKernelGGL(far, ga, dim3(kThreads), 0, s, T, part);
+    hipLaunchKernelGGL(near, gb, dim3(pl.S == 1 ? LineSize<1>::kThreads : LineSize<2>::kThreads),
+                       0, s, T, (const double *)part, part);
+  } else if (precision == DFCSR_PREC_MIXED) {
     const bool ti_far = mixed_reads_ti(*hist, false);
     const bool skip = far_skip(*hist, pl);
     if (pl.obs_major && ti_far && skip)
@@ -1219,18 +1427,26 @@ extern "C" int dfcsr_wake_mesh(const DfcsrHistory *hist, const DfcsrLattice *lat
 
 extern "C" int64_t dfcsr_wake_task_table_bytes(int k) { return table_bytes(k < 1 ? 1 : k); }
 
-extern "C" int64_t dfcsr_wake_batched_workspace_bytes(int k, const DfcsrWakeParams *p) {
-  if (k < 1 || !p) return table_bytes(1);
+// Bytes of a batched launch's workspace: by phases, or the most any form takes.
+static int64_t batched_bytes(int k, const DfcsrWakeParams *p, bool phases) {
   int64_t n = 0;
   for (int j = 0; j < k; ++j)
-    if (params_ok(p[j])) n += partial_doubles(p[j]);
+    if (params_ok(p[j])) n += phases ? phase_doubles(p[j]) : partial_doubles(p[j]);
   return table_bytes(k) + n * (int64_t)sizeof(double);
 }
 
-extern "C" int dfcsr_wake_tasks_pack(int k, const DfcsrHistory *hist, const DfcsrLattice *lat,
-                                     const DfcsrWakeParams *p, int precision,
-                                     double *const *dE_dct, double *const *x_kick, void *tasks,
-                                     int64_t tasks_bytes, DfcsrWakeBatch *batch) {
+extern "C" int64_t dfcsr_wake_batched_workspace_bytes(int k, const DfcsrWakeParams *p) {
+  if (k < 1 || !p) return table_bytes(1);
+  return batched_bytes(k, p, false);
+}
+
+namespace {
+
+// dfcsr_wake_tasks_pack; without `lines` every task goes by phases (the
+// smaller workspace).
+int pack_tasks(int k, const DfcsrHistory *hist, const DfcsrLattice *lat, const DfcsrWakeParams *p,
+               int precision, bool lines, double *const *dE_dct, double *const *x_kick,
+               void *tasks, int64_t tasks_bytes, DfcsrWakeBatch *batch) {
   if (k < 1 || k > kMaxTasks)
     return set_error(DFCSR_ERANGE, "wake_tasks_pack: %d tasks (1 to %d)", k, kMaxTasks);
   if (!hist || !lat || !p || !dE_dct || !x_kick || !tasks || !batch)
@@ -1241,6 +1457,7 @@ extern "C" int dfcsr_wake_tasks_pack(int k, const DfcsrHistory *hist, const Dfcs
     return set_error(DFCSR_EINVAL, "wake_tasks_pack: unknown precision %d", precision);
   WakeTask *th = static_cast<WakeTask *>(tasks);
   int64_t na = 0, nb = 0, nobs = 0, part = 0;
+  int forms = 0;
   for (int j = 0; j < k; ++j) {
     int rc;
     if ((rc = check_history(&hist[j], "wake_tasks_pack"))) return rc;
@@ -1249,17 +1466,21 @@ extern "C" int dfcsr_wake_tasks_pack(int k, const DfcsrHistory *hist, const Dfcs
     if (!dE_dct[j] || !x_kick[j]) return set_error(DFCSR_EINVAL, "wake_tasks_pack: NULL output");
     if ((rc = check_rings(hist[j], precision, "wake_tasks_pack"))) return rc;
     WakeTask &T = th[j];
-    if ((rc = make_task(hist[j], lat[j], p[j], dE_dct[j], x_kick[j], nullptr, nullptr, T,
-                        "wake_tasks_pack")))
+    if ((rc = make_task(hist[j], lat[j], p[j], precision, lines ? INT64_MAX : 0, dE_dct[j],
+                        x_kick[j], nullptr, nullptr, T, "wake_tasks_pack")))
       return rc;
     T.obs += part;
+    if (T.line) T.line += part;
     T.part = part;
     T.blockA0 = (int)na;
     T.blockB0 = (int)nb;
     T.obs0 = (int)nobs;
-    part += partial_doubles(p[j]);
-    na += far_blocks(make_plan(p[j]), p[j]);
-    nb += (int64_t)T.M * T.nB;
+    const PhasePlan pl = make_plan(p[j], T.cstride);
+    // (even: partial sums are read in pairs)
+    part += pl.line ? line_doubles(pl, p[j], T.cstride) : phase_doubles(p[j]);
+    forms |= !pl.line ? kFormPhases : (pl.S == 1 ? kFormLine1 : kFormLine2);
+    na += far_blocks(pl, p[j]);
+    nb += near_blocks(pl, p[j]);
     nobs += T.M;
     if (na > ((int64_t)1 << 30) || nb > ((int64_t)1 << 30))
       return set_error(DFCSR_ERANGE, "wake_tasks_pack: too many workgroups");
@@ -1270,7 +1491,17 @@ extern "C" int dfcsr_wake_tasks_pack(int k, const DfcsrHistory *hist, const Dfcs
   batch->observers = (int32_t)nobs;
   batch->partial_bytes = part * (int64_t)sizeof(double);
   batch->precision = precision;
+  batch->forms = forms;
   return DFCSR_OK;
+}
+
+}  // namespace
+
+extern "C" int dfcsr_wake_tasks_pack(int k, const DfcsrHistory *hist, const DfcsrLattice *lat,
+                                     const DfcsrWakeParams *p, int precision,
+                                     double *const *dE_dct, double *const *x_kick, void *tasks,
+                                     int64_t tasks_bytes, DfcsrWakeBatch *batch) {
+  return pack_tasks(k, hist, lat, p, precision, true, dE_dct, x_kick, tasks, tasks_bytes, batch);
 }
 
 extern "C" int dfcsr_wake_batched_launch(const void *dev_tasks, const DfcsrWakeBatch *batch,
@@ -1289,18 +1520,16 @@ extern "C" int dfcsr_wake_batched_launch(const void *dev_tasks, const DfcsrWakeB
   double *part = static_cast<double *>(partials);
   const int k = batch->tasks;
   const dim3 ga(batch->blocks_far), gb(batch->blocks_near);
-  const dim3 gf((batch->observers + kThreads - 1) / kThreads);
-  hipLaunchKernelGGL(wake_observer_batched_kernel, gf, dim3(kThreads), 0, s, dt, k,
+  const dim3 go(point_grid(batch->observers, kObsThreads));
+  const dim3 gf(point_grid(batch->observers, kSumLanes));
+  hipLaunchKernelGGL(wake_observer_batched_kernel, go, dim3(kThreads), 0, s, dt, k,
                      batch->observers, part);
-  if (precision == DFCSR_PREC_MIXED) {
-    hipLaunchKernelGGL((wake_phase_batched_kernel<true, false>), ga, dim3(kThreads), 0, s, dt, k, part);
-    hipLaunchKernelGGL((wake_phase_batched_kernel<true, true>), gb, dim3(kThreads), 0, s, dt, k, part);
-  } else if (precision == DFCSR_PREC_FP64) {
-    hipLaunchKernelGGL((wake_phase_batched_kernel<false, false>), ga, dim3(kThreads), 0, s, dt, k, part);
-    hipLaunchKernelGGL((wake_phase_batched_kernel<false, true>), gb, dim3(kThreads), 0, s, dt, k, part);
-  } else {
+  if (precision != DFCSR_PREC_FP64 && precision != DFCSR_PREC_MIXED)
     return set_error(DFCSR_EINVAL, "wake_batched_launch: unknown precision %d", precision);
-  }
+  if (precision == DFCSR_PREC_MIXED)
+    launch_batched<true>(dt, k, batch->forms, ga, gb, part, s);
+  else
+    launch_batched<false>(dt, k, batch->forms, ga, gb, part, s);
   hipLaunchKernelGGL(wake_finalize_batched_kernel, gf, dim3(kThreads), 0, s, dt, k,
                      batch->observers, (const double *)part);
   DFCSR_LAUNCH_CHECK("wake_batched_launch");
@@ -1316,12 +1545,13 @@ extern "C" int dfcsr_wake_mesh_batched(int k, const DfcsrHistory *hist, const Df
     return set_error(DFCSR_ERANGE, "wake_mesh_batched: %d tasks > %d", k, kMaxTasks);
   if (!ws) return set_error(DFCSR_EINVAL, "wake_mesh_batched: NULL workspace");
   if (!p) return set_error(DFCSR_EINVAL, "wake_mesh_batched: NULL params");
-  if (ws_bytes < dfcsr_wake_batched_workspace_bytes(k, p))
+  if (ws_bytes < batched_bytes(k, p, true))
     return set_error(DFCSR_ENOWS, "wake_mesh_batched: workspace too small");
+  const bool lines = ws_bytes >= batched_bytes(k, p, false);
   std::vector<WakeTask> tasks_h((size_t)k);
   DfcsrWakeBatch batch;
-  int rc = dfcsr_wake_tasks_pack(k, hist, lat, p, precision, dE_dct, x_kick, tasks_h.data(),
-                                 (int64_t)(tasks_h.size() * sizeof(WakeTask)), &batch);
+  int rc = pack_tasks(k, hist, lat, p, precision, lines, dE_dct, x_kick, tasks_h.data(),
+                      (int64_t)(tasks_h.size() * sizeof(WakeTask)), &batch);
   if (rc) return rc;
   hipStream_t s = as_stream(stream);
   // ordered on the stream after whatever still reads the workspace's table;
@@ -1381,7 +1611,9 @@ extern "C" int dfcsr_wake_mesh_noalloc(const DfcsrHistory *hist, const DfcsrLatt
                                        void *stream) {
   int rc;
   if ((rc = check_params(p, "wake_mesh_noalloc"))) return rc;
-  const int64_t need = dfcsr_wake_workspace_bytes(p);
+  // the scratch holds every such mesh by phases; dfcsr_wake_mesh takes the line
+  // form where it holds that too
+  const int64_t need = phase_doubles(*p) * (int64_t)sizeof(double) + 256;
   if (need > (int64_t)DFCSR_WAKE_SCRATCH_BYTES)
     return set_error(DFCSR_ERANGE,
                      "wake_mesh_noalloc: %d x %d mesh points need %lld bytes of scratch, more "

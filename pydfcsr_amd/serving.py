@@ -171,7 +171,7 @@ class BatchedWake:
         ev = torch.cuda.Event()
         ev.record(stream)
         self.copied[i] = ev
-        key = (k, batch.blocks_far, batch.blocks_near, batch.observers)
+        key = (k, batch.blocks_far, batch.blocks_near, batch.observers, batch.forms)
 
         def launch(s):
             _lib.check(self.lib.dfcsr_wake_batched_launch(self.dev.data_ptr(), ctypes.byref(batch),

@@ -63,3 +63,90 @@ def test_deposit_forms(K, ws, bins, n):
         _, v3 = K.deposit_density_vx(_t(x), _t(z), _t(bad), *a, ws)
         bad[50:64] = 0.0
         assert rel_max(v3.cpu(), O.histogram_cic_2d(x[ok], z[ok], bad[ok], *a)) <= 1e-13
+
+
+LAT_ELEMENTS = [dict(type="drift", L=0.1, nsep=1), dict(type="dipole", L=0.3, angle=0.05, nsep=1),
+                dict(type="drift", L=0.4, nsep=2), dict(type="dipole", L=0.3, angle=-0.05, nsep=1)]
+
+
+class _History:
+    """A smooth synthetic history (nt slices on Xi x Zi) with the attributes
+    DeviceHistory and the oracle's C integral read."""
+
+    def __init__(self, t, sx, sz, nt=9, Xi=37, Zi=700):
+        x, z = np.linspace(-5, 5, Xi), np.linspace(-5, 5, Zi)
+        k = np.arange(nt)[:, None, None]
+        g = np.exp(-0.5 * (x[None, :, None] ** 2 + z[None, None, :] ** 2))
+        g = np.where(g > 1e-4, g, 0.0) * (1 + 0.1 * np.sin(k + z[None, None, :]))
+        one = np.ones_like(g)
+        self.data = dict(density=g / (sx * sz), density_x=-x[None, :, None] * g / sx ** 2 / sz,
+                         density_z=-z[None, None, :] * g / sz ** 2 / sx,
+                         vx=(1e-3 * x[None, :, None] + 1e-4 * k) * one,
+                         vx_x=1e-3 / sx * one * (1 + 0.05 * z[None, None, :]))
+        self._axes = dict(min_t=t - 0.03 * (nt - 1), min_x=-5 * sx, min_z=-5 * sz, dt=0.03,
+                          dx=10 * sx / (Xi - 1), dz=10 * sz / (Zi - 1))
+
+    def axes(self):
+        return self._axes
+
+
+# mesh bins about a quarter, half and whole wave and several observer blocks;
+# odd rows and columns; sigma_x / sigma_z thin, round and wide (windows of a
+# few z cells, of the whole grid, and tiled); the mesh past the lattice's end
+@pytest.mark.parametrize("mesh,nxz,sx,sz,t", [
+    ((17, 3), (13, 9), 20e-6, 80e-6, 0.33), ((32, 4), (24, 31), 50e-6, 50e-6, 0.33),
+    ((33, 3), (21, 40), 300e-6, 30e-6, 0.33), ((64, 2), (40, 33), 20e-6, 80e-6, 0.5),
+    ((65, 2), (9, 17), 50e-6, 50e-6, 0.33), ((129, 2), (16, 16), 300e-6, 30e-6, 0.5),
+    ((300, 1), (11, 12), 50e-6, 50e-6, 0.33), ((20, 5), (10, 300), 20e-6, 80e-6, 0.33),
+    ((24, 6), (12, 15), 50e-6, 50e-6, 1.1)])
+def test_wake_line_form(K, ws, mesh, nxz, sx, sz, t):
+    """The wake by z lines (cell-major rings, |slope| <= 1) against the same
+    wake by phases (explicit observers) and the oracle's C integral, float64
+    within 1e-10 of max|W| and mixed within 1e-8 of the phases' (the same
+    float32 operations, float64 sums in another order); batched bit for bit;
+    the span table changes no bit and evaluates no more points."""
+    from oracle import csr_ref_c as C
+    from pydfcsr_amd import _lib
+    from tests.gpu_util import DeviceHistory, DeviceLattice, wake_params
+    T, lat = _History(t, sx, sz), O.LatticeTables(LAT_ELEMENTS)
+    beam = dict(sigma_x=sx, sigma_z=sz, slope=np.array([0.3, 1e-6]), mean_x=0.0)
+    xa, za = (-5 * sx, 5 * sx, mesh[0]), (-5 * sz, 5 * sz, mesh[1])
+    L = DeviceLattice(lat, DEV)
+    args = (t, beam, 0.05, 4.0, *nxz, 9.0, xa, za)
+    P = wake_params(*args)
+    rings = ("fp64", "fp32t", "cells", "cells32")
+    H = DeviceHistory(T, DEV, wrap=2, rings=rings)
+    Hz = DeviceHistory(T, DEV, wrap=2, rings=rings + ("zspan",))
+    M = mesh[0] * mesh[1]
+    out = {p: {k: v.cpu().numpy() for k, v in K.wake_mesh(H.desc, L.desc, P, p, DEV, ws).items()}
+           for p in (0, 1)}
+    obs_np = np.stack([out[0]["zmesh"], out[0]["xmesh"]], axis=1)
+    obs = _t(obs_np)
+    Po = wake_params(*args[:-2], (0.0, 0.0, 1), (0.0, 0.0, M), observers=obs)
+    keep = C._Keep()
+    ref = C.wake(C.hist_from_tracker(T, keep), C.lat_from_tables(lat, keep), t, beam, 0.05, 4.0,
+                 *nxz, 9.0, obs_np)
+    for p, tol, oracle in ((0, 1e-10, 1e-10), (1, 1e-8, 1e-4)):
+        ph = K.wake_mesh(H.desc, L.desc, Po, p, DEV, ws)
+        for k, r in zip(("dE_dct", "x_kick"), ref):
+            a, b = out[p][k], ph[k].cpu().numpy()
+            assert np.array_equal(np.isnan(a), np.isnan(b)), (p, k)
+            assert np.array_equal(np.isnan(a), np.isnan(r)), (p, k)
+            ok = np.isfinite(r)
+            assert ok.any() and np.abs(r[ok]).max() > 0
+            # observers whose sources all lie on one straight (t = 0.5) have
+            # no x kick: what each form holds there is rounding of terms as
+            # large as dE_dct's (the oracle's own is 1e-13 to 1e-12 of it)
+            straight = k == "x_kick" and np.nanmax(np.abs(r)) < 1e-9 * np.nanmax(np.abs(ref[0]))
+            scale = np.nanmax(np.abs(ref[0])) / np.nanmax(np.abs(r)) if straight else 1.0
+            assert rel_max(a[ok], b[ok]) <= tol * scale, (p, k)
+            assert rel_max(a[ok], r[ok]) <= oracle * scale, (p, k)
+        z = K.wake_mesh(Hz.desc, L.desc, P, p, DEV, ws)
+        o = [{k: torch.empty(M, dtype=torch.float64, device=DEV) for k in ("dE_dct", "x_kick")}
+             for _ in range(2)]
+        K.wake_mesh_batched([H.desc, Hz.desc], [L.desc] * 2, [P] * 2, p, o, DEV, ws)
+        for k in ("dE_dct", "x_kick"):
+            for v in (z[k], o[0][k], o[1][k]):
+                assert np.array_equal(out[p][k], v.cpu().numpy(), equal_nan=True), (p, k)
+        n = [K.wake_points_evaluated(h.desc, L.desc, P, p, DEV, ws) for h in (H, Hz)]
+        assert 0 < n[1] <= n[0]
