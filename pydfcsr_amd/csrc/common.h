@@ -78,16 +78,86 @@ __host__ __device__ inline int rgi_interval(double v, double g0, double g1, int 
   return i;
 }
 
-__device__ inline double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, DFCSR_WAVE);
+// Lane exchanges of a double as register moves (permlane swaps between and
+// within the halves of a wave, DPP rotations within a row of 16 lanes), not
+// through the LDS unit as ds_bpermute: a wave's sum is 18 vector
+// instructions, and the waves of a workgroup do not queue for the LDS.  Every
+// lane of the wave takes part.
+typedef unsigned Words __attribute__((ext_vector_type(2)));
+
+__device__ inline double from_words(unsigned lo, unsigned hi) {
+  return __hiloint2double((int)hi, (int)lo);
+}
+
+// a <- (lower half of a, lower half of b), b <- (upper half of a, of b)
+__device__ inline void swap_halves(double &a, double &b) {
+  const Words lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(a),
+                                                    (unsigned)__double2loint(b), false, false);
+  const Words hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(a),
+                                                    (unsigned)__double2hiint(b), false, false);
+  a = from_words(lo[0], hi[0]);
+  b = from_words(lo[1], hi[1]);
+}
+
+// rows (16 lanes) 0..3: a <- (a0, b0, a2, b2), b <- (a1, b1, a3, b3)
+__device__ inline void swap_rows(double &a, double &b) {
+  const Words lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(a),
+                                                    (unsigned)__double2loint(b), false, false);
+  const Words hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(a),
+                                                    (unsigned)__double2hiint(b), false, false);
+  a = from_words(lo[0], hi[0]);
+  b = from_words(lo[1], hi[1]);
+}
+
+// v of the lane N below in the row, cyclic
+template <int N>
+__device__ inline double row_rotate(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x120 + N, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x120 + N, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
+// Sum of a row's 16 lanes, in each of them.
+__device__ inline double row_sum(double v) {
+  v += row_rotate<8>(v);
+  v += row_rotate<4>(v);
+  v += row_rotate<2>(v);
+  v += row_rotate<1>(v);
   return v;
 }
 
+__device__ inline double wave_sum(double v) {
+  double u = v;
+  swap_halves(v, u);
+  v += u;
+  u = v;
+  swap_rows(v, u);
+  return row_sum(v + u);
+}
+
+// Sums over the wave of four values with the moves of one and a half: row r
+// of the result holds the sum of value wave_sum4_of(r).
+__device__ inline double wave_sum4(double a, double b, double c, double d) {
+  swap_halves(a, b);
+  a += b;
+  swap_halves(c, d);
+  c += d;
+  swap_rows(a, c);
+  return row_sum(a + c);
+}
+__device__ inline int wave_sum4_of(int row) { return (row >> 1) | ((row & 1) << 1); }
+
 __device__ inline double wave_max(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, DFCSR_WAVE));
-  return v;
+  double u = v;
+  swap_halves(v, u);
+  v = fmax(v, u);
+  u = v;
+  swap_rows(v, u);
+  v = fmax(v, u);
+  v = fmax(v, row_rotate<8>(v));
+  v = fmax(v, row_rotate<4>(v));
+  v = fmax(v, row_rotate<2>(v));
+  return fmax(v, row_rotate<1>(v));
 }
 
 // Deterministic block sum (fixed tree), result valid in all threads.

@@ -65,6 +65,46 @@ def test_deposit_forms(K, ws, bins, n):
         assert rel_max(v3.cpu(), O.histogram_cic_2d(x[ok], z[ok], bad[ok], *a)) <= 1e-13
 
 
+# one workgroup's pair tile (2048) less and more one, its last workgroup
+# holding one particle, and past one tile and two a workgroup of the full grid
+@pytest.mark.parametrize("n", [2, 3, 5, 2047, 2048, 2049, 4097, 524287, 524289, 1048577, 1572865])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_moments_forms(K, ws, n, offset):
+    """Moments and statistics against the oracle's numpy ones: rows on and off
+    16 bytes, a tilted bunch.  Both sides sum n float64 terms in trees of some
+    20 levels, and x_transform takes 10 sigma_z from x: 1e-12 of the largest
+    value summed (1e-11 for sigma_energy and the slope, squares and quotients
+    of such sums).  Counts equal, repeated bit for bit, NaN kept."""
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((6, n)) * (10.0 ** -np.arange(6))[:, None] + 0.3
+    X[4] = rng.normal(2e-5, 1e-3, n)
+    X[0] = 10.0 * X[4] + rng.normal(1e-3, 1e-3, n)
+    X[5] = rng.normal(2e-3, 1e-3, n)
+    coords = torch.empty(6 * n + 1, dtype=torch.float64, device=DEV)[offset:6 * n + offset].view(6, n)
+    coords.copy_(_t(X))
+    m, ref = K.beam_moments(coords[0], coords[4], ws), O.beam_moments(X[0], X[4])
+    big = np.abs(X[0]).max()
+    for k in ("mean_x", "mean_z", "sigma_x", "sigma_z", "mean_xt", "sigma_xt", "slice_sigma_x"):
+        near = abs(m[k] - ref[k]) <= 1e-12 * max(abs(ref[k]), big)
+        assert near or (np.isnan(m[k]) and np.isnan(ref[k])), (k, m[k], ref[k])
+    assert np.allclose(m["slope"], ref["slope"], rtol=1e-11, atol=1e-12 * big)
+    assert m["n_slice"] == ref["n_slice"]
+    m2 = K.beam_moments(coords[0], coords[4], ws)
+    assert all(np.array_equal(m2[k], m[k], equal_nan=True) for k in m)
+    v = K.beam_statistics(coords, 1e8, 510998.95, ws)
+    d, ref = K.statistics_dict(v), O.beam_statistics(*X, 1e8, 510998.95)
+    sd = np.abs(X).max(axis=1)
+    assert (np.abs(d["mean"] - X.mean(axis=1)) <= 1e-12 * sd).all()
+    assert (np.abs(d["cov"] - ref["cov"]) <= 1e-12 * np.outer(sd, sd)).all()
+    for k in ("mean_energy", "sigma_energy"):
+        assert abs(d[k] - ref[k]) <= 1e-11 * abs(ref[k]), k
+    assert torch.equal(v.nan_to_num(), K.beam_statistics(coords, 1e8, 510998.95, ws).nan_to_num())
+    coords[0, n - 1] = float("nan")
+    m = K.beam_moments(coords[0], coords[4], ws)
+    assert np.isnan([m[k] for k in ("mean_x", "sigma_x", "sigma_xt")]).all()
+    assert m["sigma_z"] == m2["sigma_z"]
+
+
 LAT_ELEMENTS = [dict(type="drift", L=0.1, nsep=1), dict(type="dipole", L=0.3, angle=0.05, nsep=1),
                 dict(type="drift", L=0.4, nsep=2), dict(type="dipole", L=0.3, angle=-0.05, nsep=1)]
 
