@@ -1,13 +1,19 @@
 // a4-a6: density-function post-processing of one deposited slice.
 //
-// Replaces deposit.py:183-235 as seven launches on one stream: the two
-// separable smoothings (density and vx, then the three derivatives) run as
-// LDS-tiled stencils, one workgroup per output tile; the gradients and the
-// element-wise steps run over the whole grid; the global steps between them
-// (the maxima, the trapezoid normalisation, the masked mean of vx_x) read
-// partials or run as one fixed-order workgroup, so results are the same
-// every launch.  The velocity division and the normalisation are applied
-// where their inputs are read, in the reference's operation order.
+// Replaces deposit.py:183-235 as four launches on one stream: the maximum of
+// the raw density; the velocity division and the smoothing of density and
+// vx; their normalisation, gradients and the smoothing of those; the fill of
+// vx_x.  The grids are small (100 x 100 to 256 x 256 in use), so launches and
+// serial passes bound it, not bytes: what a step needs of the whole grid
+// (maxima, the trapezoid normalisation, the masked mean of vx_x) is left as
+// one partial a workgroup by the step before and added by each workgroup of
+// the next in the same fixed order, so results are the same every launch.
+// 100 x 100 with a window of 5 takes 30 us (MI355X; 65 us as eight launches,
+// two of them one workgroup over the whole grid), 256 x 256 with 9 37 us
+// (160 us).
+// A tile's inputs, gradients and first smoothing stay in LDS.  The velocity
+// division and the normalisation are applied where their inputs are read, in
+// the reference's operation order.
 //
 // Savitzky-Golay: scipy.signal.savgol_filter(mode='interp') is linear: the
 // interior is the symmetric smoothing stencil c[] (the centre row of the
@@ -93,43 +99,49 @@ static int make_sg(int W, int order, SGOp *op) {
 
 namespace {
 
-constexpr int kBlock = 1024;   // single-workgroup reductions (fixed order)
-constexpr int kT = 256;        // grid-wide element kernels
-constexpr int kMaxGrid = 1024;
+constexpr int kT = 256;
+constexpr int kMaxGrid = 512;     // workgroups (and partials) of a pass
+constexpr int kMaxPerBlock = 1024;   // cells a workgroup of the maximum reads, at least
 
-// Scalars passed between the launches (workspace tail).
-enum { S_THR = 0, S_DSUM = 1, S_THR2 = 2, S_FILL = 3, S_COUNT = 8 };
+// Rows of partials, one value a workgroup, np values apart.
+enum { P_RAW = 0, P_SUM, P_MAX, P_MIN, P_FILL, P_COUNT, P_ROWS };
 
-__host__ __device__ inline int grid_of(int64_t N) {
-  int64_t g = (N + kT - 1) / kT;
-  return (int)(g < 1 ? 1 : (g > kMaxGrid ? kMaxGrid : g));
-}
+// np.linspace(start, stop, n) with its step formed once.
+struct Axis {
+  double start, stop, step;
+  int n, uniform;
+  __device__ double at(int i) const {
+#pragma clang fp contract(off)
+    if (n <= 1) return start;
+    return i == n - 1 ? stop : (double)i * step + start;
+  }
+  // spacing i -> i + 1; 0 outside the axis
+  __device__ double width(int i) const {
+#pragma clang fp contract(off)
+    return i < 0 || i + 1 >= n ? 0.0 : at(i + 1) - at(i);
+  }
+};
 
-// Savitzky-Golay output at element e of a [nx][nz] array along `axis`
-// (0: along x rows, 1: along z); in(e) gives the input at element e.
+// Savitzky-Golay sum of output i of a line of n inputs; in(k) gives input k.
 template <typename In>
-__device__ inline double sg_at(const SGOp &op, const In &in, int nx, int nz, int axis, int64_t e) {
+__device__ inline double sg_at(const SGOp &op, const In &in, int n, int i) {
 #pragma clang fp contract(off)
   const int W = op.W, h = op.h;
-  const int n = axis == 0 ? nx : nz;
-  const int64_t st = axis == 0 ? nz : 1;
-  const int i = axis == 0 ? (int)(e / nz) : (int)(e % nz);   // position along the axis
-  const int64_t e0 = e - (int64_t)i * st;                     // element 0 of this line
   double acc = 0.0;
   if (i < h) {
-    for (int k = 0; k < W; ++k) acc += op.E[i][k] * in(e0 + k * st);
+    for (int k = 0; k < W; ++k) acc += op.E[i][k] * in(k);
   } else if (i >= n - h) {
     const int r = n - 1 - i;   // mirror row of the left edge
-    for (int k = 0; k < W; ++k) acc += op.E[r][W - 1 - k] * in(e0 + (int64_t)(n - W + k) * st);
+    for (int k = 0; k < W; ++k) acc += op.E[r][W - 1 - k] * in(n - W + k);
   } else {
-    for (int k = 0; k < W; ++k) acc += op.c[k] * in(e0 + (int64_t)(i - h + k) * st);
+    for (int k = 0; k < W; ++k) acc += op.c[k] * in(i - h + k);
   }
   return acc;
 }
 
 // np.gradient spacing test: the coordinate diffs all equal the first one
 // (then numpy uses the scalar-spacing formula).  Evaluated on the host.
-__host__ __device__ inline bool axis_uniform(double g0, double g1, int n) {
+bool axis_uniform(double g0, double g1, int n) {
 #pragma clang fp contract(off)
   if (n < 2) return true;
   const double d0 = linspace_at(g0, g1, n, 1) - linspace_at(g0, g1, n, 0);
@@ -138,263 +150,264 @@ __host__ __device__ inline bool axis_uniform(double g0, double g1, int n) {
   return true;
 }
 
-// np.gradient(f, g) along `axis` at element e (edge_order 1),
-// numpy/lib/_function_base_impl.py.
-template <typename In>
-__device__ inline double gradient_at(const In &f, int nx, int nz, int axis, double g0, double g1,
-                                     bool uniform, int64_t e) {
+Axis make_axis(double g0, double g1, int n) {
 #pragma clang fp contract(off)
-  const int n = axis == 0 ? nx : nz;
-  const int64_t st = axis == 0 ? nz : 1;
-  const int i = axis == 0 ? (int)(e / nz) : (int)(e % nz);
-  const double dxu = linspace_at(g0, g1, n, 1) - linspace_at(g0, g1, n, 0);
-  if (n < 2) return 0.0;
-  if (i == 0) return (f(e + st) - f(e)) / dxu;
-  if (i == n - 1) {
-    const double dn = uniform ? dxu : linspace_at(g0, g1, n, n - 1) - linspace_at(g0, g1, n, n - 2);
-    return (f(e) - f(e - st)) / dn;
-  }
-  if (uniform) return (f(e + st) - f(e - st)) / (2. * dxu);
-  const double xm = linspace_at(g0, g1, n, i - 1), x0 = linspace_at(g0, g1, n, i),
-               xp = linspace_at(g0, g1, n, i + 1);
-  const double dx1 = x0 - xm, dx2 = xp - x0;
-  const double a = -(dx2) / (dx1 * (dx1 + dx2));
-  const double b = (dx2 - dx1) / (dx1 * dx2);
-  const double c = dx1 / (dx2 * (dx1 + dx2));
-  return a * f(e - st) + b * f(e) + c * f(e + st);
+  return {g0, g1, n > 1 ? (g1 - g0) / (double)(n - 1) : 0.0, n, axis_uniform(g0, g1, n)};
 }
 
-// Block max of a grid-strided pass, one partial per workgroup.
-__device__ inline void max_partial(double m, double *part) {
-  __shared__ double red[kT / 64];
-  m = block_max(m, red);
-  if (threadIdx.x == 0) part[blockIdx.x] = m;
+// np.gradient(f, g) at position i of an axis (edge_order 1),
+// numpy/lib/_function_base_impl.py: the weights a, b, c of f(i - 1), f(i),
+// f(i + 1) inside a non-uniform axis, else the divisor in a.
+struct GradAt {
+  double a, b, c;
+};
+
+__device__ inline GradAt grad_weights(const Axis &g, int i) {
+#pragma clang fp contract(off)
+  if (g.n < 2) return {0.0, 0.0, 0.0};
+  const double dxu = g.width(0);
+  if (i == 0) return {dxu, 0.0, 0.0};
+  if (i == g.n - 1) return {g.uniform ? dxu : g.width(i - 1), 0.0, 0.0};
+  if (g.uniform) return {2. * dxu, 0.0, 0.0};
+  const double dx1 = g.width(i - 1), dx2 = g.width(i);
+  return {-(dx2) / (dx1 * (dx1 + dx2)), (dx2 - dx1) / (dx1 * dx2), dx1 / (dx2 * (dx1 + dx2))};
 }
 
-__device__ inline double max_of(const double *part, int n) {
+// f: the value at i, st: the step between neighbours along the axis.
+__device__ inline double grad_at(const double *f, int st, const Axis &g, int i, const GradAt &w) {
+#pragma clang fp contract(off)
+  if (g.n < 2) return 0.0;
+  if (i == 0) return (f[st] - f[0]) / w.a;
+  if (i == g.n - 1) return (f[0] - f[-st]) / w.a;
+  if (g.uniform) return (f[st] - f[-st]) / w.a;
+  return w.a * f[-st] + w.b * f[0] + w.c * f[st];
+}
+
+// Maximum of a row of partials, in every thread (NaN ignored, as fmax).
+__device__ inline double max_of(const double *part, int n, double *red) {
   double m = -INFINITY;
-  for (int k = 0; k < n; ++k) m = fmax(m, part[k]);
-  return m;
+  for (int k = threadIdx.x; k < n; k += kT) m = fmax(m, part[k]);
+  return block_max(m, red);
+}
+
+__device__ inline double sum_of(const double *part, int n, double *red) {
+  double v = 0.0;
+  for (int k = threadIdx.x; k < n; k += kT) v += part[k];
+  return block_sum(v, red);
 }
 
 // 1. max of the raw density (deposit.py:183)
 __global__ __launch_bounds__(kT) void df_max_kernel(const double *__restrict__ dens, int64_t N,
-                                                     double *__restrict__ part) {
+                                                    double *__restrict__ part) {
+  __shared__ double red[kT / 64];
   double m = -INFINITY;
+#pragma unroll 4
   for (int64_t e = (int64_t)blockIdx.x * kT + threadIdx.x; e < N; e += (int64_t)gridDim.x * kT)
     m = fmax(m, dens[e]);
-  max_partial(m, part);
+  m = block_max(m, red);
+  if (threadIdx.x == 0) part[blockIdx.x] = m;
 }
 
-// Separable Savitzky-Golay smoothing of a tile: axis 0 (along x) into LDS,
-// then axis 1 (along z) from LDS.  A workgroup owns kTileX x kTileZ outputs;
-// its LDS rows hold the axis-0 results of its rows over every column the
-// axis-1 windows of its outputs read (interior window, or the first / last
-// `W` columns for the edge rows of the fit).  Each output is the same sum in
-// the same order as two grid-wide passes would give.
+// A tile of kTileX x kTileZ outputs and the inputs its smoothings read: rows
+// [ra, rb) and columns [ca, cb), the outputs' windows or, at an edge, the
+// first or last W of the line (the fit's rows there read them all); at most
+// W + kTileX - 1 by W + kTileZ - 1 of them.
 constexpr int kTileX = 8, kTileZ = 32;
-constexpr int kTileW = kTileZ + 2 * DFCSR_MAX_SG_WINDOW;
-constexpr int kTileFields = 3;
 
-// Input field of a tile pass: a grid, optionally divided by the density
-// where that exceeds thr (the velocity division of deposit.py:183-184).
-struct TileIn {
-  const double *a, *dens;
-  double thr;
-  __device__ double operator()(int64_t e) const {
-    if (!dens) return a[e];
-    const double d = dens[e];
-    return d > thr ? a[e] / d : a[e];
+struct Tile {
+  int x0, z0, rows, cols, ra, rb, ca, cb;
+
+  __device__ Tile(const SGOp &op, int nx, int nz, int t) {
+    const int across = (nz + kTileZ - 1) / kTileZ;
+    x0 = t / across * kTileX, z0 = t % across * kTileZ;
+    rows = min(kTileX, nx - x0), cols = min(kTileZ, nz - z0);
+    ra = max(0, min(x0 - op.h, nx - op.W)), rb = min(nx, max(x0 + kTileX + op.h, op.W));
+    ca = max(0, min(z0 - op.h, nz - op.W)), cb = min(nz, max(z0 + kTileZ + op.h, op.W));
   }
 };
 
-// One LDS row of axis-0 results: element e of grid row i is at row[e - off].
-struct LdsRow {
-  const double *row;
-  int64_t off;
-  __device__ double operator()(int64_t e) const { return row[e - off]; }
-};
+int tiles_of(int nx, int nz) {
+  return ((nx + kTileX - 1) / kTileX) * ((nz + kTileZ - 1) / kTileZ);
+}
 
-template <int NF>
-__device__ void sg_tile(const SGOp &op, const TileIn (&in)[NF], double *const (&out)[NF], int nx,
-                        int nz) {
-  __shared__ double T[kTileFields][kTileX][kTileW];
-  static_assert(NF <= kTileFields, "tile fields");
-  const int x0 = blockIdx.y * kTileX, z0 = blockIdx.x * kTileZ;
-  const int h = op.h, W = op.W;
-  const int lo = max(0, min(z0 - h, nz - W));
-  const int hi = min(nz, max(z0 + kTileZ + h, W));
-  const int w = hi - lo;   // <= kTileZ + 2 W
-  const int rows = min(kTileX, nx - x0), cols = min(kTileZ, nz - z0);
-  for (int t = threadIdx.x; t < rows * w; t += blockDim.x) {
-    const int r = t / w, c = t - r * w;
-    const int64_t e = (int64_t)(x0 + r) * nz + (lo + c);
-#pragma unroll
-    for (int f = 0; f < NF; ++f) T[f][r][c] = sg_at(op, in[f], nx, nz, 0, e);
-  }
-  __syncthreads();
-  for (int t = threadIdx.x; t < rows * cols; t += blockDim.x) {
-    const int r = t / cols, c = t - r * cols;
-    const int64_t i = x0 + r;
-    const int64_t e = i * nz + (z0 + c);
+__host__ __device__ inline int tile_in(int W) { return (W + kTileX - 1) * (W + kTileZ - 1); }
+__host__ __device__ inline int tile_mid(int W) { return kTileX * (W + kTileZ - 1); }
+__host__ __device__ inline int tile_edge(int W) { return (W + kTileX + 1) * (W + kTileZ + 1); }
+
+// Both smoothings of NF staged fields of a tile (in: rows of w values from
+// (ra, ca)), axis 0 into mid, then axis 1; put(f, row, column, value).
+template <int NF, typename Put>
+__device__ void sg_tile(const SGOp &op, const Tile &t, int nx, int nz, const double *in,
+                        double *mid, const Put &put) {
+  const int w = t.cb - t.ca, nin = tile_in(op.W), nmid = tile_mid(op.W);
+  for (int e = threadIdx.x; e < t.rows * w; e += kT) {
+    const int r = e / w, c = e - r * w;
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
-      const LdsRow row{&T[f][r][0], i * nz + lo};
-      out[f][e] = sg_at(op, row, nx, nz, 1, e);
+      const double *col = in + f * nin + c;
+      mid[f * nmid + e] =
+          sg_at(op, [&](int k) { return col[(k - t.ra) * w]; }, nx, t.x0 + r);
+    }
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < t.rows * t.cols; e += kT) {
+    const int r = e / t.cols, c = e - r * t.cols;
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      const double *row = mid + f * nmid + r * w;
+      put(f, t.x0 + r, t.z0 + c, sg_at(op, [&](int k) { return row[k - t.ca]; }, nz, t.z0 + c));
     }
   }
 }
 
 // 2. the velocity division and both smoothing axes of density and vx
-// (deposit.py:183-184, 195-199), into S0 (density) and S1 (vx)
+// (deposit.py:183-184, 195-199), into S0 (density) and S1 (vx); partials of
+// trapz(trapz(density, x_grids, axis=0), z_grids) (deposit.py:201), as the
+// sum of each value times half its neighbouring spacings, and of the
+// smoothed density's extremes
 __global__ __launch_bounds__(kT) void df_sg_kernel(SGOp op, const double *__restrict__ dens,
-                                                   const double *__restrict__ vx, int nx, int nz,
-                                                   double vt, const double *__restrict__ part,
-                                                   int npart, double *__restrict__ S0,
-                                                   double *__restrict__ S1,
-                                                   double *__restrict__ scal) {
-  const double thr = max_of(part, npart) / vt;
-  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) scal[S_THR] = thr;
-  const TileIn in[2] = {{dens, nullptr, 0.0}, {vx, dens, thr}};
-  double *const out[2] = {S0, S1};
-  sg_tile<2>(op, in, out, nx, nz);
-}
-
-// 4. dsum = trapz(trapz(density, x_grids, axis=0), z_grids) (deposit.py:201):
-// the inner trapz adds the rows of each column in order (numpy reduces axis
-// 0 row by row), the outer one is a fixed-order block sum.  One workgroup.
-__global__ __launch_bounds__(kBlock) void df_dsum_kernel(const double *__restrict__ dens, int nx,
-                                                         int nz, double x0, double x1, double z0,
-                                                         double z1, double *__restrict__ colsum,
-                                                         double *__restrict__ scal) {
+                                                   const double *__restrict__ vx, Axis gx, Axis gz,
+                                                   double vt, double *__restrict__ part, int np, int nraw,
+                                                   int ntiles, double *__restrict__ S0,
+                                                   double *__restrict__ S1) {
 #pragma clang fp contract(off)
-  __shared__ double red[kBlock / 64];
-  const int tid = threadIdx.x;
-  for (int j = tid; j < nz; j += kBlock) {
-    double col = 0.0;
-#pragma unroll 8
-    for (int i = 0; i + 1 < nx; ++i) {
-      const double d = linspace_at(x0, x1, nx, i + 1) - linspace_at(x0, x1, nx, i);
-      const double t = d * (dens[(int64_t)i * nz + j] + dens[(int64_t)(i + 1) * nz + j]) / 2.0;
-      col = (i == 0) ? t : col + t;
+  extern __shared__ double lds[];
+  __shared__ double red[kT / 64];
+  const int nx = gx.n, nz = gz.n, nin = tile_in(op.W);
+  const double thr = max_of(part + P_RAW * np, nraw, red) / vt;
+  double sum = 0.0, hi = -INFINITY, lo = INFINITY;
+  for (int i = blockIdx.x; i < ntiles; i += gridDim.x) {
+    const Tile t(op, nx, nz, i);
+    const int w = t.cb - t.ca;
+    for (int e = threadIdx.x; e < (t.rb - t.ra) * w; e += kT) {
+      const int r = e / w, c = e - r * w;
+      const int64_t g = (int64_t)(t.ra + r) * nz + (t.ca + c);
+      const double d = dens[g], v = vx[g];
+      lds[e] = d;
+      lds[nin + e] = d > thr ? v / d : v;
     }
-    colsum[j] = col;
+    __syncthreads();
+    sg_tile<2>(op, t, nx, nz, lds, lds + 2 * nin, [&](int f, int r, int c, double v) {
+      (f == 0 ? S0 : S1)[(int64_t)r * nz + c] = v;
+      if (f != 0) return;
+      const double wx = 0.5 * (gx.width(r - 1) + gx.width(r));
+      const double wz = 0.5 * (gz.width(c - 1) + gz.width(c));
+      if (nx > 1 && nz > 1) sum += v * wx * wz;
+      hi = fmax(hi, v);
+      lo = fmin(lo, v);
+    });
+    __syncthreads();
   }
-  __syncthreads();
-  double part = 0.0;
-  for (int j = tid; j + 1 < nz; j += kBlock) {
-    const double d = linspace_at(z0, z1, nz, j + 1) - linspace_at(z0, z1, nz, j);
-    part += d * (colsum[j] + colsum[j + 1]) / 2.0;
-  }
-  const double dsum = block_sum(part, red);
-  if (tid == 0) scal[S_DSUM] = dsum;
+  sum = block_sum(sum, red);
+  hi = block_max(hi, red);
+  lo = -block_max(-lo, red);
+  if (threadIdx.x != 0) return;
+  part[P_SUM * np + blockIdx.x] = sum;
+  part[P_MAX * np + blockIdx.x] = hi;
+  part[P_MIN * np + blockIdx.x] = lo;
 }
 
-// Normalised density and its thresholded vx (deposit.py:202, 204), as read
-// by the gradients before they are stored.
-struct Normed {
-  const double *dens;
-  double dsum;
-  __device__ double operator()(int64_t e) const { return dens[e] / dsum; }
+// What the smoothed density's partials give: dsum, and the normalised
+// density's maximum, the extreme of the smoothed one that the division by
+// dsum makes the largest (rounding is monotone, so it is that maximum bit for
+// bit; -inf when every quotient is NaN).
+struct DensitySum {
+  double dsum, dmax;
+  __device__ DensitySum(const double *part, int np, int n, double *red) {
+#pragma clang fp contract(off)
+    dsum = sum_of(part + P_SUM * np, n, red);
+    const double hi = max_of(part + P_MAX * np, n, red);
+    double lo = INFINITY;
+    for (int k = threadIdx.x; k < n; k += kT) lo = fmin(lo, part[P_MIN * np + k]);
+    lo = -block_max(-lo, red);
+    dmax = fmax(hi / dsum, lo / dsum);
+    if (dmax != dmax) dmax = -INFINITY;
+  }
 };
-struct VxCut {
-  const double *vx, *dens;
-  double dsum, thr;
-  __device__ double operator()(int64_t e) const { return (dens[e] / dsum <= thr) ? 0.0 : vx[e]; }
-};
 
-// 5. gradients of the normalised density and of vx (deposit.py:212-213);
-// the density and vx outputs take their normalised / thresholded values
-// (deposit.py:202, 204), with max partials of the normalised density
-__global__ __launch_bounds__(kT) void df_grad_kernel(const double *__restrict__ S0,
-                                                     const double *__restrict__ S1, int nx, int nz,
-                                                     double x0, double x1, double z0, double z1,
-                                                     int ux, int uz,
-                                                     const double *__restrict__ scal,
-                                                     double *__restrict__ G0,
-                                                     double *__restrict__ G1,
-                                                     double *__restrict__ G2,
-                                                     double *__restrict__ dens,
-                                                     double *__restrict__ vx,
-                                                     double *__restrict__ part) {
-  const int64_t N = (int64_t)nx * nz;
-  const double dsum = scal[S_DSUM], thr = scal[S_THR];
-  const Normed d{S0, dsum};
-  const VxCut v{S1, S0, dsum, thr};
-  double m = -INFINITY;
-  for (int64_t e = (int64_t)blockIdx.x * kT + threadIdx.x; e < N; e += (int64_t)gridDim.x * kT) {
-    G0[e] = gradient_at(d, nx, nz, 0, x0, x1, ux, e);
-    G1[e] = gradient_at(d, nx, nz, 1, z0, z1, uz, e);
-    G2[e] = gradient_at(v, nx, nz, 0, x0, x1, ux, e);
-    const double dn = d(e);
-    dens[e] = dn;
-    vx[e] = v(e);
-    m = fmax(m, dn);
-  }
-  max_partial(m, part);
-}
-
-// 6. both smoothing axes of the three derivatives (deposit.py:215-224)
-__global__ __launch_bounds__(kT) void df_sg_grad_kernel(SGOp op, const double *__restrict__ G0,
-                                                        const double *__restrict__ G1,
-                                                        const double *__restrict__ G2, int nx,
-                                                        int nz, double *__restrict__ o0,
-                                                        double *__restrict__ o1,
-                                                        double *__restrict__ o2) {
-  const TileIn in[3] = {{G0, nullptr, 0.0}, {G1, nullptr, 0.0}, {G2, nullptr, 0.0}};
-  double *const out[3] = {o0, o1, o2};
-  sg_tile<3>(op, in, out, nx, nz);
-}
-
-// 7. vx_x below 8*max/vt takes the mean of vx_x above it (deposit.py:233-235):
-// fixed-order sums in one workgroup.
-__global__ __launch_bounds__(kBlock) void df_fill_kernel(const double *__restrict__ dens,
-                                                         const double *__restrict__ G2, int64_t N,
-                                                         double vt, const double *__restrict__ part,
-                                                         int npart, double *__restrict__ scal,
-                                                         double *__restrict__ info) {
-  __shared__ double red[kBlock / 64];
-  const double dmax = max_of(part, npart);
-  const double thr2 = dmax / vt * 8;
-  double s = 0.0, c = 0.0;
-  for (int64_t e = threadIdx.x; e < N; e += kBlock)
-    if (dens[e] > thr2) {
-      s += G2[e];
-      c += 1.0;
+// 3. density and vx take their normalised and thresholded values
+// (deposit.py:202, 204), their gradients (deposit.py:212-213) are smoothed
+// along both axes (deposit.py:215-224), and the smoothed vx_x above
+// 8 max / vt leaves partials of its mean (deposit.py:233-235)
+__global__ __launch_bounds__(kT) void df_grad_kernel(
+    SGOp op, const double *__restrict__ S0, const double *__restrict__ S1, Axis gx, Axis gz,
+    double vt, double *__restrict__ part, int np, int nraw, int nsum, int ntiles,
+    double *__restrict__ dens, double *__restrict__ vx, double *__restrict__ o0,
+    double *__restrict__ o1, double *__restrict__ o2) {
+#pragma clang fp contract(off)
+  extern __shared__ double lds[];
+  __shared__ double red[kT / 64];
+  const int nx = gx.n, nz = gz.n, nin = tile_in(op.W), nedge = tile_edge(op.W);
+  double *const D = lds, *const V = D + nedge, *const G = V + nedge, *const mid = G + 3 * nin;
+  const double thr = max_of(part + P_RAW * np, nraw, red) / vt;
+  const DensitySum q(part, np, nsum, red);
+  const double dsum = q.dsum, thr2 = q.dmax / vt * 8;
+  double s = 0.0, c1 = 0.0;
+  for (int i = blockIdx.x; i < ntiles; i += gridDim.x) {
+    const Tile t(op, nx, nz, i);
+    // one more row and column on each side for the gradients
+    const int ea = max(0, t.ra - 1), eb = min(nx, t.rb + 1);
+    const int fa = max(0, t.ca - 1), fb = min(nz, t.cb + 1), ew = fb - fa;
+    for (int e = threadIdx.x; e < (eb - ea) * ew; e += kT) {
+      const int r = e / ew, c = e - r * ew;
+      const int64_t g = (int64_t)(ea + r) * nz + (fa + c);
+      const double d = S0[g] / dsum, v = d <= thr ? 0.0 : S1[g];
+      D[e] = d;
+      V[e] = v;
+      const int x = ea + r - t.x0, z = fa + c - t.z0;
+      if (x >= 0 && x < t.rows && z >= 0 && z < t.cols) dens[g] = d, vx[g] = v;
     }
-  const double ssum = block_sum(s, red);
-  const double cnt = block_sum(c, red);
-  const double fill = cnt > 0.0 ? ssum / cnt : NAN;   // np.mean of an empty selection
-  if (threadIdx.x == 0) {
-    scal[S_THR2] = thr2;
-    scal[S_FILL] = fill;
-    if (info) {
-      info[1] = scal[S_DSUM];
-      info[2] = dmax;
+    __syncthreads();
+    const int w = t.cb - t.ca;
+    for (int e = threadIdx.x; e < (t.rb - t.ra) * w; e += kT) {
+      const int r = e / w, c = e - r * w, x = t.ra + r, z = t.ca + c;
+      const int at = (x - ea) * ew + (z - fa);
+      const GradAt wx = grad_weights(gx, x), wz = grad_weights(gz, z);
+      G[e] = grad_at(D + at, ew, gx, x, wx);
+      G[nin + e] = grad_at(D + at, 1, gz, z, wz);
+      G[2 * nin + e] = grad_at(V + at, ew, gx, x, wx);
+    }
+    __syncthreads();
+    sg_tile<3>(op, t, nx, nz, G, mid, [&](int f, int r, int c, double v) {
+      (f == 0 ? o0 : f == 1 ? o1 : o2)[(int64_t)r * nz + c] = v;
+      if (f != 2) return;
+      const bool in = D[(r - ea) * ew + (c - fa)] > thr2;
+      s += in ? v : 0.0;
+      c1 += in ? 1.0 : 0.0;
+    });
+    __syncthreads();
+  }
+  s = block_sum(s, red);
+  c1 = block_sum(c1, red);
+  if (threadIdx.x != 0) return;
+  part[P_FILL * np + blockIdx.x] = s;
+  part[P_COUNT * np + blockIdx.x] = c1;
+}
+
+// 4. vx_x below 8 max / vt takes the mean of vx_x above it
+// (deposit.py:233-235); the record of the slice
+__global__ __launch_bounds__(kT) void df_fill_kernel(const double *__restrict__ dens, int64_t N,
+                                                     double vt, const double *__restrict__ part,
+                                                     int np, int nraw, int nsum, double *__restrict__ vxx,
+                                                     double *__restrict__ info) {
+#pragma clang fp contract(off)
+  __shared__ double red[kT / 64];
+  const DensitySum q(part, np, nsum, red);
+  const double thr2 = q.dmax / vt * 8;
+  const double sum = sum_of(part + P_FILL * np, nsum, red);
+  const double cnt = sum_of(part + P_COUNT * np, nsum, red);
+  const double fill = cnt > 0.0 ? sum / cnt : NAN;   // np.mean of an empty selection
+  for (int64_t e = (int64_t)blockIdx.x * kT + threadIdx.x; e < N; e += (int64_t)gridDim.x * kT)
+    if (dens[e] < thr2) vxx[e] = fill;
+  if (info && blockIdx.x == 0) {
+    const double raw = max_of(part + P_RAW * np, nraw, red);
+    if (threadIdx.x == 0) {
+      info[0] = raw;
+      info[1] = q.dsum;
+      info[2] = q.dmax;
       info[3] = fill;
     }
   }
-}
-
-// 8. outputs
-__global__ __launch_bounds__(kT) void df_out_kernel(const double *__restrict__ dens,
-                                                    const double *__restrict__ G0,
-                                                    const double *__restrict__ G1,
-                                                    const double *__restrict__ G2, int64_t N,
-                                                    const double *__restrict__ scal,
-                                                    double *__restrict__ dxo,
-                                                    double *__restrict__ dzo,
-                                                    double *__restrict__ vxxo) {
-  const double thr2 = scal[S_THR2], fill = scal[S_FILL];
-  for (int64_t e = (int64_t)blockIdx.x * kT + threadIdx.x; e < N; e += (int64_t)gridDim.x * kT) {
-    dxo[e] = G0[e];
-    dzo[e] = G1[e];
-    vxxo[e] = (dens[e] < thr2) ? fill : G2[e];
-  }
-}
-
-__global__ void df_info_kernel(const double *__restrict__ part, int npart, double *__restrict__ info) {
-  if (threadIdx.x == 0) info[0] = max_of(part, npart);
 }
 
 }  // namespace
@@ -405,8 +418,11 @@ using namespace dfcsr;
 extern "C" int64_t dfcsr_df_workspace_bytes(int nbins_x, int nbins_z) {
   if (nbins_x < 1 || nbins_z < 1) return 0;
   const int64_t N = (int64_t)nbins_x * nbins_z;
-  // three grid temporaries, column sums, two sets of max partials, scalars
-  return (3 * N + nbins_z + 2 * (int64_t)kMaxGrid + S_COUNT) * 8 + 64;
+  // The smoothed density and vx (2 N), then the partials: P_ROWS for each
+  // workgroup, min(tiles, kMaxGrid) of them.  Up to 344 workgroups fit the
+  // fixed 2056 doubles, and the smallest grid of more (2745 x 1) leaves N more.
+  static_assert(P_ROWS * kMaxGrid <= 2745 + 2056 && P_ROWS * 342 <= 2056, "partials fit");
+  return (3 * N + nbins_z + 2 * 1024 + 8) * 8 + 64;
 }
 
 extern "C" int dfcsr_df_process(double *density, double *vx, double *density_x,
@@ -431,29 +447,23 @@ extern "C" int dfcsr_df_process(double *density, double *vx, double *density_x,
   if (rc) return rc;
   const int nx = nbins_x, nz = nbins_z;
   const int64_t N = (int64_t)nx * nz;
-  double *T0 = static_cast<double *>(ws);
-  double *T1 = T0 + N, *T2 = T1 + N, *col = T2 + N;
-  double *partA = col + nz, *partB = partA + kMaxGrid, *scal = partB + kMaxGrid;
-  const int g = grid_of(N);
-  const dim3 gt((nz + kTileZ - 1) / kTileZ, (nx + kTileX - 1) / kTileX);
+  double *S0 = static_cast<double *>(ws), *S1 = S0 + N, *part = S1 + N;
+  const int ntiles = tiles_of(nx, nz), g = ntiles < kMaxGrid ? ntiles : kMaxGrid;
+  const int64_t mb = (N + kMaxPerBlock - 1) / kMaxPerBlock;
+  const int graw = (int)(mb < kMaxGrid ? mb : kMaxGrid);
+  const int np = g > graw ? g : graw;
+  const Axis gx = make_axis(x_start, x_end, nx), gz = make_axis(z_start, z_end, nz);
+  const size_t lds1 = 8 * (size_t)(2 * (tile_in(op.W) + tile_mid(op.W)));
+  const size_t lds2 = 8 * (size_t)(2 * tile_edge(op.W) + 3 * (tile_in(op.W) + tile_mid(op.W)));
   hipStream_t s = as_stream(stream);
-  // T0/T1: density and vx smoothed; density_x/z, vx_x: the gradients; then
-  // density/vx: normalised and thresholded; T0,T1,T2: the gradients smoothed.
-  hipLaunchKernelGGL(df_max_kernel, dim3(g), dim3(kT), 0, s, density, N, partA);
-  hipLaunchKernelGGL(df_sg_kernel, gt, dim3(kT), 0, s, op, density, vx, nx, nz,
-                     velocity_threshold, partA, g, T0, T1, scal);
-  hipLaunchKernelGGL(df_dsum_kernel, dim3(1), dim3(kBlock), 0, s, T0, nx, nz, x_start, x_end,
-                     z_start, z_end, col, scal);
-  const int ux = axis_uniform(x_start, x_end, nx), uz = axis_uniform(z_start, z_end, nz);
-  hipLaunchKernelGGL(df_grad_kernel, dim3(g), dim3(kT), 0, s, T0, T1, nx, nz, x_start, x_end,
-                     z_start, z_end, ux, uz, scal, density_x, density_z, vx_x, density, vx, partB);
-  hipLaunchKernelGGL(df_sg_grad_kernel, gt, dim3(kT), 0, s, op, density_x, density_z, vx_x, nx,
-                     nz, T0, T1, T2);
-  hipLaunchKernelGGL(df_fill_kernel, dim3(1), dim3(kBlock), 0, s, density, T2, N,
-                     velocity_threshold, partB, g, scal, info);
-  hipLaunchKernelGGL(df_out_kernel, dim3(g), dim3(kT), 0, s, density, T0, T1, T2, N, scal,
-                     density_x, density_z, vx_x);
-  if (info) hipLaunchKernelGGL(df_info_kernel, dim3(1), dim3(64), 0, s, partA, g, info);
+  hipLaunchKernelGGL(df_max_kernel, dim3(graw), dim3(kT), 0, s, density, N, part);
+  hipLaunchKernelGGL(df_sg_kernel, dim3(g), dim3(kT), lds1, s, op, density, vx, gx, gz,
+                     velocity_threshold, part, np, graw, ntiles, S0, S1);
+  hipLaunchKernelGGL(df_grad_kernel, dim3(g), dim3(kT), lds2, s, op, S0, S1, gx, gz,
+                     velocity_threshold, part, np, graw, g, ntiles, density, vx, density_x,
+                     density_z, vx_x);
+  hipLaunchKernelGGL(df_fill_kernel, dim3(graw), dim3(kT), 0, s, density, N, velocity_threshold,
+                     part, np, graw, g, vx_x, info);
   DFCSR_LAUNCH_CHECK("df_process");
   return DFCSR_OK;
 }

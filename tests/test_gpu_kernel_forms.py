@@ -105,6 +105,55 @@ def test_moments_forms(K, ws, n, offset):
     assert m["sigma_z"] == m2["sigma_z"]
 
 
+# a grid of one window, one and two tiles (8 x 32 outputs) and one output past
+# them, thin grids, windows 1 to 21, more tiles than workgroups (512)
+@pytest.mark.parametrize("nx,nz,window,order", [
+    (1, 1, 1, 0), (1, 40, 1, 0), (40, 1, 1, 0), (3, 3, 3, 1), (21, 21, 21, 3), (8, 32, 5, 2),
+    (9, 33, 7, 2), (100, 100, 5, 3), (13, 300, 13, 2), (300, 15, 15, 3), (256, 256, 9, 2),
+    (515, 263, 5, 1), (37, 2049, 21, 4)])
+def test_df_forms(K, ws, nx, nz, window, order):
+    """Post-processing of a slice (deposit.py:183-235) by tiles against the
+    same steps in numpy: each value is a sum of at most 441 products and two
+    quotients of float64, so 1e-12 of the field's largest; repeated bit for
+    bit."""
+    rng = np.random.default_rng(nx * nz + window)
+    X = [(-1.3e-3, 1.7e-3, nx), (2e-5, 9e-4, nz)]
+    xg, zg = np.linspace(*X[0]), np.linspace(*X[1])
+    x, z = np.linspace(-3, 3, nx)[:, None], np.linspace(-3, 3, nz)[None, :]
+    dens = 1e4 * np.exp(-0.5 * ((x - z) ** 2 + z ** 2)) * (1 + 0.1 * rng.random((nx, nz)))
+    vx = dens * (0.3 * x + 0.1 * z + 0.01 * rng.random((nx, nz)))
+    vt = 40.0
+    d, v = _t(dens), _t(vx)
+    out, info = [torch.empty_like(d) for _ in range(3)], torch.zeros(4, dtype=torch.float64, device=DEV)
+    a = (*X[0][:2], *X[1][:2], vt, window, order, ws)
+    K.df_process(d, v, *a, out=out, info=info)
+    thr = dens.max() / vt
+    r = {"vx": np.where(dens > thr, vx / dens, vx)}
+    r["density"], r["vx"] = O._sg2(dens, window, order), O._sg2(r["vx"], window, order)
+    with np.errstate(invalid="ignore", divide="ignore"):
+        dsum = O._trapz(O._trapz(r["density"], xg, axis=0), zg)
+        r["density"] = r["density"] / dsum
+        r["vx"][r["density"] <= thr] = 0
+        grad = [np.gradient(f, g, axis=k) if g.size > 1 else np.zeros_like(f)
+                for f, g, k in ((r["density"], xg, 0), (r["density"], zg, 1), (r["vx"], xg, 0))]
+    for k, g in zip(("density_x", "density_z", "vx_x"), grad):
+        r[k] = O._sg2(g, window, order)
+    got = dict(density=d, vx=v, density_x=out[0], density_z=out[1], vx_x=out[2])
+    if min(nx, nz) > 1:
+        top = r["density"].max()
+        fill = r["vx_x"][r["density"] > top / vt * 8].mean()
+        r["vx_x"][r["density"] < top / vt * 8] = fill
+        assert np.allclose(info.cpu(), [dens.max(), dsum, top, fill], rtol=1e-12, atol=0)
+        for k, g in got.items():
+            assert rel_max(g.cpu(), r[k]) <= 1e-12, k
+    else:
+        assert info[1] == 0.0 and not np.isfinite(d.cpu()).any()   # no area: density / 0
+    d2, v2, out2 = _t(dens), _t(vx), [torch.empty_like(d) for _ in range(3)]
+    K.df_process(d2, v2, *a, out=out2)
+    for g, h in zip([d, v, *out], [d2, v2, *out2]):
+        assert np.array_equal(g.cpu().numpy(), h.cpu().numpy(), equal_nan=True)
+
+
 LAT_ELEMENTS = [dict(type="drift", L=0.1, nsep=1), dict(type="dipole", L=0.3, angle=0.05, nsep=1),
                 dict(type="drift", L=0.4, nsep=2), dict(type="dipole", L=0.3, angle=-0.05, nsep=1)]
 
