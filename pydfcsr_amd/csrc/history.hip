@@ -24,107 +24,135 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kMaxJobs = 4096;
 
-// per-job mean of the raw vx_x field (np.mean(vx_x), deposit.py:332, 384)
-__global__ __launch_bounds__(kThreads) void vxx_mean_kernel(const double *__restrict__ src,
-                                                            int64_t slot_stride,
-                                                            const DfcsrRegridJob *__restrict__ jobs,
-                                                            double *__restrict__ means) {
-  __shared__ double red[kThreads / 64];
-  const DfcsrRegridJob J = jobs[blockIdx.x];
+// Jobs of one launch, as a kernel argument: no copy of them on the stream.
+constexpr int kJobs = 64;
+struct RegridJobs {
+  DfcsrRegridJob j[kJobs];
+};
+static_assert(sizeof(RegridJobs) <= 3584, "kernel arguments");
+
+// per-job mean of the raw vx_x field (np.mean(vx_x), deposit.py:332, 384):
+// one workgroup a job, wide enough that a 100 x 100 slice is ten loads in
+// flight a thread (12 us as 256 threads, 5 us now)
+constexpr int kMeanThreads = 1024;
+
+__global__ __launch_bounds__(kMeanThreads) void vxx_mean_kernel(const double *__restrict__ src,
+                                                                int64_t slot_stride,
+                                                                RegridJobs jobs,
+                                                                double *__restrict__ means) {
+  __shared__ double red[kMeanThreads / 64];
+  const DfcsrRegridJob &J = jobs.j[blockIdx.x];
   const int64_t N = (int64_t)J.nbx * J.nbz;
   const double *f = src + (int64_t)J.src_slot * slot_stride + (int64_t)DFCSR_F_VX_X * N;
   double s = 0.0;
-  for (int64_t e = threadIdx.x; e < N; e += kThreads) s += f[e];
+#pragma unroll 8
+  for (int64_t e = threadIdx.x; e < N; e += kMeanThreads) s += f[e];
   s = block_sum(s, red);
   if (threadIdx.x == 0) means[blockIdx.x] = s / (double)N;
 }
 
-// RegularGridInterpolator value of the five fields of job J at (xq, zq).
-__device__ inline void rgi5(const DfcsrRegridJob &J, const double *__restrict__ base,
-                            double fill_vxx, double xq, double zq, double v[5]) {
+// Where a target coordinate lies on an axis of the slice: its interval and
+// norm distance, i < 0 outside.
+struct AxisAt {
+  int i;
+  double y;
+};
+
+__device__ inline AxisAt axis_at(double q, double g0, double g1, int n) {
 #pragma clang fp contract(off)
-  const int64_t Nsrc = (int64_t)J.nbx * J.nbz;
-  bool oob = !(xq >= J.x0 && xq <= J.x1 && zq >= J.z0 && zq <= J.z1);
-  if (oob || J.nbx < 2 || J.nbz < 2) {
-    for (int f = 0; f < 5; ++f) v[f] = (f == DFCSR_F_VX_X) ? fill_vxx : 0.0;
-    return;
-  }
-  int i = rgi_interval(xq, J.x0, J.x1, J.nbx);
-  int j = rgi_interval(zq, J.z0, J.z1, J.nbz);
-  double gi = linspace_at(J.x0, J.x1, J.nbx, i), gi1 = linspace_at(J.x0, J.x1, J.nbx, i + 1);
-  double gj = linspace_at(J.z0, J.z1, J.nbz, j), gj1 = linspace_at(J.z0, J.z1, J.nbz, j + 1);
-  double y0 = (xq - gi) / (gi1 - gi);
-  double y1 = (zq - gj) / (gj1 - gj);
-  int64_t o = (int64_t)i * J.nbz + j;
-  for (int f = 0; f < 5; ++f) {
-    const double *F = base + (int64_t)f * Nsrc;
-    double r = F[o] * (1 - y0) * (1 - y1);
-    r = r + F[o + 1] * (1 - y0) * y1;
-    r = r + F[o + J.nbz] * y0 * (1 - y1);
-    r = r + F[o + J.nbz + 1] * y0 * y1;
-    v[f] = r;
-  }
+  if (!(q >= g0 && q <= g1) || n < 2) return {-1, 0.0};
+  const int i = rgi_interval(q, g0, g1, n);
+  const double a = linspace_at(g0, g1, n, i), b = linspace_at(g0, g1, n, i + 1);
+  return {i, (q - a) / (b - a)};
 }
 
-// One thread per target record: evaluates the four corner points of the
-// record and writes the corner-packed record into each ring present, and
-// the record's own grid node (its first corner) into each cell-major ring
-// (at the last z also into the row's extra cell, its copy).
+// A tile of kTX x kTZ records a workgroup.  The interval searches and norm
+// distances are one per row and column of the tile, the five fields one per
+// node (the records' last row and column of corners included), held in LDS;
+// the rings are then written in their own order, so that neighbouring lanes
+// store neighbouring bytes: ten lanes a 160-byte record of the float64 ring,
+// whole row pieces of the cell-major rings (their pad cell, a copy of the
+// last one, is the clamped column past the edge).  Bound by the
+// stores, whose records are cap apart (tiles from 4 x 32 to 4 x 128 take the
+// same): one 500 x 500 slice into the float64 rings 23 us (MI355X; 32 with a
+// lane per record evaluating its four corners), into the float32 ones 19 (25).
+constexpr int kTX = 8, kTZ = 32, kNodeX = kTX + 1, kNodeZ = kTZ + 1;
+
 __global__ __launch_bounds__(kThreads) void regrid_kernel(
-    const double *__restrict__ src, int64_t slot_stride, const DfcsrRegridJob *__restrict__ jobs,
+    const double *__restrict__ src, int64_t slot_stride, RegridJobs jobs,
     const double *__restrict__ means, double *__restrict__ h64, float *__restrict__ h32,
     float *__restrict__ h32t, double *__restrict__ c64, float *__restrict__ c32, int Xi, int Zi,
     int cap, double xi0, double xi1, double zi0, double zi1) {
-  const DfcsrRegridJob J = jobs[blockIdx.y];
-  const int64_t cells = (int64_t)Xi * Zi;
-  const double *base = src + (int64_t)J.src_slot * slot_stride;
+#pragma clang fp contract(off)
+  __shared__ AxisAt ax[kNodeX + kNodeZ];
+  __shared__ double v[kNodeX * kNodeZ * 5];
+  const DfcsrRegridJob &J = jobs.j[blockIdx.y];
+  const int across = (Zi + kTZ - 1) / kTZ;
+  const int x0 = (int)blockIdx.x / across * kTX, z0 = (int)blockIdx.x % across * kTZ;
+  const int rows = min(kTX, Xi - x0), cols = min(kTZ, Zi - z0);
+  const int t = threadIdx.x;
+  if (t < kNodeX)
+    ax[t] = axis_at(linspace_at(xi0, xi1, Xi, min(x0 + t, Xi - 1)), J.x0, J.x1, J.nbx);
+  else if (t < kNodeX + kNodeZ)
+    ax[t] = axis_at(linspace_at(zi0, zi1, Zi, min(z0 + t - kNodeX, Zi - 1)), J.z0, J.z1, J.nbz);
   const double fill_vxx = means[blockIdx.y];
-  for (int64_t c = (int64_t)blockIdx.x * kThreads + threadIdx.x; c < cells;
-       c += (int64_t)gridDim.x * kThreads) {
-    const int ix = (int)(c / Zi), iz = (int)(c % Zi);
-    const int ix1 = ix + 1 < Xi ? ix + 1 : ix, iz1 = iz + 1 < Zi ? iz + 1 : iz;
-    const double x0 = linspace_at(xi0, xi1, Xi, ix), x1 = linspace_at(xi0, xi1, Xi, ix1);
-    const double z0 = linspace_at(zi0, zi1, Zi, iz), z1 = linspace_at(zi0, zi1, Zi, iz1);
-    double v[4][5];
-    rgi5(J, base, fill_vxx, x0, z0, v[0]);
-    rgi5(J, base, fill_vxx, x0, z1, v[1]);
-    rgi5(J, base, fill_vxx, x1, z0, v[2]);
-    rgi5(J, base, fill_vxx, x1, z1, v[3]);
-    if (h64) {
-      double2 *d2 = reinterpret_cast<double2 *>(h64 + (c * cap + J.dst_slot) * DFCSR_HIST_REC64);
-#pragma unroll
-      for (int f = 0; f < 5; ++f) {
-        d2[2 * f] = make_double2(v[0][f], v[1][f]);
-        d2[2 * f + 1] = make_double2(v[2][f], v[3][f]);
-      }
-    }
-    if (h32t) {
-      float4 *t4 = reinterpret_cast<float4 *>(h32t + (c * cap + J.dst_slot) * DFCSR_HIST_REC32);
-#pragma unroll
-      for (int f = 0; f < 5; ++f)
-        t4[f] = make_float4((float)v[0][f], (float)v[1][f], (float)v[2][f], (float)v[3][f]);
-    }
-    if (h32) {
-      const int64_t blk = (int64_t)ix * cap + J.dst_slot;
-      float4 *s4 = reinterpret_cast<float4 *>(h32) + blk * DFCSR_HIST_CHUNKS32 * Zi + iz;
-#pragma unroll
-      for (int f = 0; f < 5; ++f)
-        s4[f * (int64_t)Zi] = make_float4((float)v[0][f], (float)v[1][f], (float)v[2][f],
-                                          (float)v[3][f]);
-    }
-    const int64_t cell =
-        (((int64_t)J.dst_slot * Xi + ix) * DFCSR_CELL_ROW(Zi) + iz) * DFCSR_CELL;
-    const bool pad = iz == Zi - 1;   // also the row's copy of its last cell
+  const int64_t Nsrc = (int64_t)J.nbx * J.nbz;
+  const double *base = src + (int64_t)J.src_slot * slot_stride;
+  __syncthreads();
+  for (int e = t; e < kNodeX * kNodeZ; e += kThreads) {
+    const AxisAt px = ax[e / kNodeZ], pz = ax[kNodeX + e % kNodeZ];
+    const bool in = px.i >= 0 && pz.i >= 0;
+    const double y0 = px.y, y1 = pz.y;
+    const int64_t o = (int64_t)px.i * J.nbz + pz.i;
 #pragma unroll
     for (int f = 0; f < 5; ++f) {
-      if (c64) {
-        c64[cell + f] = v[0][f];
-        if (pad) c64[cell + DFCSR_CELL + f] = v[0][f];
+      double r = f == DFCSR_F_VX_X ? fill_vxx : 0.0;
+      if (in) {
+        const double *F = base + (int64_t)f * Nsrc + o;
+        r = F[0] * (1 - y0) * (1 - y1);
+        r = r + F[1] * (1 - y0) * y1;
+        r = r + F[J.nbz] * y0 * (1 - y1);
+        r = r + F[J.nbz + 1] * y0 * y1;
       }
-      if (c32) {
-        c32[cell + f] = (float)v[0][f];
-        if (pad) c32[cell + DFCSR_CELL + f] = (float)v[0][f];
-      }
+      v[e * 5 + f] = r;
+    }
+  }
+  __syncthreads();
+  // corner (dx, dz) of field f of record (r, c)
+  auto at = [&](int r, int c, int f) { return v[(r * kNodeZ + c) * 5 + f]; };
+  if (h64)
+    for (int e = t; e < rows * cols * 10; e += kThreads) {
+      const int rec = e / 10, h = e - rec * 10, r = rec / cols, c = rec - r * cols;
+      const int f = h >> 1, d = h & 1;
+      const int64_t cell = (int64_t)(x0 + r) * Zi + (z0 + c);
+      double2 *out = reinterpret_cast<double2 *>(h64 + (cell * cap + J.dst_slot) * DFCSR_HIST_REC64);
+      out[h] = make_double2(at(r + d, c, f), at(r + d, c + 1, f));
+    }
+  if (h32t)
+    for (int e = t; e < rows * cols * 5; e += kThreads) {
+      const int rec = e / 5, f = e - rec * 5, r = rec / cols, c = rec - r * cols;
+      const int64_t cell = (int64_t)(x0 + r) * Zi + (z0 + c);
+      float4 *out = reinterpret_cast<float4 *>(h32t + (cell * cap + J.dst_slot) * DFCSR_HIST_REC32);
+      out[f] = make_float4((float)at(r, c, f), (float)at(r, c + 1, f), (float)at(r + 1, c, f),
+                           (float)at(r + 1, c + 1, f));
+    }
+  if (h32)
+    for (int e = t; e < rows * 5 * cols; e += kThreads) {
+      const int q = e / cols, c = e - q * cols, r = q / 5, f = q - r * 5;
+      const int64_t blk = (int64_t)(x0 + r) * cap + J.dst_slot;
+      float4 *out = reinterpret_cast<float4 *>(h32) + (blk * DFCSR_HIST_CHUNKS32 + f) * Zi + z0 + c;
+      *out = make_float4((float)at(r, c, f), (float)at(r, c + 1, f), (float)at(r + 1, c, f),
+                         (float)at(r + 1, c + 1, f));
+    }
+  if (c64 || c32) {
+    const int w = (cols + (z0 + cols == Zi ? 1 : 0)) * DFCSR_CELL;   // with the pad cell
+    for (int e = t; e < rows * w; e += kThreads) {
+      const int r = e / w, k = e - r * w;
+      const int64_t to =
+          (((int64_t)J.dst_slot * Xi + x0 + r) * DFCSR_CELL_ROW(Zi) + z0) * DFCSR_CELL + k;
+      const double u = v[r * kNodeZ * 5 + k];
+      if (c64) c64[to] = u;
+      if (c32) c32[to] = (float)u;
     }
   }
 }
@@ -169,26 +197,30 @@ template <typename T>
 __device__ inline bool cell_contributes(const T *c) {
   const T big = (T)3.4028234663852886e38;   // FLT_MAX
   const T vx = c[DFCSR_F_VX], vxx = c[DFCSR_F_VX_X];
-  return c[DFCSR_F_DENSITY] != (T)0 || c[DFCSR_F_DENSITY_X] != (T)0 ||
-         c[DFCSR_F_DENSITY_Z] != (T)0 || !(vx <= big && vx >= -big) ||
-         !(vxx <= big && vxx >= -big);
+  // no short circuit: the five loads go out together
+  return (c[DFCSR_F_DENSITY] != (T)0) | (c[DFCSR_F_DENSITY_X] != (T)0) |
+         (c[DFCSR_F_DENSITY_Z] != (T)0) | !((vx <= big) & (vx >= -big)) |
+         !((vxx <= big) & (vxx >= -big));
 }
 
 // x rows per workgroup of zspan_kernel: a step refreshes two slices, so 4
-// rows give 2 x 125 workgroups on a 500-row grid (16 gave 64: 49 us per step)
+// rows give 2 x 125 workgroups on a 500-row grid, and 16 waves take the ten
+// rows of cells these read at once, all fields of four cells a lane together
+// (9 us float64, 6 float32; 17 and 16 with 4 waves and a test field by field)
 constexpr int kSpanRows = 4;
+constexpr int kSpanThreads = 1024;
 
 // zspan entries (x, slot of slice i) for x in one block of kSpanRows rows:
 // each wave finds the z span of whole rows (its own cells) of slices i and
 // i + 1 into LDS, then each entry joins rows x, x + 1 of both slices.
 template <typename T>
-__global__ __launch_bounds__(kThreads) void zspan_kernel(const T *__restrict__ cells,
+__global__ __launch_bounds__(kSpanThreads) void zspan_kernel(const T *__restrict__ cells,
                                                          uint32_t *__restrict__ zspan, int Xi,
                                                          int Zi, int cap, int head, int nt,
                                                          int first) {
   __shared__ int lo_s[2][kSpanRows + 1], hi_s[2][kSpanRows + 1];
   const int xb = blockIdx.x * kSpanRows;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwave = kThreads / 64;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwave = kSpanThreads / 64;
   const int nrow = min(kSpanRows + 1, Xi - xb);   // rows xb .. xb + nrow - 1 (x + 1 clamped)
   const int64_t plane = (int64_t)Xi * DFCSR_CELL_ROW(Zi) * DFCSR_CELL;
   for (int i = first + (int)blockIdx.y; i < nt; i += (int)gridDim.y) {
@@ -198,6 +230,7 @@ __global__ __launch_bounds__(kThreads) void zspan_kernel(const T *__restrict__ c
       const T *row = cells + (int64_t)((head + i + p) % cap) * plane +
                      (int64_t)(xb + r) * DFCSR_CELL_ROW(Zi) * DFCSR_CELL;
       int lo = 0x7fffffff, hi = -1;
+#pragma unroll 4
       for (int z = lane; z < Zi; z += 64) {
         if (cell_contributes(row + (int64_t)z * DFCSR_CELL)) {
           lo = min(lo, z);
@@ -250,10 +283,10 @@ extern "C" int dfcsr_history_zspan(const double *cells, const float *cells32, ui
   if (gy > 1024) gy = 1024;
   hipStream_t s = as_stream(stream);
   if (cells)
-    hipLaunchKernelGGL(zspan_kernel<double>, dim3(gx, gy), dim3(kThreads), 0, s, cells, zspan,
+    hipLaunchKernelGGL(zspan_kernel<double>, dim3(gx, gy), dim3(kSpanThreads), 0, s, cells, zspan,
                        Xi, Zi, cap, head, nt, first);
   else
-    hipLaunchKernelGGL(zspan_kernel<float>, dim3(gx, gy), dim3(kThreads), 0, s, cells32, zspan,
+    hipLaunchKernelGGL(zspan_kernel<float>, dim3(gx, gy), dim3(kSpanThreads), 0, s, cells32, zspan,
                        Xi, Zi, cap, head, nt, first);
   DFCSR_LAUNCH_CHECK("history_zspan");
   return DFCSR_OK;
@@ -312,21 +345,18 @@ extern "C" int dfcsr_regrid(const double *src, int64_t src_slot_stride, const Df
                        J.nbz, J.src_slot, J.dst_slot);
   }
   hipStream_t s = as_stream(stream);
-  // Job descriptors travel in the workspace: written by a host->device copy
-  // ordered on the stream.
-  DfcsrRegridJob *djobs = static_cast<DfcsrRegridJob *>(ws);
-  double *means = reinterpret_cast<double *>(
-      static_cast<char *>(ws) + (((int64_t)njobs * sizeof(DfcsrRegridJob) + 63) / 64) * 64);
-  DFCSR_CHECK_HIP(hipMemcpyAsync(djobs, jobs, (size_t)njobs * sizeof(DfcsrRegridJob),
-                                 hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(vxx_mean_kernel, dim3(njobs), dim3(kThreads), 0, s, src, src_slot_stride,
-                     (const DfcsrRegridJob *)djobs, means);
-  const int64_t npts = (int64_t)Xi * Zi;
-  int gx = (int)((npts + kThreads - 1) / kThreads);
-  if (gx > 2048) gx = 2048;
-  hipLaunchKernelGGL(regrid_kernel, dim3(gx, njobs), dim3(kThreads), 0, s, src, src_slot_stride,
-                     (const DfcsrRegridJob *)djobs, (const double *)means, hist64, hist32, hist32t,
-                     cells, cells32, Xi, Zi, cap, xi0, xi1, zi0, zi1);
+  double *means = static_cast<double *>(ws);
+  const int gx = ((Xi + kTX - 1) / kTX) * ((Zi + kTZ - 1) / kTZ);
+  for (int k = 0; k < njobs; k += kJobs) {
+    const int m = njobs - k < kJobs ? njobs - k : kJobs;
+    RegridJobs J = {};
+    for (int i = 0; i < m; ++i) J.j[i] = jobs[k + i];
+    hipLaunchKernelGGL(vxx_mean_kernel, dim3(m), dim3(kMeanThreads), 0, s, src, src_slot_stride, J,
+                       means + k);
+    hipLaunchKernelGGL(regrid_kernel, dim3(gx, m), dim3(kThreads), 0, s, src, src_slot_stride, J,
+                       (const double *)(means + k), hist64, hist32, hist32t, cells, cells32, Xi, Zi,
+                       cap, xi0, xi1, zi0, zi1);
+  }
   DFCSR_LAUNCH_CHECK("regrid");
   return DFCSR_OK;
 }
