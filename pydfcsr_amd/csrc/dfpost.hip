@@ -8,8 +8,8 @@
 // (maxima, the trapezoid normalisation, the masked mean of vx_x) is left as
 // one partial a workgroup by the step before and added by each workgroup of
 // the next in the same fixed order, so results are the same every launch.
-// 100 x 100 with a window of 5 takes 30 us (MI355X; 65 us as eight launches,
-// two of them one workgroup over the whole grid), 256 x 256 with 9 37 us
+// 100 x 100 with a window of 5 takes 27 us (MI355X; 65 us as eight launches,
+// two of them one workgroup over the whole grid), 256 x 256 with 9 30 us
 // (160 us).
 // A tile's inputs, gradients and first smoothing stay in LDS.  The velocity
 // division and the normalisation are applied where their inputs are read, in
@@ -122,20 +122,34 @@ struct Axis {
   }
 };
 
+// The operator's rows in LDS (a lane's row is its own, and kernel arguments
+// are slow to load by lane): h edge rows, then the interior stencil.
+struct SGRows {
+  const double *c;
+  int W, h;
+};
+
+__host__ __device__ inline int sg_rows_size(int W) { return (W / 2 + 1) * W; }
+
+__device__ inline SGRows sg_rows(const SGOp &op, double *lds) {
+  for (int e = threadIdx.x; e < (op.h + 1) * op.W; e += kT) {
+    const int r = e / op.W, k = e - r * op.W;
+    lds[e] = r == op.h ? op.c[k] : op.E[r][k];
+  }
+  return {lds, op.W, op.h};
+}
+
 // Savitzky-Golay sum of output i of a line of n inputs; in(k) gives input k.
+// The last h rows mirror the left edge's.
 template <typename In>
-__device__ inline double sg_at(const SGOp &op, const In &in, int n, int i) {
+__device__ inline double sg_at(const SGRows &op, const In &in, int n, int i) {
 #pragma clang fp contract(off)
   const int W = op.W, h = op.h;
+  const bool left = i < h, right = !left && i >= n - h;
+  const int from = left ? 0 : right ? n - W : i - h, step = right ? -1 : 1;
+  const double *c = op.c + (left ? i : right ? n - 1 - i : h) * W + (right ? W - 1 : 0);
   double acc = 0.0;
-  if (i < h) {
-    for (int k = 0; k < W; ++k) acc += op.E[i][k] * in(k);
-  } else if (i >= n - h) {
-    const int r = n - 1 - i;   // mirror row of the left edge
-    for (int k = 0; k < W; ++k) acc += op.E[r][W - 1 - k] * in(n - W + k);
-  } else {
-    for (int k = 0; k < W; ++k) acc += op.c[k] * in(i - h + k);
-  }
+  for (int k = 0; k < W; ++k, c += step) acc += *c * in(from + k);
   return acc;
 }
 
@@ -190,12 +204,6 @@ __device__ inline double max_of(const double *part, int n, double *red) {
   return block_max(m, red);
 }
 
-__device__ inline double sum_of(const double *part, int n, double *red) {
-  double v = 0.0;
-  for (int k = threadIdx.x; k < n; k += kT) v += part[k];
-  return block_sum(v, red);
-}
-
 // 1. max of the raw density (deposit.py:183)
 __global__ __launch_bounds__(kT) void df_max_kernel(const double *__restrict__ dens, int64_t N,
                                                     double *__restrict__ part) {
@@ -217,7 +225,7 @@ constexpr int kTileX = 8, kTileZ = 32;
 struct Tile {
   int x0, z0, rows, cols, ra, rb, ca, cb;
 
-  __device__ Tile(const SGOp &op, int nx, int nz, int t) {
+  __device__ Tile(const SGRows &op, int nx, int nz, int t) {
     const int across = (nz + kTileZ - 1) / kTileZ;
     x0 = t / across * kTileX, z0 = t % across * kTileZ;
     rows = min(kTileX, nx - x0), cols = min(kTileZ, nz - z0);
@@ -237,7 +245,7 @@ __host__ __device__ inline int tile_edge(int W) { return (W + kTileX + 1) * (W +
 // Both smoothings of NF staged fields of a tile (in: rows of w values from
 // (ra, ca)), axis 0 into mid, then axis 1; put(f, row, column, value).
 template <int NF, typename Put>
-__device__ void sg_tile(const SGOp &op, const Tile &t, int nx, int nz, const double *in,
+__device__ void sg_tile(const SGRows &op, const Tile &t, int nx, int nz, const double *in,
                         double *mid, const Put &put) {
   const int w = t.cb - t.ca, nin = tile_in(op.W), nmid = tile_mid(op.W);
   for (int e = threadIdx.x; e < t.rows * w; e += kT) {
@@ -265,7 +273,7 @@ __device__ void sg_tile(const SGOp &op, const Tile &t, int nx, int nz, const dou
 // trapz(trapz(density, x_grids, axis=0), z_grids) (deposit.py:201), as the
 // sum of each value times half its neighbouring spacings, and of the
 // smoothed density's extremes
-__global__ __launch_bounds__(kT) void df_sg_kernel(SGOp op, const double *__restrict__ dens,
+__global__ __launch_bounds__(kT) void df_sg_kernel(SGOp arg, const double *__restrict__ dens,
                                                    const double *__restrict__ vx, Axis gx, Axis gz,
                                                    double vt, double *__restrict__ part, int np, int nraw,
                                                    int ntiles, double *__restrict__ S0,
@@ -273,7 +281,8 @@ __global__ __launch_bounds__(kT) void df_sg_kernel(SGOp op, const double *__rest
 #pragma clang fp contract(off)
   extern __shared__ double lds[];
   __shared__ double red[kT / 64];
-  const int nx = gx.n, nz = gz.n, nin = tile_in(op.W);
+  const int nx = gx.n, nz = gz.n, nin = tile_in(arg.W), nmid = tile_mid(arg.W);
+  const SGRows op = sg_rows(arg, lds + 2 * (nin + nmid));
   const double thr = max_of(part + P_RAW * np, nraw, red) / vt;
   double sum = 0.0, hi = -INFINITY, lo = INFINITY;
   for (int i = blockIdx.x; i < ntiles; i += gridDim.x) {
@@ -307,20 +316,37 @@ __global__ __launch_bounds__(kT) void df_sg_kernel(SGOp op, const double *__rest
   part[P_MIN * np + blockIdx.x] = lo;
 }
 
-// What the smoothed density's partials give: dsum, and the normalised
-// density's maximum, the extreme of the smoothed one that the division by
-// dsum makes the largest (rounding is monotone, so it is that maximum bit for
-// bit; -inf when every quotient is NaN).
+// What the partials of the first two passes give: the raw density's maximum,
+// dsum, and the normalised density's maximum, the extreme of the smoothed
+// one that the division by dsum makes the largest (rounding is monotone, so
+// it is that maximum bit for bit; -inf when every quotient is NaN).  One
+// barrier for the four.
 struct DensitySum {
-  double dsum, dmax;
-  __device__ DensitySum(const double *part, int np, int n, double *red) {
+  double raw, dsum, dmax;
+  __device__ DensitySum(const double *part, int np, int nraw, int n) {
 #pragma clang fp contract(off)
-    dsum = sum_of(part + P_SUM * np, n, red);
-    const double hi = max_of(part + P_MAX * np, n, red);
-    double lo = INFINITY;
-    for (int k = threadIdx.x; k < n; k += kT) lo = fmin(lo, part[P_MIN * np + k]);
-    lo = -block_max(-lo, red);
-    dmax = fmax(hi / dsum, lo / dsum);
+    __shared__ double red[4][kT / 64];
+    double v = -INFINITY, s = 0.0, hi = -INFINITY, lo = INFINITY;
+    for (int k = threadIdx.x; k < nraw; k += kT) v = fmax(v, part[P_RAW * np + k]);
+    for (int k = threadIdx.x; k < n; k += kT) {
+      s += part[P_SUM * np + k];
+      hi = fmax(hi, part[P_MAX * np + k]);
+      lo = fmin(lo, part[P_MIN * np + k]);
+    }
+    const double w[4] = {wave_max(v), wave_sum(s), wave_max(hi), wave_max(-lo)};
+#pragma unroll
+    for (int f = 0; f < 4; ++f)
+      if ((threadIdx.x & 63) == 0) red[f][threadIdx.x >> 6] = w[f];
+    __syncthreads();
+    raw = red[0][0], dsum = red[1][0], hi = red[2][0], lo = red[3][0];
+#pragma unroll
+    for (int k = 1; k < kT / 64; ++k) {
+      raw = fmax(raw, red[0][k]);
+      dsum += red[1][k];
+      hi = fmax(hi, red[2][k]);
+      lo = fmax(lo, red[3][k]);
+    }
+    dmax = fmax(hi / dsum, -lo / dsum);
     if (dmax != dmax) dmax = -INFINITY;
   }
 };
@@ -330,18 +356,21 @@ struct DensitySum {
 // along both axes (deposit.py:215-224), and the smoothed vx_x above
 // 8 max / vt leaves partials of its mean (deposit.py:233-235)
 __global__ __launch_bounds__(kT) void df_grad_kernel(
-    SGOp op, const double *__restrict__ S0, const double *__restrict__ S1, Axis gx, Axis gz,
+    SGOp arg, const double *__restrict__ S0, const double *__restrict__ S1, Axis gx, Axis gz,
     double vt, double *__restrict__ part, int np, int nraw, int nsum, int ntiles,
     double *__restrict__ dens, double *__restrict__ vx, double *__restrict__ o0,
     double *__restrict__ o1, double *__restrict__ o2) {
 #pragma clang fp contract(off)
   extern __shared__ double lds[];
   __shared__ double red[kT / 64];
-  const int nx = gx.n, nz = gz.n, nin = tile_in(op.W), nedge = tile_edge(op.W);
+  const int nx = gx.n, nz = gz.n, nin = tile_in(arg.W), nedge = tile_edge(arg.W);
   double *const D = lds, *const V = D + nedge, *const G = V + nedge, *const mid = G + 3 * nin;
-  const double thr = max_of(part + P_RAW * np, nraw, red) / vt;
-  const DensitySum q(part, np, nsum, red);
-  const double dsum = q.dsum, thr2 = q.dmax / vt * 8;
+  double *const rows = mid + 3 * tile_mid(arg.W);
+  GradAt *const wx = reinterpret_cast<GradAt *>(rows + sg_rows_size(arg.W));
+  GradAt *const wz = wx + arg.W + kTileX;
+  const SGRows op = sg_rows(arg, rows);
+  const DensitySum q(part, np, nraw, nsum);
+  const double thr = q.raw / vt, dsum = q.dsum, thr2 = q.dmax / vt * 8;
   double s = 0.0, c1 = 0.0;
   for (int i = blockIdx.x; i < ntiles; i += gridDim.x) {
     const Tile t(op, nx, nz, i);
@@ -357,15 +386,19 @@ __global__ __launch_bounds__(kT) void df_grad_kernel(
       const int x = ea + r - t.x0, z = fa + c - t.z0;
       if (x >= 0 && x < t.rows && z >= 0 && z < t.cols) dens[g] = d, vx[g] = v;
     }
-    __syncthreads();
     const int w = t.cb - t.ca;
+    for (int e = threadIdx.x; e < t.rb - t.ra + w; e += kT) {
+      const int k = e - (t.rb - t.ra);
+      if (k < 0) wx[e] = grad_weights(gx, t.ra + e);
+      else wz[k] = grad_weights(gz, t.ca + k);
+    }
+    __syncthreads();
     for (int e = threadIdx.x; e < (t.rb - t.ra) * w; e += kT) {
       const int r = e / w, c = e - r * w, x = t.ra + r, z = t.ca + c;
       const int at = (x - ea) * ew + (z - fa);
-      const GradAt wx = grad_weights(gx, x), wz = grad_weights(gz, z);
-      G[e] = grad_at(D + at, ew, gx, x, wx);
-      G[nin + e] = grad_at(D + at, 1, gz, z, wz);
-      G[2 * nin + e] = grad_at(V + at, ew, gx, x, wx);
+      G[e] = grad_at(D + at, ew, gx, x, wx[r]);
+      G[nin + e] = grad_at(D + at, 1, gz, z, wz[c]);
+      G[2 * nin + e] = grad_at(V + at, ew, gx, x, wx[r]);
     }
     __syncthreads();
     sg_tile<3>(op, t, nx, nz, G, mid, [&](int f, int r, int c, double v) {
@@ -391,22 +424,24 @@ __global__ __launch_bounds__(kT) void df_fill_kernel(const double *__restrict__ 
                                                      int np, int nraw, int nsum, double *__restrict__ vxx,
                                                      double *__restrict__ info) {
 #pragma clang fp contract(off)
-  __shared__ double red[kT / 64];
-  const DensitySum q(part, np, nsum, red);
+  __shared__ double red[2 * (kT / 64)];
+  double sum = 0.0, cnt = 0.0;
+  for (int k = threadIdx.x; k < nsum; k += kT) {
+    sum += part[P_FILL * np + k];
+    cnt += part[P_COUNT * np + k];
+  }
+  const DensitySum q(part, np, nraw, nsum);
   const double thr2 = q.dmax / vt * 8;
-  const double sum = sum_of(part + P_FILL * np, nsum, red);
-  const double cnt = sum_of(part + P_COUNT * np, nsum, red);
+  sum = block_sum(sum, red);
+  cnt = block_sum(cnt, red + kT / 64);
   const double fill = cnt > 0.0 ? sum / cnt : NAN;   // np.mean of an empty selection
   for (int64_t e = (int64_t)blockIdx.x * kT + threadIdx.x; e < N; e += (int64_t)gridDim.x * kT)
     if (dens[e] < thr2) vxx[e] = fill;
-  if (info && blockIdx.x == 0) {
-    const double raw = max_of(part + P_RAW * np, nraw, red);
-    if (threadIdx.x == 0) {
-      info[0] = raw;
-      info[1] = q.dsum;
-      info[2] = q.dmax;
-      info[3] = fill;
-    }
+  if (info && blockIdx.x == 0 && threadIdx.x == 0) {
+    info[0] = q.raw;
+    info[1] = q.dsum;
+    info[2] = q.dmax;
+    info[3] = fill;
   }
 }
 
@@ -453,8 +488,10 @@ extern "C" int dfcsr_df_process(double *density, double *vx, double *density_x,
   const int graw = (int)(mb < kMaxGrid ? mb : kMaxGrid);
   const int np = g > graw ? g : graw;
   const Axis gx = make_axis(x_start, x_end, nx), gz = make_axis(z_start, z_end, nz);
-  const size_t lds1 = 8 * (size_t)(2 * (tile_in(op.W) + tile_mid(op.W)));
-  const size_t lds2 = 8 * (size_t)(2 * tile_edge(op.W) + 3 * (tile_in(op.W) + tile_mid(op.W)));
+  const int pass = tile_in(op.W) + tile_mid(op.W), rows = sg_rows_size(op.W);
+  const size_t lds1 = 8 * (size_t)(2 * pass + rows);
+  const size_t lds2 = 8 * (size_t)(2 * tile_edge(op.W) + 3 * pass + rows) +
+                      sizeof(GradAt) * (size_t)(2 * op.W + kTileX + kTileZ);
   hipStream_t s = as_stream(stream);
   hipLaunchKernelGGL(df_max_kernel, dim3(graw), dim3(kT), 0, s, density, N, part);
   hipLaunchKernelGGL(df_sg_kernel, dim3(g), dim3(kT), lds1, s, op, density, vx, gx, gz,
