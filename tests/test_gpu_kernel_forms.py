@@ -154,6 +154,50 @@ def test_df_forms(K, ws, nx, nz, window, order):
         assert np.array_equal(g.cpu().numpy(), h.cpu().numpy(), equal_nan=True)
 
 
+# the smallest mesh, one that is no mesh, odd ones, the largest two wakes and
+# the largest one wake that fit the LDS whole, and meshes of which the middle is
+# held: one row too many, thin ones
+@pytest.mark.parametrize("nx,nz,two", [(2, 2, 1), (1, 5, 1), (31, 33, 1), (103, 99, 1),
+                                       (142, 144, 0), (103, 100, 1), (256, 300, 1), (2, 9000, 1),
+                                       (30000, 2, 0)])
+def test_kick_forms(K, nx, nz, two):
+    """The kick with the wakes in LDS (1.25e6 particles or more, 4e6 for dE
+    alone) against the same particles in smaller calls, bit for bit, and against
+    scipy's interpolator within 1e-12 of the largest kick (four products and
+    their sum); particles on and off the mesh's edges, NaN positions."""
+    from scipy.interpolate import RegularGridInterpolator
+    n, few = 1250000 if two else 4000001, 500000
+    rng = np.random.default_rng(nx)
+    x, z = rng.normal(0, 1e-4, n), rng.normal(1e-5, 5e-5, n)
+    xr, zr, slope = (-2e-4, 2.5e-4), (-1e-4, 1.1e-4), (0.7, 1e-6)
+    x[:4] = np.array([*xr, *xr]) + slope[0] * np.array([*zr, 0, 0]) + slope[1]
+    z[:4] = [*zr, 0, 0]
+    x[4:6], z[6:8] = np.nan, [np.nan, np.inf]
+    px, pz = rng.normal(0, 1e-6, n), rng.normal(0, 1e-6, n)
+    w = [rng.normal(0, 1e3, (nx, nz)) for _ in range(2)]
+    d = [_t(w[0]), _t(w[1]) if two else None]
+    whole, parts = [_t(px), _t(pz)], [_t(px), _t(pz)]
+    X, Z, a = _t(x), _t(z), (*xr, *zr, *slope, 0.013, 2e9, two, nx, nz)
+    K.apply_wakes(*whole, X, Z, *d, *a)
+    for k in range(0, n, few):
+        K.apply_wakes(*(v[k:k + few] for v in parts), X[k:k + few], Z[k:k + few], *d, *a)
+    for u, v in zip(whole, parts):
+        assert torch.equal(u, v)
+    xt = x[:few] - (slope[0] * z[:few] + slope[1])
+    for u, v, k in ((whole[1], pz, 0), (whole[0], px, 1)):
+        got = u[:few].cpu().numpy() - v[:few]
+        if min(nx, nz) < 2 or (k and not two):
+            assert (got == 0).all()
+            continue
+        f = RegularGridInterpolator((np.linspace(*xr, nx), np.linspace(*zr, nz)),
+                                    0.013 * w[k] * 1e6 / 2e9, fill_value=0.0, bounds_error=False)
+        ok = np.isfinite(x[:few] + z[:few])
+        ref = f(np.array([xt[ok], z[:few][ok]]).T)
+        # the kick is what is left of px + kick - px: an ulp of px beside it
+        assert np.abs(got[ok] - ref).max() <= 1e-12 * np.abs(ref).max() + 2e-21
+        assert (got[~ok] == 0).all()
+
+
 LAT_ELEMENTS = [dict(type="drift", L=0.1, nsep=1), dict(type="dipole", L=0.3, angle=0.05, nsep=1),
                 dict(type="drift", L=0.4, nsep=2), dict(type="dipole", L=0.3, angle=-0.05, nsep=1)]
 
