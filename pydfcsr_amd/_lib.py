@@ -187,7 +187,18 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 
 def stream_handle(device=None) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The handle of torch.cuda.current_stream(device), without the Stream
+    object around it (2.2 us a call, of which a step makes nine)."""
+    if not isinstance(device, torch.device) or device.type != "cuda":
+        return torch.cuda.current_stream(device).cuda_stream
+    index = torch.cuda.current_device() if device.index is None else device.index
+    return torch._C._cuda_getCurrentRawStream(index)
+
+
+def row_ptrs(t: torch.Tensor) -> list:
+    """Addresses of the rows of a contiguous (k, n) float64 tensor."""
+    p, step = t.data_ptr(), 8 * t.shape[1]
+    return [p + k * step for k in range(t.shape[0])]
 
 
 def require_device_tensor(t: torch.Tensor, dtype=torch.float64, name="tensor"):

@@ -25,11 +25,10 @@ constexpr int kThreads = 256;
 constexpr int kMaxJobs = 4096;
 
 // Jobs of one launch, as a kernel argument: no copy of them on the stream.
-constexpr int kJobs = 64;
+constexpr int kJobs = 16;
 struct RegridJobs {
   DfcsrRegridJob j[kJobs];
 };
-static_assert(sizeof(RegridJobs) <= 3584, "kernel arguments");
 
 // per-job mean of the raw vx_x field (np.mean(vx_x), deposit.py:332, 384):
 // one workgroup a job, wide enough that a 100 x 100 slice is ten loads in

@@ -198,8 +198,7 @@ class DF_tracker:
         else:
             slot, m = self._slot(i), self.log[i]
         n = m.nbx * m.nbz
-        base = self.raw[slot]
-        return [base[f * n:(f + 1) * n].view(m.nbx, m.nbz) for f in range(5)]
+        return list(self.raw[slot][:5 * n].view(5, m.nbx, m.nbz).unbind(0))
 
     # -- deposit.py:145-245 ----------------------------------------------------------
     def get_DF(self, x, z, px, t, moments=None):

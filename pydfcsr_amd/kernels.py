@@ -76,8 +76,7 @@ def beam_statistics(coords: torch.Tensor, p0c, mc2, ws: _lib.Workspace,
         raise DfcsrError("beam_statistics: out must be a contiguous float64 device vector of "
                          f"{_lib.STATS_COUNT}")
     b = ws.get("statistics", lib.dfcsr_beam_statistics_workspace_bytes(n))
-    rows = [coords[k] for k in range(6)]
-    check(lib.dfcsr_beam_statistics(*[ptr(r) for r in rows], n, float(p0c), float(mc2), ptr(b),
+    check(lib.dfcsr_beam_statistics(*_lib.row_ptrs(coords), n, float(p0c), float(mc2), ptr(b),
                                     b.numel(), ptr(out), stream_handle(coords.device)),
           "beam_statistics")
     return out
@@ -109,9 +108,9 @@ def track_element(coords: torch.Tensor, ele: _lib.Element, p0c, mc2):
     _f64(coords, "coords")
     if coords.dim() != 2 or coords.shape[0] != 6:
         raise DfcsrError(f"track_element: coords must be (6, N), got {tuple(coords.shape)}")
-    rows = [ptr(coords[k]) for k in range(6)]
-    check(lib.dfcsr_track_element(*rows, coords.shape[1], ctypes.byref(ele), float(p0c),
-                                  float(mc2), stream_handle(coords.device)), "track_element")
+    check(lib.dfcsr_track_element(*_lib.row_ptrs(coords), coords.shape[1], ctypes.byref(ele),
+                                  float(p0c), float(mc2), stream_handle(coords.device)),
+          "track_element")
     return coords
 
 
