@@ -181,10 +181,16 @@ __device__ inline void mesh_point(const DfcsrWakeParams &P, int i, double &xm, d
 // Groups of G consecutive logical workgroups on one XCD, consecutive groups
 // on consecutive XCDs: the XCDs together sweep the logical order while each
 // L2 sees G neighbours.  Workgroups past the last full round keep their index.
+// kTurn: each round starts one XCD further on.  Without it a mesh whose x bins
+// are a multiple of G gives an XCD the same x in every round, and the work
+// goes with x (near phases of a 32 x 32 mesh, 200 x 200 points, float64: 829
+// us, 28 x 32: 400; with it 450 and 410); whole z lines are dealt evenly
+// without it.
+template <bool kTurn>
 __device__ inline int xcd_group(int b, int nb, int G) {
   const int round = kNumXcd * G;
   if (b >= (nb / round) * round) return b;
-  const int q = b / kNumXcd, x = b % kNumXcd;
+  const int q = b / kNumXcd, x = (b + (kTurn ? q / G : 0)) % kNumXcd;
   return ((q / G) * kNumXcd + x) * G + q % G;
 }
 
@@ -504,10 +510,14 @@ __host__ __device__ inline PhasePlan make_plan(const DfcsrWakeParams &P, int cst
     pl.nA = pl.ch0;
   }
   // By z lines: off the chirp branch (all observers of a line then share rows
-  // and columns), a quarter wave of observers or more.
+  // and columns), from more than a quarter wave of observers (float64) or half
+  // a wave (mixed: the phases' cells are half as large and cached).  Measured,
+  // lines / phases, us, mesh x bins by 32, 200 x 200 points: float64 17: 480 /
+  // 620, 32: 500 / 749, 48: 671 / 1125 (16 by phases 470); mixed 17: 496 / 382,
+  // 32: 494 / 484, 33: 623 / 639, 48: 628 / 733.
   pl.line = false;
   pl.obg = pl.nog = pl.ng = 0;
-  if (cstride && pl.obs_major && pl.nreg == 3 && pl.S <= 2) {
+  if (cstride && pl.obs_major && pl.nreg == 3 && pl.S <= (cstride == kColMixed ? 1 : 2)) {
     pl.line = true;
     pl.obg = pl.nob == 1 ? 1 : (pl.nob == 2 ? 2 : 4);
     pl.nog = (pl.nob + pl.obg - 1) / pl.obg;
@@ -600,6 +610,27 @@ __device__ inline LinAxis load_axis(const double *o) {
   return a;
 }
 
+// A value every lane holds, as a scalar.
+__device__ inline double uniform(double v) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((int)b);
+  const unsigned hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+__device__ inline float uniform(float v) {
+  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+
+__device__ inline LinAxis uniform(const LinAxis &a) {
+  LinAxis u;
+  u.a = uniform(a.a);
+  u.b = uniform(a.b);
+  u.step = uniform(a.step);
+  u.n = __builtin_amdgcn_readfirstlane(a.n);
+  return u;
+}
+
 __device__ inline void observer_point(const WakeTask &T, int i, double *__restrict__ od) {
   double xm, zm;
   mesh_point(T.P, i, xm, zm);
@@ -671,8 +702,8 @@ __device__ void wake_phase(const WakeTask &T, const double *__restrict__ od, int
   const double inv_ds = 1.0 / L.ds;
   int r, j0, j1;
   phase_rows(make_plan(T.P, 0), ph, r, j0, j1);
-  const LinAxis xa = load_axis(od + 16 + 4 * r);
-  const LinAxis sa = load_axis(od + 32 + 4 * r);
+  const LinAxis xa = uniform(load_axis(od + 16 + 4 * r));
+  const LinAxis sa = uniform(load_axis(od + 32 + 4 * r));
   // (all branches below are uniform over the workgroup)
   if (xa.n < 2 || sa.n < 2) {   // trapz over a single sample is 0, NaN or not
     out_z = out_x = 0.0;
@@ -704,17 +735,19 @@ __device__ void wake_phase(const WakeTask &T, const double *__restrict__ od, int
     out_z = out_x = 0.0;
     return;
   }
+  // the observer's values as scalars: 18 vector registers that make room for
+  // a fourth wave
   Observer o;
-  o.s = od[0];
-  o.x = od[1];
+  o.s = uniform(od[0]);
+  o.x = uniform(od[1]);
   o.t = t;
-  o.L.X0 = od[2];
-  o.L.Y0 = od[3];
-  o.L.nx = od[4];
-  o.L.ny = od[5];
-  o.L.tx = od[6];
-  o.L.ty = od[7];
-  o.vx = od[8];
+  o.L.X0 = uniform(od[2]);
+  o.L.Y0 = uniform(od[3]);
+  o.L.nx = uniform(od[4]);
+  o.L.ny = uniform(od[5]);
+  o.L.tx = uniform(od[6]);
+  o.L.ty = uniform(od[7]);
+  o.vx = uniform(od[8]);
   // kSkip (the near regions, whose lookups fall on the newest slices): the
   // span entries of the phase's rows for the newest kSpanPlanes slices
   __shared__ uint32_t zs[kSkip ? kMaxRows : 1][kSpanPlanes];
@@ -749,9 +782,21 @@ __device__ void wake_phase(const WakeTask &T, const double *__restrict__ od, int
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwave = blockDim.x >> 6;
   const int ngroup = (sa.n + 63) >> 6;
+  // Groups of 64 columns to waves: one each where they deal out evenly, or
+  // one to two or four waves that share its rows; else every wave takes every
+  // group and each nwave-th row.  A wave a group in every case left waves idle
+  // with a workgroup's place: float64 on the chirp branch, 64 x 64, 100
+  // columns 2027 -> 1504 us, 150 columns (three groups) 1112 -> 978.  But 200
+  // columns, of which the fourth wave has 8, stay a group a wave: each column's
+  // constants four times took 1888 us against 1724.
+  const bool deal = ngroup % nwave == 0, share = nwave % ngroup == 0;
+  const int rsplit = deal ? 1 : share ? nwave / ngroup : nwave;
+  const int r0 = deal ? 0 : share ? wave / ngroup : wave;
+  const int g0 = deal ? wave : share ? wave % ngroup : 0;
+  const int gstep = deal ? nwave : share ? ngroup : 1;
   double acc_z = 0.0, acc_x = 0.0;
   unsigned evaluated = 0;   // points this lane evaluated (for the optional counter)
-  for (int g = wave; g < ngroup; g += nwave) {
+  for (int g = g0; g < ngroup; g += gstep) {
     // a group of m < 64 columns (the last one) spreads its rows over 64 / m
     // lane sets, so the wave still does a full wave's work
     const int m = min(64, sa.n - 64 * g);
@@ -765,7 +810,7 @@ __device__ void wake_phase(const WakeTask &T, const double *__restrict__ od, int
       const ColumnMixed col = make_column_mixed(L, o, A, sp, inv_ds);
       const double ut0 = (t - A.min_t) * A.it;
       double cz = 0.0, cx = 0.0;
-      for (int r = q; r < v1 - v0; r += nq) {
+      for (int r = q + nq * r0; r < v1 - v0; r += nq * rsplit) {
         if (!rt.ok[r]) continue;
         float Iz, Ix;
         if (!csr_point_mixed<kTI, kCells>(H, A, ut0, col, rt.xp[r], rt.xpf[r], rt.i0[r],
@@ -782,7 +827,7 @@ __device__ void wake_phase(const WakeTask &T, const double *__restrict__ od, int
     } else {
       const Column col = make_column<true>(L, o, sp, inv_ds);
       double cz = 0.0, cx = 0.0;
-      for (int r = q; r < v1 - v0; r += nq) {
+      for (int r = q + nq * r0; r < v1 - v0; r += nq * rsplit) {
         if (!rt.ok[r]) continue;
         const TruncIdx X = {rt.i0[r], rt.i1[r], rt.frac[r], true};
         double Iz, Ix;
@@ -1016,25 +1061,31 @@ __host__ __device__ inline bool cells32_ring32(const DfcsrHistory &H) {
 }
 
 // Workgroups per CU the register allocation must allow: the near phases on
-// the cell-major ring 3 (FP64) or 4 (mixed: 128 registers), the others 2.
+// the cell-major ring 4 (128 registers), the others 2.
 template <bool kMixed, bool kNear, bool kTI, int kCells = kRings>
-__global__ __launch_bounds__(kThreads, kCells ? (kMixed ? 4 : 3) : DFCSR_WAKE_MINBLOCKS) void wake_phase_kernel(
+__global__ __launch_bounds__(kThreads, kCells ? 4 : DFCSR_WAKE_MINBLOCKS) void wake_phase_kernel(
     WakeTask T, double *__restrict__ partials) {
   __shared__ double red[kThreads / 64];
   const int b = blockIdx.x, nb = gridDim.x;
   run_phase_block<kMixed, kNear, kTI, kCells>(
-      T, kNear ? xcd_group(b, nb, kNearGroup) : xcd_remap(b, nb), partials, red);
+      T, kNear ? xcd_group<true>(b, nb, kNearGroup) : xcd_remap(b, nb), partials, red);
 }
 
-// The observer-major region-0 launch: each XCD a contiguous range of z lines.
-// Three workgroups per CU (FP64: 168 VGPRs and a few spilled, against 191 at
-// two; large run FP64 far phases -10 %).  kSkip: the span-table skip
-// (far_skip).
+// The observer-major region-0 launch.  kSkip: the span-table skip (far_skip,
+// the chirp branch).  There whole z lines are dealt round the XCDs, since with
+// the skip the lines near the bunch have most of the work (64 x 64 mesh,
+// float64: 506 us with a contiguous range of lines an XCD, 390 dealt), and
+// float64 fits four workgroups per CU; otherwise each XCD takes a contiguous
+// range (dealt: 0 to 2 % slower) and three workgroups per CU (four: float64
+// 16 x 32 216 -> 238 us; mixed, 32 x 32 on the chirp branch, 141 -> 151 us for
+// the whole wake).
 template <bool kMixed, bool kTI, bool kSkip = false>
-__global__ __launch_bounds__(kThreads, 3) void wake_far_kernel(
+__global__ __launch_bounds__(kThreads, !kMixed && kSkip ? 4 : 3) void wake_far_kernel(
     WakeTask T, double *__restrict__ partials) {
   __shared__ RowTable rt;
-  far_obs_block<kMixed, kTI, kSkip>(T, xcd_remap(blockIdx.x, gridDim.x), partials, rt);
+  const int b = blockIdx.x, nb = gridDim.x;
+  far_obs_block<kMixed, kTI, kSkip>(
+      T, kSkip ? xcd_group<false>(b, nb, nb / T.P.mesh_zbins) : xcd_remap(b, nb), partials, rt);
 }
 
 // Whether a wake's observer-major region 0 skips lookups on the span table:
@@ -1065,8 +1116,9 @@ template <bool kMixed, bool kNear>
 __global__ __launch_bounds__(kThreads, kMixed && kNear ? 4 : DFCSR_WAKE_MINBLOCKS) void wake_phase_batched_kernel(
     const WakeTask *__restrict__ tasks, int ntask, double *__restrict__ partials) {
   __shared__ double red[kThreads / 64];
-  const int b = kNear ? xcd_group(blockIdx.x, gridDim.x, kNearGroup)
-                      : xcd_remap(blockIdx.x, gridDim.x);
+  // (region 0 of tasks of 45, 32 and 19 by 32 mesh points, mixed: 1027 us the
+  // whole wake with a contiguous range an XCD, 870 in groups)
+  const int b = xcd_group<true>(blockIdx.x, gridDim.x, kNearGroup);
   const int j = find_task(tasks, ntask, b,
                           [](const WakeTask &T) { return kNear ? T.blockB0 : T.blockA0; });
   const WakeTask &T = tasks[j];
@@ -1109,14 +1161,18 @@ __global__ __launch_bounds__(kThreads, kMixed && kNear ? 4 : DFCSR_WAKE_MINBLOCK
 }
 
 // Threads per mesh point of the observer launch: the first M of a task's
-// kObsThreads * M compute its observers, and (line form) all of them its z
-// lines' columns, of which there are several per mesh point.
-constexpr int kObsThreads = 8;
+// kObsThreads * M compute its observers, and (line form) the others its z
+// lines' columns, of which there are several per mesh point.  Each is one
+// chain of divisions and dependent loads, so none waits for another's.
+// 8 a point, columns after observers in the same thread: 16.6 us, 21.0 for a
+// batch of three; 16 apart: 8.9 and 15.0 (32 x 32, MI355X).
+constexpr int kObsThreads = 16;
 
 __device__ inline void observer_data(const WakeTask &T, int i, double *__restrict__ partials) {
-  if (i < T.M) observer_point(T, i, partials + obs_at(T, i));
-  if (T.line)
-    for (int e = i; e < 2 * T.P.Nz * T.P.mesh_zbins; e += kObsThreads * T.M)
+  if (i < T.M)
+    observer_point(T, i, partials + obs_at(T, i));
+  else if (T.line)
+    for (int e = i - T.M; e < 2 * T.P.Nz * T.P.mesh_zbins; e += (kObsThreads - 1) * T.M)
       line_column(T, e, partials);
 }
 
@@ -1310,8 +1366,8 @@ void launch_batched(const WakeTask *dt, int k, int forms, dim3 ga, dim3 gb, doub
   if (forms & kFormLine1)
     hipLaunchKernelGGL((wake_line_batched_kernel<kMixed, false, 1>), ga, dim3(kThreads), 0, s, dt,
                        k, lines, part);
-  if (forms & kFormLine2)
-    hipLaunchKernelGGL((wake_line_batched_kernel<kMixed, false, 2>), ga, dim3(kThreads), 0, s, dt,
+  if (!kMixed && (forms & kFormLine2))
+    hipLaunchKernelGGL((wake_line_batched_kernel<false, false, 2>), ga, dim3(kThreads), 0, s, dt,
                        k, lines, part);
   if (forms & kFormPhases)
     hipLaunchKernelGGL((wake_phase_batched_kernel<kMixed, true>), gb, dim3(kThreads), 0, s, dt, k,
@@ -1320,8 +1376,8 @@ void launch_batched(const WakeTask *dt, int k, int forms, dim3 ga, dim3 gb, doub
     hipLaunchKernelGGL((wake_line_batched_kernel<kMixed, true, 1>), gb,
                        dim3(LineSize<1>::kThreads), 0, s, dt,
                        k, lines, part);
-  if (forms & kFormLine2)
-    hipLaunchKernelGGL((wake_line_batched_kernel<kMixed, true, 2>), gb,
+  if (!kMixed && (forms & kFormLine2))
+    hipLaunchKernelGGL((wake_line_batched_kernel<false, true, 2>), gb,
                        dim3(LineSize<2>::kThreads), 0, s, dt,
                        k, lines, part);
 }
@@ -1372,10 +1428,10 @@ extern "C" int dfcsr_wake_mesh(const DfcsrHistory *hist, const DfcsrLattice *lat
   hipLaunchKernelGGL(wake_observer_kernel, go, dim3(kThreads), 0, s, T, part);
   if (pl.line) {
     const bool mixed = precision == DFCSR_PREC_MIXED;
-    auto far = mixed ? (pl.S == 1 ? wake_far_line_kernel<true, 1> : wake_far_line_kernel<true, 2>)
-                     : (pl.S == 1 ? wake_far_line_kernel<false, 1> : wake_far_line_kernel<false, 2>);
-    auto near = mixed ? (pl.S == 1 ? wake_line_kernel<true, 1> : wake_line_kernel<true, 2>)
-                      : (pl.S == 1 ? wake_line_kernel<false, 1> : wake_line_kernel<false, 2>);
+    auto far = mixed ? wake_far_line_kernel<true, 1>
+               : (pl.S == 1 ? wake_far_line_kernel<false, 1> : wake_far_line_kernel<false, 2>);
+    auto near = mixed ? wake_line_kernel<true, 1>
+                : (pl.S == 1 ? wake_line_kernel<false, 1> : wake_line_kernel<false, 2>);
     hipLaunchKernelGGL(far, ga, dim3(kThreads), 0, s, T, part);
     hipLaunchKernelGGL(near, gb, dim3(pl.S == 1 ? LineSize<1>::kThreads : LineSize<2>::kThreads),
                        0, s, T, (const double *)part, part);

@@ -18,13 +18,13 @@
 //     in flight over the points of the current ones.
 // z lines are dealt round the XCDs and rows round the workgroups, since those
 // near the bunch have most of the work (contiguous ranges per XCD: 1.3x
-// slower at 128 x 128).
+// slower at 128 x 128).  The rule is make_plan's.
 // Bound: vector ALU issue, about 95 (float64) and 125 (mixed) instructions a
 // point; near regions 86 % of the issue cycles.  Measured, the phase and
 // observer-major forms and this one: float64 128 x 128 mesh, 355 slices (near
-// 6116 -> 1580 us, region 0 3386 -> 1156 us); float64 32 x 32, 91 slices (804
-// -> 326, 343 -> 190 us); mixed 64 x 57, 187 slices (848 -> 476, 549 -> 356
-// us); three mixed simulations batched (1320 -> 887, 1498 -> 488 us).
+// 5661 and 1610 us, region 0 3386 and 1134 us); float64 32 x 32, 91 slices (436
+// and 320, 343 and 188 us); mixed 64 x 57, 187 slices (868 and 478, 549 and 360
+// us); three mixed simulations batched (1207 and 875, 1282 and 482 us).
 #pragma once
 
 // What one column (fixed s') gives every observer of a z line: r - r' =
@@ -126,19 +126,7 @@ __device__ inline LineColumn load_column(const double *at) {
   return c;
 }
 
-// A value every lane holds, as a scalar.
-__device__ inline double uniform(double v) {
-  const long long b = __double_as_longlong(v);
-  const unsigned lo = __builtin_amdgcn_readfirstlane((int)b);
-  const unsigned hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
 // A column every lane holds the same values of, as scalars.
-__device__ inline float uniform(float v) {
-  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
-}
-
 __device__ inline void uniform_column(LineColumn &c) {
   c.ax = uniform(c.ax), c.ay = uniform(c.ay), c.nx = uniform(c.nx), c.ny = uniform(c.ny);
   c.tx = uniform(c.tx), c.ty = uniform(c.ty), c.rho = uniform(c.rho), c.uz0 = uniform(c.uz0);
@@ -935,7 +923,7 @@ __device__ void far_line_block(const WakeTask &T, int l, double *__restrict__ pa
 // Logical workgroup of a line-form launch: whole z lines dealt round the
 // XCDs, since the lines near the bunch carry most of the work.
 __device__ inline int line_group(const WakeTask &T, int b, int nb) {
-  return xcd_group(b, nb, nb / T.P.mesh_zbins);
+  return xcd_group<false>(b, nb, nb / T.P.mesh_zbins);
 }
 
 template <bool kMixed, int S>

@@ -283,3 +283,35 @@ def test_wake_line_form(K, ws, mesh, nxz, sx, sz, t):
                 assert np.array_equal(out[p][k], v.cpu().numpy(), equal_nan=True), (p, k)
         n = [K.wake_points_evaluated(h.desc, L.desc, P, p, DEV, ws) for h in (H, Hz)]
         assert 0 < n[1] <= n[0]
+
+
+# s' columns in one to five groups of 64, dealt a wave each, shared by two or
+# four waves, or each to all waves; the chirp branch (four regions) and not
+@pytest.mark.parametrize("nz", [5, 64, 65, 128, 150, 200, 256, 257])
+@pytest.mark.parametrize("slope", [0.3, -1.7])
+def test_wake_phase_groups(K, ws, nz, slope):
+    """The wake by phases (a mesh of 5 x bins) against the oracle's C integral,
+    as test_wake_line_form's, and batched bit for bit."""
+    from oracle import csr_ref_c as C
+    from tests.gpu_util import DeviceHistory, DeviceLattice, wake_params
+    sx, sz, t = 50e-6, 50e-6, 0.33
+    T, lat = _History(t, sx, sz), O.LatticeTables(LAT_ELEMENTS)
+    beam = dict(sigma_x=sx, sigma_z=sz, slope=np.array([slope, 1e-6]), mean_x=0.0)
+    args = (t, beam, 0.05, 4.0, 70, nz, 9.0, (-sx, sx, 5), (-sz, sz, 3))
+    H = DeviceHistory(T, DEV, wrap=2, rings=("fp64", "fp32t", "cells", "cells32", "zspan"))
+    L, P = DeviceLattice(lat, DEV), wake_params(*args)
+    keep, ref = C._Keep(), None
+    for p, tol in ((0, 1e-10), (1, 1e-4)):
+        out = K.wake_mesh(H.desc, L.desc, P, p, DEV, ws)
+        if ref is None:
+            obs = np.stack([out["zmesh"].cpu().numpy(), out["xmesh"].cpu().numpy()], axis=1)
+            ref = C.wake(C.hist_from_tracker(T, keep), C.lat_from_tables(lat, keep), t, beam, 0.05,
+                         4.0, 70, nz, 9.0, obs)
+        o = [{k: torch.empty_like(out["dE_dct"]) for k in ("dE_dct", "x_kick")} for _ in range(2)]
+        K.wake_mesh_batched([H.desc] * 2, [L.desc] * 2, [P] * 2, p, o, DEV, ws)
+        for k, r in zip(("dE_dct", "x_kick"), ref):
+            a, ok = out[k].cpu().numpy(), np.isfinite(r)
+            assert np.array_equal(np.isnan(a), np.isnan(r)) and ok.any()
+            assert rel_max(a[ok], r[ok]) <= tol, (p, k)
+            for v in o:
+                assert np.array_equal(a, v[k].cpu().numpy(), equal_nan=True), (p, k)
