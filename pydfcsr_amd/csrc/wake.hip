@@ -463,6 +463,13 @@ constexpr int kLineHead = 24, kColFp64 = 12, kColMixed = 18;
 // the more, the better the rows near the bunch spread over the chip.  128 x
 // 128 float64 near regions: 1728 us with 3072 or 4096, 1920 with 2048.
 constexpr int kLineWgTarget = 4096;
+// Workgroups of its region-0 launch; each wave takes at least one column.
+// Measured, the whole wake with 1024 / 2048 / 4096 / 6144 / 8192: float64 128 x
+// 128 2583 / 2554 / 2634 / 2545 / 2644 us, 32 x 32 496 / 472 / 473 / 472 / 475,
+// 48 x 48 (100 x 100 points) 301 / 276 / 277 / 275 / 279; mixed 64 x 57 787 /
+// 811 / 761 / 748 / 766 (as many as the observer-major form's: 2656, 491, 284,
+// 794).
+constexpr int kLineFarTarget = 6144;
 
 // Doubles per mesh point of a wake by phases: partial sums and observer data.
 __host__ __device__ inline int64_t point_doubles(const PhasePlan &pl) {
@@ -519,6 +526,11 @@ __host__ __device__ inline PhasePlan make_plan(const DfcsrWakeParams &P, int cst
   pl.obg = pl.nog = pl.ng = 0;
   if (cstride && pl.obs_major && pl.nreg == 3 && pl.S <= (cstride == kColMixed ? 1 : 2)) {
     pl.line = true;
+    // region 0: a workgroup's four waves take columns of their own, S rows at a
+    // time
+    const int fl = P.mesh_zbins * pl.nob, fmost = (P.Nz + 3) / 4;
+    const int fq = (kLineFarTarget + fl - 1) / fl;
+    pl.nA = fq > fmost ? fmost : fq;
     pl.obg = pl.nob == 1 ? 1 : (pl.nob == 2 ? 2 : 4);
     pl.nog = (pl.nob + pl.obg - 1) / pl.obg;
     const int64_t lines = (int64_t)P.mesh_zbins * pl.nog * 2;
@@ -553,7 +565,7 @@ __host__ __device__ inline int64_t near_blocks(const PhasePlan &pl, const DfcsrW
 
 // Workgroups of the region-0 launch of one simulation.
 __host__ __device__ inline int64_t far_blocks(const PhasePlan &pl, const DfcsrWakeParams &P) {
-  return pl.obs_major ? (int64_t)P.mesh_zbins * pl.nob * pl.q
+  return pl.obs_major ? (int64_t)P.mesh_zbins * pl.nob * pl.nA
                       : (int64_t)P.mesh_xbins * P.mesh_zbins * pl.nA;
 }
 

@@ -747,16 +747,16 @@ __device__ void far_line_block(const WakeTask &T, int l, double *__restrict__ pa
   const DfcsrHistory &H = T.H;
   const PhasePlan pl = make_plan(T.P, T.cstride);
   const int xb = T.P.mesh_xbins, zb = T.P.mesh_zbins, Nz = T.P.Nz;
-  const int per_line = pl.nob * pl.q;
+  const int per_line = pl.nob * pl.nA;
   const int zl = __builtin_amdgcn_readfirstlane(l / per_line), rem = l - zl * per_line;
-  const int ob = __builtin_amdgcn_readfirstlane(rem / pl.q), g = rem - ob * pl.q;
+  const int ob = __builtin_amdgcn_readfirstlane(rem / pl.nA), g = rem - ob * pl.nA;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sub = lane / W, ol = lane - sub * W;
   const int ix = ob * W + ol;
   const bool valid = ix < xb;
   const int ixa = ob * W, ixb = min(ixa + W, xb) - 1;
-  const int ncb = 4 * pl.q, cb = 4 * g + wave;
+  const int ncb = 4 * pl.nA, cb = 4 * g + wave;
   const int k0 = (int)((int64_t)cb * Nz / ncb), k1 = (int)((int64_t)(cb + 1) * Nz / ncb);
   const HistAxes A = make_axes(H);
   const double inv_ds = 1.0 / T.L.ds;
