@@ -1,9 +1,12 @@
 // a13-a15: the retarded CSR integral on the wake mesh.
 //
 // Replaces CSR2D.get_CSR_mesh / calculate_2D_CSR / get_CSR_wake /
-// get_CSR_integrand (CSR.py:361-782).  A mesh point's integral over its
-// regions (3 without chirp, 4 with) is split into phases: one phase is one
-// region and one chunk of its x' rows, over all s' columns.
+// get_CSR_integrand (CSR.py:361-782).  Off the chirp branch, with cell-major
+// rings and enough x bins (make_plan), a mesh is integrated by z lines
+// (wake_line.h); what follows is the form of every other wake.  A mesh
+// point's integral over its regions (3 without chirp, 4 with) is split into
+// phases: one phase is one region and one chunk of its x' rows, over all s'
+// columns.
 //   observer   : lattice lookups at s, vx at the observer and the region
 //                table, once per mesh point (wake_observer_kernel).
 //   workgroup  = one (mesh point, phase); lanes of a wavefront take
@@ -20,12 +23,13 @@
 //                per phase, then the phases of a mesh point in phase order:
 //                deterministic, the same every launch.
 // Launch order: both launches run the mesh points of one z line phase by
-// phase.  Region 0 (the far region) runs first and each XCD takes a
-// contiguous range (its L2 holds what a z line shares: the same x' rows and
-// retarded planes, nearly the same z').  The near regions' z line shares
+// phase.  Region 0 (the far region) runs first and each XCD takes whole z
+// lines, a contiguous range of them or (chirp branch) every eighth (its L2
+// holds what a z line shares: the same x' rows and retarded planes, nearly
+// the same z').  The near regions' z line shares
 // ~130 MB, more than an L2 but within the 256 MB last-level cache: all XCDs
 // sweep the same z line together, each taking groups of 16 neighbouring
-// workgroups.
+// workgroups, a different one of the round each time.
 #include <mutex>
 #include <type_traits>
 #include <vector>
@@ -439,8 +443,9 @@ __device__ inline bool csr_point_mixed(const DfcsrHistory &H, const HistAxes &A,
 // on the same or neighbouring records.  A workgroup covers one z line, a
 // block of W observers along x (W = 64, or the mesh's x bins rounded up to a
 // power of two) and 4 S column blocks (S = 64 / W lane groups per wave); its
-// row table holds the region's rows inside the history, 64 at a time.  The
-// partial sums of region 0 are then per (observer, column block): nA = nCB.
+// row table holds the region's rows inside the history, 64 at a time.  Its
+// column blocks are added in the workgroup: region 0 leaves nA partial sums an
+// observer, one a workgroup.
 struct PhasePlan {
   int nreg;                 // 3 without chirp, 4 with
   int rows0, ch0, per0;     // region 0 by row chunks: rows, chunks, rows per chunk
@@ -449,6 +454,7 @@ struct PhasePlan {
   bool obs_major;           // region 0 observer-major (mesh observers)
   int W, S, nob, q;         // observer-major: lanes per observer block, column blocks
                             // per wave, observer blocks per z line, workgroups per block
+                            // (those the workspace is sized for; nA are launched)
   bool line;                // the near regions by z lines (line_block)
   int obg, nog, ng;         // line: observer blocks per workgroup, groups of them per z
                             // line, row groups per region
@@ -480,8 +486,10 @@ __host__ __device__ inline int64_t point_doubles(const PhasePlan &pl) {
 // Waves of an observer-major region-0 launch wanted per simulation: about
 // 2048 workgroups of 4 waves, 8 per CU, at most 32 per (z line, observer
 // block).  Measured: the large run (128 x 128, 8 per block) is fastest there
-// and slows with 16 or 32 per block (FP64 12.43 -> 12.51 / 12.65 ms); the
-// chicane (64 x 64) gains from 16 to 32 per block (FP64 6.29 -> 5.97 ms).
+// and slows with 16 or 32 per block (FP64 12.43 -> 12.51 / 12.65 ms).  The chirp
+// branch takes 4096 workgroups (64 x 64, 200 x 200 points, the whole wake with
+// 1024 / 2048 / 4096 / 8192: float64 2077 / 2050 / 1975 / 1974 us, mixed 1417 /
+// 1387 / 1346 / 1351).
 constexpr int kFarWaveTarget = 8192;
 
 // cstride: doubles per column of the line form, 0 when the history lacks the
@@ -511,7 +519,10 @@ __host__ __device__ inline PhasePlan make_plan(const DfcsrWakeParams &P, int cst
     q = q > 32 ? 32 : q;
     q = q > qmax ? (qmax < 1 ? 1 : qmax) : q;
     pl.q = q;
-    pl.nA = q;
+    // the chirp branch, whose workgroups skip most lookups, takes twice as many
+    // where its columns and the workspace of q allow
+    const int64_t chirp = (kFarWaveTarget / 2 + lines - 1) / lines;
+    pl.nA = pl.nreg == 3 ? q : (int)min(chirp, (int64_t)min(qmax < 1 ? 1 : qmax, 4 * pl.S * q));
   } else {
     pl.W = pl.S = pl.nob = pl.q = 0;
     pl.nA = pl.ch0;
@@ -909,9 +920,9 @@ __device__ void far_obs_block(const WakeTask &T, int l, double *__restrict__ par
   const DfcsrLattice &L = T.L;
   const PhasePlan pl = make_plan(T.P, T.cstride);
   const int xb = T.P.mesh_xbins, zb = T.P.mesh_zbins;
-  const int per_line = pl.nob * pl.q;
+  const int per_line = pl.nob * pl.nA;
   const int zl = l / per_line, rem = l - zl * per_line;
-  const int ob = rem / pl.q, g = rem - ob * pl.q;
+  const int ob = rem / pl.nA, g = rem - ob * pl.nA;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int sub = lane / pl.W, ol = lane - sub * pl.W;
   const int ix = ob * pl.W + ol;
@@ -919,7 +930,7 @@ __device__ void far_obs_block(const WakeTask &T, int l, double *__restrict__ par
   const int i = (valid ? ix : ob * pl.W) * zb + zl;   // padding lanes follow the block's first
   const int cb = (4 * g + wave) * pl.S + sub;
   const int Nz = T.P.Nz;
-  const int ncb = 4 * pl.S * pl.q;
+  const int ncb = 4 * pl.S * pl.nA;
   const int k0 = (int)((int64_t)cb * Nz / ncb), k1 = (int)((int64_t)(cb + 1) * Nz / ncb);
   const double *__restrict__ od = partials + obs_at(T, i);
   const double t = T.P.t;
