@@ -229,10 +229,11 @@ __global__ __launch_bounds__(kThreads) void fx_to_double(const int64_t *__restri
 // kQueue (T > 2, where most of a wave's particles miss its tile): the wave
 // scans x alone and queues the hits in LDS; every 64 of them are deposited by
 // a full wave.
-// Measured (both grids, whole call): 1e7 particles on 100 x 100 112 us (544 us
+// Measured (both grids, whole call): 1e7 particles on 100 x 100 114 us (544 us
 // with 48 KB row tiles, which left most lanes idle, and a flush by global
-// atomics), 128 x 128 180 us (801); 3e6 on 256 x 256 106 us (2157 us with 16
-// global atomics a particle, about 17 G atomics/s); 1e5 on 64 x 64 18 us (32).
+// atomics), 5e6 on 128 x 128 95 us; 3e6 on 256 x 256 108 us (2157 us with 16
+// global atomics a particle, about 17 G atomics/s; 114 with two row map reads
+// a scanned particle); 1e5 on 64 x 64 18 us (32).
 constexpr int kTileThreads = 1024;
 constexpr int kLdsBytes = 160 * 1024 - 256;   // a CU's LDS, less the static part
 constexpr int kQueueLen = 128;                                   // per wave
@@ -291,14 +292,16 @@ __global__ __launch_bounds__(kTileThreads) void cic_tile_kernel(
   __shared__ double red[kTileThreads / 64];
   unsigned long long *hi = lds, *lo = lds + cells;
   // first cell of grid row i in the tile, at [i + 1]; -1 when the row is in
-  // another tile or off the grid (i = -1 and nb1)
+  // another tile or off the grid (i = -1 and nb1), -2 when the next row is in
+  // the tile
   int *rowmap = reinterpret_cast<int *>(lds + 2 * (size_t)cells);
   const int grid = blockIdx.y / T, tile = blockIdx.y - grid * T;
   const double *w = grid ? wB : wA;
   for (int e = threadIdx.x; e < 2 * cells; e += kTileThreads) lds[e] = 0ull;
   for (int i = (int)threadIdx.x - 1; i <= nb1; i += kTileThreads) {
-    const int g = i / G;
-    rowmap[i + 1] = (i >= 0 && i < nb1 && g % T == tile) ? ((g / T) * G + (i - g * G)) * nb2 : -1;
+    const int g = i / G, h = (i + 1) / G;
+    const bool in = i >= 0 && i < nb1 && g % T == tile, after = i + 1 < nb1 && h % T == tile;
+    rowmap[i + 1] = in ? ((g / T) * G + (i - g * G)) * nb2 : after ? -2 : -1;
   }
   const FxScale f = fx_scale(w ? max_weight(hdr + 8, npart, red) : 1.0, n);
   if (blockIdx.x == 0 && tile == 0 && threadIdx.x == 0) {
@@ -330,26 +333,32 @@ __global__ __launch_bounds__(kTileThreads) void cic_tile_kernel(
   };
   const int64_t p0 = (int64_t)blockIdx.x * per, p1 = min(p0 + per, n);
   if (!kQueue) {
-    int64_t p = p0 + threadIdx.x;
-    double x = 0.0, z = 0.0, wt = 1.0;
-    if (p < p1) {
-      x = q1[p];
-      z = q2[p];
-      if (w) wt = w[p];
-    }
-    while (p < p1) {   // the next particle's loads in flight over this one's sums
-      const int64_t pn = p + kTileThreads;
-      double xn = 0.0, zn = 0.0, wn = 1.0;
-      if (pn < p1) {
-        xn = q1[pn];
-        zn = q2[pn];
-        if (w) wn = w[pn];
+    // kAhead particles a lane at once, the next kAhead's loads in flight over
+    // their sums (one: 1e7 on 100 x 100 119 us, 5e6 on 128 x 128 102; four: 114
+    // and 95)
+    constexpr int kAhead = 4;
+    struct Batch {
+      double x[kAhead], z[kAhead], w[kAhead];
+    };
+    const auto load = [&](int64_t p, Batch &b) {
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) {
+        const int64_t q = p + k * kTileThreads;
+        const bool in = q < p1;
+        b.x[k] = in ? q1[q] : NAN;   // off the grid
+        b.z[k] = in ? q2[q] : 0.0;
+        b.w[k] = in && w ? w[q] : 1.0;
       }
-      deposit(x, z, fx_weight(wt));
-      p = pn;
-      x = xn;
-      z = zn;
-      wt = wn;
+    };
+    Batch cur, next;
+    int64_t p = p0 + threadIdx.x;
+    load(p, cur);
+    while (p < p1) {
+      p += kAhead * kTileThreads;
+      load(p, next);
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) deposit(cur.x[k], cur.z[k], fx_weight(cur.w[k]));
+      cur = next;
     }
   } else {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -385,7 +394,7 @@ __global__ __launch_bounds__(kTileThreads) void cic_tile_kernel(
         bool hit = c >= -1.0 && c < (double)nb1;
         if (hit) {
           const int i = (int)c;
-          hit = rowmap[i + 1] >= 0 || rowmap[i + 2] >= 0;
+          hit = rowmap[i + 1] != -1;
         }
         const unsigned long long m = __ballot(hit);
         if (hit)
