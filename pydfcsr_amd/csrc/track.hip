@@ -17,7 +17,7 @@
 // five square roots, a dozen divisions) takes as long.  What only the element
 // and the reference momentum enter -- the sines, cosines and tangents of its
 // angles, beta0 -- is formed once on the host: a bend piece of 1e6 particles
-// takes 20 us on MI355X, 4.8 TB/s (50 with these formed for each particle).
+// takes 17.5 us on MI355X, 5.5 TB/s (50 with these formed for each particle).
 #include "common.h"
 
 namespace dfcsr {
@@ -205,6 +205,11 @@ __device__ inline void sextupole(Coords &c, const Piece &m) {
   offset_unset(c, m);
 }
 
+// One kernel an element type: the registers of the one that needs most (quad:
+// the sine and cosine of any angle) would leave the others fewer waves.  1e6
+// particles from HBM, one kernel for all (160 registers) and now: drift 24.6
+// and 16.6 us, bend 25.5 and 21.8, sextupole 35.2 and 31.2, quad 36.7 and 36.3.
+template <int kType>
 __global__ __launch_bounds__(kThreads) void track_kernel(double *__restrict__ x,
                                                          double *__restrict__ px,
                                                          double *__restrict__ y,
@@ -215,12 +220,10 @@ __global__ __launch_bounds__(kThreads) void track_kernel(double *__restrict__ x,
   const int64_t stride = (int64_t)gridDim.x * kThreads;
   for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride) {
     Coords c = {x[i], px[i], y[i], py[i], z[i], pz[i]};
-    switch (m.e.type) {
-      case DFCSR_ELE_DRIFT: drift(c, m.e.L, m.p0c, m.mc2); break;
-      case DFCSR_ELE_SBEND: sbend(c, m); break;
-      case DFCSR_ELE_QUAD: quadrupole(c, m); break;
-      default: sextupole(c, m); break;
-    }
+    if (kType == DFCSR_ELE_DRIFT) drift(c, m.e.L, m.p0c, m.mc2);
+    else if (kType == DFCSR_ELE_SBEND) sbend(c, m);
+    else if (kType == DFCSR_ELE_QUAD) quadrupole(c, m);
+    else sextupole(c, m);
     x[i] = c.x;
     px[i] = c.px;
     y[i] = c.y;
@@ -250,8 +253,12 @@ extern "C" int dfcsr_track_element(double *x, double *px, double *y, double *py,
   if (n <= 0) return DFCSR_OK;
   int64_t b = (n + kThreads - 1) / kThreads;
   if (b > 8192) b = 8192;
-  hipLaunchKernelGGL(track_kernel, dim3((unsigned)b), dim3(kThreads), 0, as_stream(stream), x, px,
-                     y, py, z, pz, n, make_piece(*ele, p0c, mc2));
+  const auto kernel = ele->type == DFCSR_ELE_DRIFT   ? track_kernel<DFCSR_ELE_DRIFT>
+                      : ele->type == DFCSR_ELE_SBEND ? track_kernel<DFCSR_ELE_SBEND>
+                      : ele->type == DFCSR_ELE_QUAD  ? track_kernel<DFCSR_ELE_QUAD>
+                                                     : track_kernel<DFCSR_ELE_SEXTUPOLE>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)b), dim3(kThreads), 0, as_stream(stream), x, px, y, py,
+                     z, pz, n, make_piece(*ele, p0c, mc2));
   DFCSR_LAUNCH_CHECK("track_element");
   return DFCSR_OK;
 }
