@@ -1598,6 +1598,10 @@ extern "C" int dfcsr_wake_batched_launch(const void *dev_tasks, const DfcsrWakeB
   const WakeTask *dt = static_cast<const WakeTask *>(dev_tasks);
   double *part = static_cast<double *>(partials);
   const int k = batch->tasks;
+  // a shape that tells no form (one kept without the field) gets them all: a
+  // form's workgroups return from other forms' tasks
+  const int any = kFormPhases | kFormLine1 | kFormLine2;
+  const int forms = batch->forms > 0 && batch->forms <= any ? batch->forms : any;
   const dim3 ga(batch->blocks_far), gb(batch->blocks_near);
   const dim3 go(point_grid(batch->observers, kObsThreads));
   const dim3 gf(point_grid(batch->observers, kSumLanes));
@@ -1606,9 +1610,9 @@ extern "C" int dfcsr_wake_batched_launch(const void *dev_tasks, const DfcsrWakeB
   if (precision != DFCSR_PREC_FP64 && precision != DFCSR_PREC_MIXED)
     return set_error(DFCSR_EINVAL, "wake_batched_launch: unknown precision %d", precision);
   if (precision == DFCSR_PREC_MIXED)
-    launch_batched<true>(dt, k, batch->forms, ga, gb, part, s);
+    launch_batched<true>(dt, k, forms, ga, gb, part, s);
   else
-    launch_batched<false>(dt, k, batch->forms, ga, gb, part, s);
+    launch_batched<false>(dt, k, forms, ga, gb, part, s);
   hipLaunchKernelGGL(wake_finalize_batched_kernel, gf, dim3(kThreads), 0, s, dt, k,
                      batch->observers, (const double *)part);
   DFCSR_LAUNCH_CHECK("wake_batched_launch");

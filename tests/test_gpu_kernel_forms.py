@@ -315,3 +315,39 @@ def test_wake_phase_groups(K, ws, nz, slope):
             assert rel_max(a[ok], r[ok]) <= tol, (p, k)
             for v in o:
                 assert np.array_equal(a, v[k].cpu().numpy(), equal_nan=True), (p, k)
+
+
+@pytest.mark.parametrize("forms", [0, -1, 8])
+def test_wake_batch_forms_unset(K, ws, forms):
+    """A batch shape that tells no valid form launches them all: tasks of every
+    form (5, 20 and 33 x bins) equal the single launches bit for bit."""
+    import ctypes
+    from pydfcsr_amd import _lib
+    from tests.gpu_util import DeviceHistory, DeviceLattice, wake_params
+    sx, sz, t = 50e-6, 50e-6, 0.33
+    T, lat = _History(t, sx, sz), O.LatticeTables(LAT_ELEMENTS)
+    beam = dict(sigma_x=sx, sigma_z=sz, slope=np.array([0.3, 1e-6]), mean_x=0.0)
+    H = DeviceHistory(T, DEV, wrap=2, rings=("fp64", "fp32t", "cells", "cells32", "zspan"))
+    L, lib = DeviceLattice(lat, DEV), _lib.load()
+    Ps = [wake_params(t, beam, 0.05, 4.0, 70, 65, 9.0, (-sx, sx, m), (-sz, sz, 3))
+          for m in (5, 20, 33)]
+    k = len(Ps)
+    for p in (0, 1):
+        one = [K.wake_mesh(H.desc, L.desc, P, p, DEV, ws) for P in Ps]
+        o = [{n: torch.full_like(w[n], 7.0) for n in ("dE_dct", "x_kick")} for w in one]
+        host = torch.empty(lib.dfcsr_wake_task_table_bytes(k), dtype=torch.uint8)
+        batch = _lib.WakeBatch()
+        _lib.check(lib.dfcsr_wake_tasks_pack(
+            k, (_lib.History * k)(*[H.desc] * k), (_lib.Lattice * k)(*[L.desc] * k),
+            (_lib.WakeParams * k)(*Ps), p, (_lib.c_dp * k)(*[v["dE_dct"].data_ptr() for v in o]),
+            (_lib.c_dp * k)(*[v["x_kick"].data_ptr() for v in o]), host.data_ptr(), host.numel(),
+            ctypes.byref(batch)), "pack")
+        batch.forms = forms
+        dev = host.to(DEV)
+        part = torch.empty(int(batch.partial_bytes), dtype=torch.uint8, device=DEV)
+        _lib.check(lib.dfcsr_wake_batched_launch(
+            dev.data_ptr(), ctypes.byref(batch), p, part.data_ptr(), part.numel(),
+            torch.cuda.current_stream().cuda_stream), "launch")
+        for w, v in zip(one, o):
+            for n in v:
+                assert np.array_equal(w[n].cpu().numpy(), v[n].cpu().numpy(), equal_nan=True), (p, n)
