@@ -8,9 +8,9 @@
 // (maxima, the trapezoid normalisation, the masked mean of vx_x) is left as
 // one partial a workgroup by the step before and added by each workgroup of
 // the next in the same fixed order, so results are the same every launch.
-// 100 x 100 with a window of 5 takes 27 us (MI355X; 65 us as eight launches,
-// two of them one workgroup over the whole grid), 256 x 256 with 9 30 us
-// (160 us).
+// The four kernels with a window of 9 take 24 us at 100 x 100 and 25 us at
+// 256 x 256 (MI355X; as eight launches, two of them one workgroup over the
+// whole grid, 256 x 256 took 160 us).
 // A tile's inputs, gradients and first smoothing stay in LDS.  The velocity
 // division and the normalisation are applied where their inputs are read, in
 // the reference's operation order.
@@ -99,7 +99,14 @@ static int make_sg(int W, int order, SGOp *op) {
 
 namespace {
 
-constexpr int kT = 256;
+// Threads of a workgroup.  There is at most one workgroup a CU at the grids in
+// use, so a launch lasts as long as one chain: 512 threads pass over a tile
+// with its margins (640 inputs at a window of 9) in two rounds where 256 take
+// three, the inputs are on their way while the partials are added, and the
+// fields of a tile are summed side by side.  The second and third kernel at
+// 256 x 256: 7.9 and 13.0 us before, 5.9 and 9.5 with 512 (6.2 and 10.9 with
+// 256, 6.9 and 10.8 with 1024).
+constexpr int kT = 512;
 constexpr int kMaxGrid = 512;     // workgroups (and partials) of a pass
 constexpr int kMaxPerBlock = 1024;   // cells a workgroup of the maximum reads, at least
 
@@ -139,18 +146,23 @@ __device__ inline SGRows sg_rows(const SGOp &op, double *lds) {
   return {lds, op.W, op.h};
 }
 
-// Savitzky-Golay sum of output i of a line of n inputs; in(k) gives input k.
-// The last h rows mirror the left edge's.
-template <typename In>
-__device__ inline double sg_at(const SGRows &op, const In &in, int n, int i) {
+// Savitzky-Golay sums of output i of NF lines of n inputs; in(f, k) gives
+// input k of line f.  The last h rows mirror the left edge's.  The lines go
+// on side by side, so that their reads are in flight together.
+template <int NF, typename In>
+__device__ inline void sg_at(const SGRows &op, const In &in, int n, int i, double (&acc)[NF]) {
 #pragma clang fp contract(off)
   const int W = op.W, h = op.h;
   const bool left = i < h, right = !left && i >= n - h;
   const int from = left ? 0 : right ? n - W : i - h, step = right ? -1 : 1;
   const double *c = op.c + (left ? i : right ? n - 1 - i : h) * W + (right ? W - 1 : 0);
-  double acc = 0.0;
-  for (int k = 0; k < W; ++k, c += step) acc += *c * in(from + k);
-  return acc;
+#pragma unroll
+  for (int f = 0; f < NF; ++f) acc[f] = 0.0;
+#pragma unroll 4
+  for (int k = 0; k < W; ++k, c += step) {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) acc[f] += *c * in(f, from + k);
+  }
 }
 
 // np.gradient spacing test: the coordinate diffs all equal the first one
@@ -195,6 +207,16 @@ __device__ inline double grad_at(const double *f, int st, const Axis &g, int i, 
   if (i == g.n - 1) return (f[0] - f[-st]) / w.a;
   if (g.uniform) return (f[st] - f[-st]) / w.a;
   return w.a * f[-st] + w.b * f[0] + w.c * f[st];
+}
+
+// A wave's values w, the same in its lanes, for every thread to add in the
+// order of the waves.
+template <int N>
+__device__ inline void to_waves(const double (&w)[N], double (&each)[N][kT / 64]) {
+#pragma unroll
+  for (int f = 0; f < N; ++f)
+    if ((threadIdx.x & 63) == 0) each[f][threadIdx.x >> 6] = w[f];
+  __syncthreads();
 }
 
 // Maximum of a row of partials, in every thread (NaN ignored, as fmax).
@@ -248,23 +270,21 @@ template <int NF, typename Put>
 __device__ void sg_tile(const SGRows &op, const Tile &t, int nx, int nz, const double *in,
                         double *mid, const Put &put) {
   const int w = t.cb - t.ca, nin = tile_in(op.W), nmid = tile_mid(op.W);
+  double v[NF];
   for (int e = threadIdx.x; e < t.rows * w; e += kT) {
     const int r = e / w, c = e - r * w;
+    const double *col = in + c;
+    sg_at(op, [&](int f, int k) { return col[f * nin + (k - t.ra) * w]; }, nx, t.x0 + r, v);
 #pragma unroll
-    for (int f = 0; f < NF; ++f) {
-      const double *col = in + f * nin + c;
-      mid[f * nmid + e] =
-          sg_at(op, [&](int k) { return col[(k - t.ra) * w]; }, nx, t.x0 + r);
-    }
+    for (int f = 0; f < NF; ++f) mid[f * nmid + e] = v[f];
   }
   __syncthreads();
   for (int e = threadIdx.x; e < t.rows * t.cols; e += kT) {
     const int r = e / t.cols, c = e - r * t.cols;
+    const double *row = mid + r * w;
+    sg_at(op, [&](int f, int k) { return row[f * nmid + k - t.ca]; }, nz, t.z0 + c, v);
 #pragma unroll
-    for (int f = 0; f < NF; ++f) {
-      const double *row = mid + f * nmid + r * w;
-      put(f, t.x0 + r, t.z0 + c, sg_at(op, [&](int k) { return row[k - t.ca]; }, nz, t.z0 + c));
-    }
+    for (int f = 0; f < NF; ++f) put(f, t.x0 + r, t.z0 + c, v[f]);
   }
 }
 
@@ -280,20 +300,28 @@ __global__ __launch_bounds__(kT) void df_sg_kernel(SGOp arg, const double *__res
                                                    double *__restrict__ S1) {
 #pragma clang fp contract(off)
   extern __shared__ double lds[];
-  __shared__ double red[kT / 64];
+  __shared__ double red[kT / 64], each[3][kT / 64];
   const int nx = gx.n, nz = gz.n, nin = tile_in(arg.W), nmid = tile_mid(arg.W);
   const SGRows op = sg_rows(arg, lds + 2 * (nin + nmid));
-  const double thr = max_of(part + P_RAW * np, nraw, red) / vt;
-  double sum = 0.0, hi = -INFINITY, lo = INFINITY;
-  for (int i = blockIdx.x; i < ntiles; i += gridDim.x) {
-    const Tile t(op, nx, nz, i);
+  const auto stage = [&](const Tile &t) {
     const int w = t.cb - t.ca;
     for (int e = threadIdx.x; e < (t.rb - t.ra) * w; e += kT) {
       const int r = e / w, c = e - r * w;
       const int64_t g = (int64_t)(t.ra + r) * nz + (t.ca + c);
-      const double d = dens[g], v = vx[g];
-      lds[e] = d;
-      lds[nin + e] = d > thr ? v / d : v;
+      lds[e] = dens[g];
+      lds[nin + e] = vx[g];
+    }
+  };
+  stage(Tile(op, nx, nz, blockIdx.x));
+  const double thr = max_of(part + P_RAW * np, nraw, red) / vt;
+  double sum = 0.0, hi = -INFINITY, lo = INFINITY;
+  for (int i = blockIdx.x; i < ntiles; i += gridDim.x) {
+    const Tile t(op, nx, nz, i);
+    if (i != blockIdx.x) stage(t);
+    // each thread divides what it staged
+    for (int e = threadIdx.x; e < (t.rb - t.ra) * (t.cb - t.ca); e += kT) {
+      const double d = lds[e], v = lds[nin + e];
+      if (d > thr) lds[nin + e] = v / d;
     }
     __syncthreads();
     sg_tile<2>(op, t, nx, nz, lds, lds + 2 * nin, [&](int f, int r, int c, double v) {
@@ -307,13 +335,19 @@ __global__ __launch_bounds__(kT) void df_sg_kernel(SGOp arg, const double *__res
     });
     __syncthreads();
   }
-  sum = block_sum(sum, red);
-  hi = block_max(hi, red);
-  lo = -block_max(-lo, red);
+  const double w[3] = {wave_sum(sum), wave_max(hi), wave_max(-lo)};
+  to_waves(w, each);
   if (threadIdx.x != 0) return;
+  sum = each[0][0], hi = each[1][0], lo = each[2][0];
+#pragma unroll
+  for (int k = 1; k < kT / 64; ++k) {
+    sum += each[0][k];
+    hi = fmax(hi, each[1][k]);
+    lo = fmax(lo, each[2][k]);
+  }
   part[P_SUM * np + blockIdx.x] = sum;
   part[P_MAX * np + blockIdx.x] = hi;
-  part[P_MIN * np + blockIdx.x] = lo;
+  part[P_MIN * np + blockIdx.x] = -lo;
 }
 
 // What the partials of the first two passes give: the raw density's maximum,
@@ -334,10 +368,7 @@ struct DensitySum {
       lo = fmin(lo, part[P_MIN * np + k]);
     }
     const double w[4] = {wave_max(v), wave_sum(s), wave_max(hi), wave_max(-lo)};
-#pragma unroll
-    for (int f = 0; f < 4; ++f)
-      if ((threadIdx.x & 63) == 0) red[f][threadIdx.x >> 6] = w[f];
-    __syncthreads();
+    to_waves(w, red);
     raw = red[0][0], dsum = red[1][0], hi = red[2][0], lo = red[3][0];
 #pragma unroll
     for (int k = 1; k < kT / 64; ++k) {
@@ -362,29 +393,48 @@ __global__ __launch_bounds__(kT) void df_grad_kernel(
     double *__restrict__ o1, double *__restrict__ o2) {
 #pragma clang fp contract(off)
   extern __shared__ double lds[];
-  __shared__ double red[kT / 64];
+  __shared__ double each[2][kT / 64];
   const int nx = gx.n, nz = gz.n, nin = tile_in(arg.W), nedge = tile_edge(arg.W);
   double *const D = lds, *const V = D + nedge, *const G = V + nedge, *const mid = G + 3 * nin;
   double *const rows = mid + 3 * tile_mid(arg.W);
   GradAt *const wx = reinterpret_cast<GradAt *>(rows + sg_rows_size(arg.W));
   GradAt *const wz = wx + arg.W + kTileX;
   const SGRows op = sg_rows(arg, rows);
+  // one more row and column on each side for the gradients
+  struct Edge {
+    int ea, fa, eh, ew;
+    __device__ Edge(const Tile &t, int nx, int nz)
+        : ea(max(0, t.ra - 1)), fa(max(0, t.ca - 1)), eh(min(nx, t.rb + 1) - ea),
+          ew(min(nz, t.cb + 1) - fa) {}
+  };
+  const auto stage = [&](const Edge &m) {
+    for (int e = threadIdx.x; e < m.eh * m.ew; e += kT) {
+      const int r = e / m.ew, c = e - r * m.ew;
+      const int64_t g = (int64_t)(m.ea + r) * nz + (m.fa + c);
+      D[e] = S0[g];
+      V[e] = S1[g];
+    }
+  };
+  stage(Edge(Tile(op, nx, nz, blockIdx.x), nx, nz));
   const DensitySum q(part, np, nraw, nsum);
   const double thr = q.raw / vt, dsum = q.dsum, thr2 = q.dmax / vt * 8;
   double s = 0.0, c1 = 0.0;
   for (int i = blockIdx.x; i < ntiles; i += gridDim.x) {
     const Tile t(op, nx, nz, i);
-    // one more row and column on each side for the gradients
-    const int ea = max(0, t.ra - 1), eb = min(nx, t.rb + 1);
-    const int fa = max(0, t.ca - 1), fb = min(nz, t.cb + 1), ew = fb - fa;
-    for (int e = threadIdx.x; e < (eb - ea) * ew; e += kT) {
+    const Edge m(t, nx, nz);
+    const int ea = m.ea, fa = m.fa, ew = m.ew;
+    if (i != blockIdx.x) stage(m);
+    // each thread normalises what it staged
+    for (int e = threadIdx.x; e < m.eh * ew; e += kT) {
       const int r = e / ew, c = e - r * ew;
-      const int64_t g = (int64_t)(ea + r) * nz + (fa + c);
-      const double d = S0[g] / dsum, v = d <= thr ? 0.0 : S1[g];
+      const double d = D[e] / dsum, v = d <= thr ? 0.0 : V[e];
       D[e] = d;
       V[e] = v;
       const int x = ea + r - t.x0, z = fa + c - t.z0;
-      if (x >= 0 && x < t.rows && z >= 0 && z < t.cols) dens[g] = d, vx[g] = v;
+      if (x >= 0 && x < t.rows && z >= 0 && z < t.cols) {
+        const int64_t g = (int64_t)(ea + r) * nz + (fa + c);
+        dens[g] = d, vx[g] = v;
+      }
     }
     const int w = t.cb - t.ca;
     for (int e = threadIdx.x; e < t.rb - t.ra + w; e += kT) {
@@ -410,9 +460,12 @@ __global__ __launch_bounds__(kT) void df_grad_kernel(
     });
     __syncthreads();
   }
-  s = block_sum(s, red);
-  c1 = block_sum(c1, red);
+  const double w[2] = {wave_sum(s), wave_sum(c1)};
+  to_waves(w, each);
   if (threadIdx.x != 0) return;
+  s = each[0][0], c1 = each[1][0];
+#pragma unroll
+  for (int k = 1; k < kT / 64; ++k) s += each[0][k], c1 += each[1][k];
   part[P_FILL * np + blockIdx.x] = s;
   part[P_COUNT * np + blockIdx.x] = c1;
 }
@@ -487,6 +540,8 @@ extern "C" int dfcsr_df_process(double *density, double *vx, double *density_x,
   const int64_t mb = (N + kMaxPerBlock - 1) / kMaxPerBlock;
   const int graw = (int)(mb < kMaxGrid ? mb : kMaxGrid);
   const int np = g > graw ? g : graw;
+  const int64_t fb = (N + kT - 1) / kT;
+  const int fill = (int)(fb < kMaxGrid ? fb : kMaxGrid);
   const Axis gx = make_axis(x_start, x_end, nx), gz = make_axis(z_start, z_end, nz);
   const int pass = tile_in(op.W) + tile_mid(op.W), rows = sg_rows_size(op.W);
   const size_t lds1 = 8 * (size_t)(2 * pass + rows);
@@ -499,7 +554,7 @@ extern "C" int dfcsr_df_process(double *density, double *vx, double *density_x,
   hipLaunchKernelGGL(df_grad_kernel, dim3(g), dim3(kT), lds2, s, op, S0, S1, gx, gz,
                      velocity_threshold, part, np, graw, g, ntiles, density, vx, density_x,
                      density_z, vx_x);
-  hipLaunchKernelGGL(df_fill_kernel, dim3(graw), dim3(kT), 0, s, density, N, velocity_threshold,
+  hipLaunchKernelGGL(df_fill_kernel, dim3(fill), dim3(kT), 0, s, density, N, velocity_threshold,
                      part, np, graw, g, vx_x, info);
   DFCSR_LAUNCH_CHECK("df_process");
   return DFCSR_OK;
