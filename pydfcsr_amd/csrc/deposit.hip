@@ -231,9 +231,8 @@ __global__ __launch_bounds__(kThreads) void fx_to_double(const int64_t *__restri
 // a full wave.
 // Measured (both grids, whole call): 1e7 particles on 100 x 100 114 us (544 us
 // with 48 KB row tiles, which left most lanes idle, and a flush by global
-// atomics), 5e6 on 128 x 128 95 us; 3e6 on 256 x 256 108 us (2157 us with 16
-// global atomics a particle, about 17 G atomics/s; 114 with two row map reads
-// a scanned particle); 1e5 on 64 x 64 18 us (32).
+// atomics), 5e6 on 128 x 128 95 us; 3e6 on 256 x 256 98 us (2157 us with 16
+// global atomics a particle, about 17 G atomics/s); 1e5 on 64 x 64 18 us (32).
 constexpr int kTileThreads = 1024;
 constexpr int kLdsBytes = 160 * 1024 - 256;   // a CU's LDS, less the static part
 constexpr int kQueueLen = 128;                                   // per wave
@@ -255,7 +254,7 @@ struct TilePlan {
 // 8.0 ms and 39 us; kMaxTiles keeps to that range.
 TilePlan tile_plan(int nb1, int nb2) {
   TilePlan p = {0, 0, 0, 0, 0};
-  const int64_t map = (int64_t)(nb1 + 2) * 4 + 16;
+  const int64_t map = (int64_t)(nb1 + 2) * 4 + 16;   // rows -2 to nb1, rounded up
   for (int G = 4; G >= 1; G >>= 1) {
     const int groups = (nb1 + G - 1) / G;
     for (int T = 1; T <= kMaxTiles && T <= groups; ++T) {
@@ -291,17 +290,18 @@ __global__ __launch_bounds__(kTileThreads) void cic_tile_kernel(
   extern __shared__ __align__(16) unsigned long long lds[];
   __shared__ double red[kTileThreads / 64];
   unsigned long long *hi = lds, *lo = lds + cells;
-  // first cell of grid row i in the tile, at [i + 1]; -1 when the row is in
-  // another tile or off the grid (i = -1 and nb1), -2 when the next row is in
-  // the tile
+  // first cell of grid row i in the tile, at [i + 2]; -1 when the row is in
+  // another tile or off the grid (i = -2, -1 and nb1), -2 when the next row is
+  // in the tile
   int *rowmap = reinterpret_cast<int *>(lds + 2 * (size_t)cells);
   const int grid = blockIdx.y / T, tile = blockIdx.y - grid * T;
   const double *w = grid ? wB : wA;
   for (int e = threadIdx.x; e < 2 * cells; e += kTileThreads) lds[e] = 0ull;
-  for (int i = (int)threadIdx.x - 1; i <= nb1; i += kTileThreads) {
+  for (int i = (int)threadIdx.x - 2; i <= nb1; i += kTileThreads) {
     const int g = i / G, h = (i + 1) / G;
-    const bool in = i >= 0 && i < nb1 && g % T == tile, after = i + 1 < nb1 && h % T == tile;
-    rowmap[i + 1] = in ? ((g / T) * G + (i - g * G)) * nb2 : after ? -2 : -1;
+    const bool in = i >= 0 && i < nb1 && g % T == tile,
+               after = i >= -1 && i + 1 < nb1 && h % T == tile;
+    rowmap[i + 2] = in ? ((g / T) * G + (i - g * G)) * nb2 : after ? -2 : -1;
   }
   const FxScale f = fx_scale(w ? max_weight(hdr + 8, npart, red) : 1.0, n);
   if (blockIdx.x == 0 && tile == 0 && threadIdx.x == 0) {
@@ -318,7 +318,7 @@ __global__ __launch_bounds__(kTileThreads) void cic_tile_kernel(
   const auto deposit = [&](double x, double z, double wt) {
     const CicAxis A = cic_axis(x, start1, inv1, nb1), B = cic_axis(z, start2, inv2, nb2);
     if (A.i < -1 || A.i >= nb1) return;
-    const int ra = rowmap[A.i + 1], rb = rowmap[A.i + 2];
+    const int ra = rowmap[A.i + 2], rb = rowmap[A.i + 3];
     const bool b0 = B.i >= 0 && B.i < nb2, b1 = B.i + 1 >= 0 && B.i + 1 < nb2;
     // Corner weights in the reference's association: (w*S1)*S2.
     const double t0 = wt * A.S, t1 = wt * (1.0 - A.S);
@@ -362,18 +362,30 @@ __global__ __launch_bounds__(kTileThreads) void cic_tile_kernel(
     }
   } else {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int *queue = rowmap + nb1 + 2 + wave * kQueueLen;
+    int *queue = rowmap + nb1 + 3 + wave * kQueueLen;
     int count = 0;   // wave-uniform
+    // the last particles taken off the queue: their loads are in flight while
+    // the scan goes on, their sums are made when the next ones are taken
+    double hx = NAN, hz = 0.0, hw = 1.0;
     const auto drain = [&](int take) {
+      deposit(hx, hz, fx_weight(hw));
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      hx = NAN;   // off the grid
       if (lane < take) {
         const int64_t p = p0 + queue[count - take + lane];
-        deposit(q1[p], q2[p], w ? fx_weight(w[p]) : 1.0);
+        hx = q1[p];
+        hz = q2[p];
+        if (w) hw = w[p];
       }
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       count -= take;
     };
-    // kScan groups of 64 particles a time, the next kScan in flight
+    // kScan groups of 64 particles a time, the next kScan in flight.  Every
+    // tile of either grid scans all particles, so the scan's instructions bound
+    // the kernel (3e6 on 256 x 256: 91 us with the hits' loads waited for and
+    // the row tested against both ends, 88.3 with those loads in flight, 86
+    // with two sets of scanned positions in turn, 81 with the clamped row; one
+    // XCD for a chunk's tiles, so that they share its L2, made no difference)
     constexpr int kScan = 4;
     const auto load = [&](int64_t b, double (&x)[kScan]) {
 #pragma unroll
@@ -382,30 +394,35 @@ __global__ __launch_bounds__(kTileThreads) void cic_tile_kernel(
         x[k] = p < p1 ? q1[p] : NAN;   // misses every tile
       }
     };
-    double x[kScan], xn[kScan];
-    int64_t b = p0 + wave * (64 * kScan);
-    load(b, x);
-    while (b < p1) {
-      const int64_t bn = b + kTileThreads * kScan;
-      load(bn, xn);
+    const auto scan = [&](int64_t b, const double (&x)[kScan]) {
+      const int at = (int)(b - p0) + lane;
 #pragma unroll
       for (int k = 0; k < kScan; ++k) {
-        const double c = floor((x[k] - start1) * inv1);
-        bool hit = c >= -1.0 && c < (double)nb1;
-        if (hit) {
-          const int i = (int)c;
-          hit = rowmap[i + 1] != -1;
-        }
+        // off the grid (or NaN): rows -2 and nb1, which no tile holds
+        const double u = fmin(fmax((x[k] - start1) * inv1, -2.0), (double)nb1);
+        const bool hit = rowmap[(int)floor(u) + 2] != -1;
         const unsigned long long m = __ballot(hit);
         if (hit)
-          queue[count + __popcll(m & ((1ull << lane) - 1ull))] = (int)(b + k * 64 + lane - p0);
+          queue[count + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                                  __builtin_amdgcn_mbcnt_lo((unsigned)m, 0))] =
+              at + k * 64;
         count += __popcll(m);
         if (count >= 64) drain(64);
-        x[k] = xn[k];
       }
-      b = bn;
+    };
+    constexpr int kStep = kTileThreads * kScan;
+    double xa[kScan], xb[kScan];
+    int64_t b = p0 + wave * (64 * kScan);
+    load(b, xa);
+    while (b < p1) {
+      load(b + kStep, xb);
+      scan(b, xa);
+      load(b + 2 * kStep, xa);
+      scan(b + kStep, xb);
+      b += 2 * kStep;
     }
     if (count) drain(count);
+    deposit(hx, hz, fx_weight(hw));
   }
   __syncthreads();
   unsigned long long *out = words + ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * 2 * cells;
