@@ -132,13 +132,14 @@ struct MeshPart {
   int i0, j0, ni, nj;
 };
 
-// The middle of an nx x nz mesh, its sides in proportion, of at most `most`
-// points.
+// The middle of an nx x nz mesh (both 2 or more), its sides in proportion, of
+// at most `most` points.  Each side keeps 2 points, one cell, however thin the
+// mesh is.
 MeshPart middle(int nx, int nz, int most) {
   MeshPart m = {0, 0, nx, nz};
   if ((int64_t)nx * nz > most) {
     const double f = std::sqrt((double)most / ((double)nx * nz));
-    m.ni = std::max(1, (int)(nx * f));
+    m.ni = std::clamp((int)(nx * f), 2, std::min(nx, most / 2));
     m.nj = std::min(nz, most / m.ni);
     m.ni = std::min(nx, most / m.nj);
   }
@@ -223,10 +224,11 @@ extern "C" int dfcsr_apply_wakes(double *px, double *pz, const double *x, const 
   if (n <= 0) return DFCSR_OK;
   const MeshAxis ax = make_axis(xr0, xr1, xbins), az = make_axis(zr0, zr1, zbins);
   hipStream_t s = as_stream(stream);
-  const int value = transverse_on ? 16 : 8;
-  const MeshPart part = middle(xbins, zbins, kLdsBytes / value);
-  const int64_t cells = (int64_t)part.ni * part.nj, bytes = cells * value;
-  if (n >= (transverse_on ? kLdsFromTwo : kLdsFromOne)) {
+  // (a mesh one point wide has no cells: no particle is kicked)
+  if (n >= (transverse_on ? kLdsFromTwo : kLdsFromOne) && xbins >= 2 && zbins >= 2) {
+    const int value = transverse_on ? 16 : 8;
+    const MeshPart part = middle(xbins, zbins, kLdsBytes / value);
+    const int64_t bytes = (int64_t)part.ni * part.nj * value;
     int64_t b = (n + kLdsThreads - 1) / kLdsThreads;
     const int64_t most = 256 * (bytes <= kLdsBytes / 2 ? 2 : 1);   // what the CUs' LDS holds
     if (b > most) b = most;

@@ -3,9 +3,12 @@ header declares, rejects bad arguments before touching a device, and its
 host-side Savitzky-Golay operator equals scipy's."""
 import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
+import torch
 from scipy.signal import savgol_coeffs, savgol_filter
 
 from pydfcsr_amd import _lib
@@ -71,6 +74,22 @@ def test_argument_errors_without_device():
     rc = lib.dfcsr_history_zspan(None, 2, 3, 8, 8, 4, 4, 2, 0, None)
     assert rc == -1 and b"cap" in lib.dfcsr_last_error()
     assert lib.dfcsr_history_zspan(1, None, 3, 8, 8, 4, 0, 2, 2, None) == 0
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the pointers are not memory of a device")
+@pytest.mark.parametrize("n", [10, 5000000])
+@pytest.mark.parametrize("nx,nz,two", [(30000, 2, 1), (12000, 1, 1), (25000, 1, 0), (50000, 2, 0),
+                                       (2, 30000, 1), (2147483647, 1, 1), (2147483647, 2, 0)])
+def test_kick_of_a_thin_mesh_plans(nx, nz, two, n):
+    """The kick's plan of a mesh of any shape: without a device the call ends
+    with the launch's error (in a process of its own: a trap would end it)."""
+    code = ("from pydfcsr_amd import _lib; lib = _lib.load(); rc = lib.dfcsr_apply_wakes("
+            f"8, 8, 8, 8, {n}, 8, {8 if two else None}, {nx}, {nz}, 0., 1., 0., 1., 0., 0., 1., "
+            f"1., {two}, None); print(rc, lib.dfcsr_last_error())")
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120,
+                       cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert r.returncode == 0, r.stderr
+    assert r.stdout.startswith("-2 ") and "launch of apply_wakes" in r.stdout
 
 
 @pytest.mark.parametrize("window,order", [(5, 2), (7, 2), (9, 3), (5, 0), (9, 1), (21, 4)])

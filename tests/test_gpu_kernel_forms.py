@@ -198,6 +198,15 @@ def test_kick_forms(K, nx, nz, two):
         assert (got[~ok] == 0).all()
 
 
+# meshes whose middle would be less than one cell wide if its sides were only in
+# proportion, and meshes without a cell
+@pytest.mark.parametrize("nx,nz,two", [(30000, 2, 1), (2, 9000, 1), (3, 50000, 1), (50000, 2, 0),
+                                       (2, 30000, 0), (12000, 1, 1), (25000, 1, 0), (1, 12000, 1)])
+def test_kick_thin_meshes(K, nx, nz, two):
+    """As test_kick_forms: few particles a call and many, and scipy's."""
+    test_kick_forms(K, nx, nz, two)
+
+
 LAT_ELEMENTS = [dict(type="drift", L=0.1, nsep=1), dict(type="dipole", L=0.3, angle=0.05, nsep=1),
                 dict(type="drift", L=0.4, nsep=2), dict(type="dipole", L=0.3, angle=-0.05, nsep=1)]
 
