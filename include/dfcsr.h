@@ -355,7 +355,9 @@ int dfcsr_wake_mesh_noalloc(const DfcsrHistory *hist, const DfcsrLattice *lat,
                             double *zmesh, double *dE_dct, double *x_kick, void *stream);
 
 /* Batched form for serving: k independent simulations (each its own history,
- * lattice and parameters) in one launch, 1 <= k <= DFCSR_WAKE_MAX_TASKS.  All
+ * lattice and parameters) in one launch, 1 <= k <= DFCSR_WAKE_MAX_TASKS, of
+ * fewer than 2^27 mesh points together (DFCSR_ERANGE; also for more than 2^30
+ * workgroups of the near regions by phases, whatever form the tasks take).  All
  * descriptor arrays are HOST arrays of length k; output pointers per
  * simulation.  The task table is copied into the workspace on the stream and
  * the call waits for that copy before it returns (the kernels stay

@@ -477,6 +477,11 @@ constexpr int kLineWgTarget = 4096;
 // 794).
 constexpr int kLineFarTarget = 6144;
 
+// Most near-region columns of a mesh by z lines: a thread of the observer
+// launch steps past the last by up to 15 x 2^24 (mesh points, check_params), and
+// that fits an int.
+constexpr int64_t kMaxLineColumns = (int64_t)1 << 30;
+
 // Doubles per mesh point of a wake by phases: partial sums and observer data.
 __host__ __device__ inline int64_t point_doubles(const PhasePlan &pl) {
   const int sums = pl.obs_major ? 4 * pl.S * pl.q : pl.ch0;
@@ -533,9 +538,11 @@ __host__ __device__ inline PhasePlan make_plan(const DfcsrWakeParams &P, int cst
   // lines / phases, us, mesh x bins by 32, 200 x 200 points: float64 17: 480 /
   // 620, 32: 500 / 749, 48: 671 / 1125 (16 by phases 470); mixed 17: 496 / 382,
   // 32: 494 / 484, 33: 623 / 639, 48: 628 / 733.
+  // A launch's threads count a mesh's columns in 32 bits (kMaxLineColumns).
   pl.line = false;
   pl.obg = pl.nog = pl.ng = 0;
-  if (cstride && pl.obs_major && pl.nreg == 3 && pl.S <= (cstride == kColMixed ? 1 : 2)) {
+  if (cstride && pl.obs_major && pl.nreg == 3 && pl.S <= (cstride == kColMixed ? 1 : 2) &&
+      2 * (int64_t)P.Nz * P.mesh_zbins <= kMaxLineColumns) {
     pl.line = true;
     // region 0: a workgroup's four waves take columns of their own, S rows at a
     // time
@@ -1405,6 +1412,10 @@ void launch_batched(const WakeTask *dt, int k, int forms, dim3 ga, dim3 gb, doub
                        k, lines, part);
 }
 
+// Most mesh points of a batch: kObsThreads or kSumLanes threads each, counted
+// in 32 bits.
+constexpr int64_t kMaxPoints = INT32_MAX / (kObsThreads > kSumLanes ? kObsThreads : kSumLanes);
+
 constexpr int64_t kTableAlign = 256;
 constexpr int kMaxTasks = DFCSR_WAKE_MAX_TASKS;
 
@@ -1536,6 +1547,7 @@ int pack_tasks(int k, const DfcsrHistory *hist, const DfcsrLattice *lat, const D
     return set_error(DFCSR_EINVAL, "wake_tasks_pack: unknown precision %d", precision);
   WakeTask *th = static_cast<WakeTask *>(tasks);
   int64_t na = 0, nb = 0, nobs = 0, part = 0;
+  int64_t phases = 0;   // of the near regions, whatever form the tasks take
   int forms = 0;
   for (int j = 0; j < k; ++j) {
     int rc;
@@ -1561,8 +1573,12 @@ int pack_tasks(int k, const DfcsrHistory *hist, const DfcsrLattice *lat, const D
     na += far_blocks(pl, p[j]);
     nb += near_blocks(pl, p[j]);
     nobs += T.M;
-    if (na > ((int64_t)1 << 30) || nb > ((int64_t)1 << 30))
+    phases += (int64_t)T.M * make_plan(p[j], 0).nB;
+    if (na > ((int64_t)1 << 30) || phases > ((int64_t)1 << 30))
       return set_error(DFCSR_ERANGE, "wake_tasks_pack: too many workgroups");
+    if (nobs > kMaxPoints)
+      return set_error(DFCSR_ERANGE, "wake_tasks_pack: more than %lld mesh points",
+                       (long long)kMaxPoints);
   }
   batch->tasks = k;
   batch->blocks_far = (int32_t)na;

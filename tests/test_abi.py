@@ -231,6 +231,44 @@ def test_wake_tasks_pack_host_logic():
     assert rc != 0 and b"too small" in lib.dfcsr_last_error()
 
 
+def test_wake_batch_limits():
+    """Large batches are refused on the host before any launch: mesh points
+    whose threads (16 each) would pass 32 bits, near regions of more than 2^30
+    workgroups by phases; a mesh of more columns than 2^30 goes by phases."""
+    import ctypes
+    lib = _lib.load()
+
+    def pack(k, xb, zb, Nx, Nz, prec):
+        # shared history with every ring; off the chirp branch
+        h = _lib.History(1, 2, 3, None, None, 8, 0, 5, 16, 16, 0, 0, 0, 1, 1, 1)
+        h.cells, h.cells32, h.dcells32 = 7, 8, 9
+        p = _params(0.3)
+        p.Nx, p.Nz, p.mesh_xbins, p.mesh_zbins = Nx, Nz, xb, zb
+        out = (_lib.c_dp * k)(*[8] * k)
+        nb = int(lib.dfcsr_wake_task_table_bytes(k))
+        tbl, batch = ctypes.create_string_buffer(nb), _lib.WakeBatch()
+        rc = lib.dfcsr_wake_tasks_pack(
+            k, (_lib.History * k)(*[h] * k),
+            (_lib.Lattice * k)(*[_lib.Lattice(3, 100, 1, 0.0, 0.01, 4, 5)] * k),
+            (_lib.WakeParams * k)(*[p] * k), prec, out, out, tbl, nb, ctypes.byref(batch))
+        return rc, lib.dfcsr_last_error(), batch
+
+    for prec in (_lib.DFCSR_PREC_FP64, _lib.DFCSR_PREC_MIXED):
+        # 4096 x 182 x 182 points: 1.1e9 workgroups by phases, and 1.36e8 points
+        rc, msg, _ = pack(4096, 182, 182, 200, 200, prec)
+        assert rc == -3 and b"too many workgroups" in msg
+        # one row: few workgroups, 2^24 points a task
+        rc, msg, _ = pack(7, 4096, 4096, 1, 1, prec)
+        assert rc == 0, msg
+        rc, msg, _ = pack(8, 4096, 4096, 1, 1, prec)
+        assert rc == -3 and b"mesh points" in msg
+        # 1.18e9 columns of 2 x 500000 x 1184: by phases
+        rc, msg, batch = pack(1, 33, 500000, 1, 1073, prec)
+        assert rc == 0 and batch.forms == 2, msg
+        rc, msg, batch = pack(1, 33, 500000, 1, 1184, prec)
+        assert rc == 0 and batch.forms == 1, msg
+
+
 def test_bench_workload_lattices():
     """The three bench workloads: 400-step chicane, 100-step dipole, 1000-step large run."""
     import bench
