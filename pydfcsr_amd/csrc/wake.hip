@@ -1144,11 +1144,11 @@ __device__ inline int find_task(const WakeTask *__restrict__ tasks, int ntask, i
 
 template <bool kMixed, bool kNear>
 __global__ __launch_bounds__(kThreads, kMixed && kNear ? 4 : DFCSR_WAKE_MINBLOCKS) void wake_phase_batched_kernel(
-    const WakeTask *__restrict__ tasks, int ntask, double *__restrict__ partials) {
+    const WakeTask *__restrict__ tasks, int ntask, int first, double *__restrict__ partials) {
   __shared__ double red[kThreads / 64];
   // (region 0 of tasks of 45, 32 and 19 by 32 mesh points, mixed: 1027 us the
   // whole wake with a contiguous range an XCD, 870 in groups)
-  const int b = xcd_group<true>(blockIdx.x, gridDim.x, kNearGroup);
+  const int b = first + xcd_group<true>(blockIdx.x, gridDim.x, kNearGroup);
   const int j = find_task(tasks, ntask, b,
                           [](const WakeTask &T) { return kNear ? T.blockB0 : T.blockA0; });
   const WakeTask &T = tasks[j];
@@ -1212,13 +1212,13 @@ __global__ __launch_bounds__(kThreads) void wake_observer_kernel(WakeTask T,
   if (i < kObsThreads * T.M) observer_data(T, i, partials);
 }
 
-// The line form's workgroups of a batched launch (kNear or region 0): S as
-// the task's plan; workgroups of other tasks return.
+// The line form's workgroups of a batched launch (kNear or region 0), from
+// workgroup `first` on: S as the task's plan; workgroups of other tasks return.
 template <bool kMixed, bool kNear, int S>
 __global__ __launch_bounds__((kNear ? LineSize<S>::kThreads : kThreads), 4) void
-wake_line_batched_kernel(const WakeTask *__restrict__ tasks, int ntask,
+wake_line_batched_kernel(const WakeTask *__restrict__ tasks, int ntask, int first,
                          const double *__restrict__ lines, double *__restrict__ partials) {
-  const int b = blockIdx.x;
+  const int b = first + blockIdx.x;
   const int j = find_task(tasks, ntask, b,
                           [](const WakeTask &T) { return kNear ? T.blockB0 : T.blockA0; });
   const WakeTask &T = tasks[j];
@@ -1386,35 +1386,35 @@ int make_task(const DfcsrHistory &H, const DfcsrLattice &L, const DfcsrWakeParam
 // The forms a batch's tasks take (DfcsrWakeBatch.forms): one launch each.
 enum { kFormPhases = 1, kFormLine1 = 2, kFormLine2 = 4 };
 
-template <bool kMixed>
-void launch_batched(const WakeTask *dt, int k, int forms, dim3 ga, dim3 gb, double *part,
-                    hipStream_t s) {
-  const double *lines = part;
-  if (forms & kFormPhases)
-    hipLaunchKernelGGL((wake_phase_batched_kernel<kMixed, false>), ga, dim3(kThreads), 0, s, dt, k,
-                       part);
-  if (forms & kFormLine1)
-    hipLaunchKernelGGL((wake_line_batched_kernel<kMixed, false, 1>), ga, dim3(kThreads), 0, s, dt,
-                       k, lines, part);
-  if (!kMixed && (forms & kFormLine2))
-    hipLaunchKernelGGL((wake_line_batched_kernel<false, false, 2>), ga, dim3(kThreads), 0, s, dt,
-                       k, lines, part);
-  if (forms & kFormPhases)
-    hipLaunchKernelGGL((wake_phase_batched_kernel<kMixed, true>), gb, dim3(kThreads), 0, s, dt, k,
-                       part);
-  if (forms & kFormLine1)
-    hipLaunchKernelGGL((wake_line_batched_kernel<kMixed, true, 1>), gb,
-                       dim3(LineSize<1>::kThreads), 0, s, dt,
-                       k, lines, part);
-  if (!kMixed && (forms & kFormLine2))
-    hipLaunchKernelGGL((wake_line_batched_kernel<false, true, 2>), gb,
-                       dim3(LineSize<2>::kThreads), 0, s, dt,
-                       k, lines, part);
-}
+// Most workgroups of one launch, of 512 threads or fewer: a launch of 2^32
+// threads or more runs the remainder alone, with no error.  A large batch takes
+// several (region 0 of 4096 tasks of a 17 x 17 mesh with 1500 columns: 25
+// million workgroups).
+constexpr int kMaxGrid = 1 << 22;
 
 // Most mesh points of a batch: kObsThreads or kSumLanes threads each, counted
 // in 32 bits.
 constexpr int64_t kMaxPoints = INT32_MAX / (kObsThreads > kSumLanes ? kObsThreads : kSumLanes);
+
+template <bool kMixed, bool kNear>
+void launch_regions(const WakeTask *dt, int k, int forms, int blocks, double *part,
+                    hipStream_t s) {
+  const double *lines = part;
+  const int n1 = kNear ? LineSize<1>::kThreads : kThreads;
+  const int n2 = kNear ? LineSize<2>::kThreads : kThreads;
+  for (int at = 0; at < blocks; at += kMaxGrid) {
+    const dim3 g(blocks - at < kMaxGrid ? blocks - at : kMaxGrid);
+    if (forms & kFormPhases)
+      hipLaunchKernelGGL((wake_phase_batched_kernel<kMixed, kNear>), g, dim3(kThreads), 0, s, dt,
+                         k, at, part);
+    if (forms & kFormLine1)
+      hipLaunchKernelGGL((wake_line_batched_kernel<kMixed, kNear, 1>), g, dim3(n1), 0, s, dt, k,
+                         at, lines, part);
+    if (!kMixed && (forms & kFormLine2))
+      hipLaunchKernelGGL((wake_line_batched_kernel<false, kNear, 2>), g, dim3(n2), 0, s, dt, k,
+                         at, lines, part);
+  }
+}
 
 constexpr int64_t kTableAlign = 256;
 constexpr int kMaxTasks = DFCSR_WAKE_MAX_TASKS;
@@ -1618,17 +1618,19 @@ extern "C" int dfcsr_wake_batched_launch(const void *dev_tasks, const DfcsrWakeB
   // form's workgroups return from other forms' tasks
   const int any = kFormPhases | kFormLine1 | kFormLine2;
   const int forms = batch->forms > 0 && batch->forms <= any ? batch->forms : any;
-  const dim3 ga(batch->blocks_far), gb(batch->blocks_near);
   const dim3 go(point_grid(batch->observers, kObsThreads));
   const dim3 gf(point_grid(batch->observers, kSumLanes));
   hipLaunchKernelGGL(wake_observer_batched_kernel, go, dim3(kThreads), 0, s, dt, k,
                      batch->observers, part);
   if (precision != DFCSR_PREC_FP64 && precision != DFCSR_PREC_MIXED)
     return set_error(DFCSR_EINVAL, "wake_batched_launch: unknown precision %d", precision);
-  if (precision == DFCSR_PREC_MIXED)
-    launch_batched<true>(dt, k, forms, ga, gb, part, s);
-  else
-    launch_batched<false>(dt, k, forms, ga, gb, part, s);
+  if (precision == DFCSR_PREC_MIXED) {
+    launch_regions<true, false>(dt, k, forms, batch->blocks_far, part, s);
+    launch_regions<true, true>(dt, k, forms, batch->blocks_near, part, s);
+  } else {
+    launch_regions<false, false>(dt, k, forms, batch->blocks_far, part, s);
+    launch_regions<false, true>(dt, k, forms, batch->blocks_near, part, s);
+  }
   hipLaunchKernelGGL(wake_finalize_batched_kernel, gf, dim3(kThreads), 0, s, dt, k,
                      batch->observers, (const double *)part);
   DFCSR_LAUNCH_CHECK("wake_batched_launch");

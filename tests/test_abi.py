@@ -234,7 +234,8 @@ def test_wake_tasks_pack_host_logic():
 def test_wake_batch_limits():
     """Large batches are refused on the host before any launch: mesh points
     whose threads (16 each) would pass 32 bits, near regions of more than 2^30
-    workgroups by phases; a mesh of more columns than 2^30 goes by phases."""
+    workgroups by phases; a mesh of more columns than 2^30 goes by phases.  A
+    batch whose region 0 takes more workgroups than one launch holds packs."""
     import ctypes
     lib = _lib.load()
 
@@ -262,6 +263,10 @@ def test_wake_batch_limits():
         assert rc == 0, msg
         rc, msg, _ = pack(8, 4096, 4096, 1, 1, prec)
         assert rc == -3 and b"mesh points" in msg
+        # 4096 workgroups and more of region 0 a task
+        rc, msg, batch = pack(4096, 33, 33, 2, 1500, prec)
+        assert rc == 0 and batch.blocks_far * 256 >= 1 << 32, msg
+        assert batch.forms & 2
         # 1.18e9 columns of 2 x 500000 x 1184: by phases
         rc, msg, batch = pack(1, 33, 500000, 1, 1073, prec)
         assert rc == 0 and batch.forms == 2, msg

@@ -360,3 +360,29 @@ def test_wake_batch_forms_unset(K, ws, forms):
         for w, v in zip(one, o):
             for n in v:
                 assert np.array_equal(w[n].cpu().numpy(), v[n].cpu().numpy(), equal_nan=True), (p, n)
+
+
+def test_wake_batch_of_many_launches(K, ws):
+    """A batch whose region 0 takes more workgroups than a launch holds (4096
+    tasks of 17 x 17 points, 1500 columns by z lines, a chirp-branch task among
+    them): each task equals its single launch bit for bit."""
+    from pydfcsr_amd import _lib
+    from tests.gpu_util import DeviceHistory, DeviceLattice, wake_params
+    sx, sz, t, k = 50e-6, 50e-6, 0.33, 4096
+    T, lat = _History(t, sx, sz), O.LatticeTables(LAT_ELEMENTS)
+    H = DeviceHistory(T, DEV, wrap=2, rings=("fp64", "cells", "zspan"))
+    L = DeviceLattice(lat, DEV)
+    P = [wake_params(t, dict(sigma_x=sx, sigma_z=sz, slope=np.array([s, 1e-6]), mean_x=0.0), 0.05,
+                     4.0, 3, 1500, 9.0, (-sx, sx, 17), (-sz, sz, 17)) for s in (0.3, -0.4, -1.7)]
+    one = [K.wake_mesh(H.desc, L.desc, p, 0, DEV, ws) for p in P]
+    which = [2 if j == 2000 else j % 2 for j in range(k)]
+    out = {n: torch.full((k, 17 * 17), 7.0, dtype=torch.float64, device=DEV)
+           for n in ("dE_dct", "x_kick")}
+    o = [{n: v[j] for n, v in out.items()} for j in range(k)]
+    # (its 27 GB go with this workspace)
+    K.wake_mesh_batched([H.desc] * k, [L.desc] * k, [P[w] for w in which], 0, o, DEV,
+                        _lib.Workspace(DEV))
+    for n in out:
+        ref = torch.stack([w[n].flatten() for w in one])[torch.tensor(which, device=DEV)]
+        assert torch.isfinite(ref).any()
+        assert torch.equal(out[n].nan_to_num(nan=1e300), ref.nan_to_num(nan=1e300)), n
