@@ -1091,12 +1091,13 @@ __host__ __device__ inline bool cells32_ring32(const DfcsrHistory &H) {
 }
 
 // Workgroups per CU the register allocation must allow: the near phases on
-// the cell-major ring 4 (128 registers), the others 2.
+// the cell-major ring 4 (128 registers), the others 2.  The launch's
+// workgroups are those from `first` on of the nb (launch_blocks).
 template <bool kMixed, bool kNear, bool kTI, int kCells = kRings>
 __global__ __launch_bounds__(kThreads, kCells ? 4 : DFCSR_WAKE_MINBLOCKS) void wake_phase_kernel(
-    WakeTask T, double *__restrict__ partials) {
+    WakeTask T, int first, int nb, double *__restrict__ partials) {
   __shared__ double red[kThreads / 64];
-  const int b = blockIdx.x, nb = gridDim.x;
+  const int b = first + (int)blockIdx.x;
   run_phase_block<kMixed, kNear, kTI, kCells>(
       T, kNear ? xcd_group<true>(b, nb, kNearGroup) : xcd_remap(b, nb), partials, red);
 }
@@ -1111,9 +1112,9 @@ __global__ __launch_bounds__(kThreads, kCells ? 4 : DFCSR_WAKE_MINBLOCKS) void w
 // the whole wake).
 template <bool kMixed, bool kTI, bool kSkip = false>
 __global__ __launch_bounds__(kThreads, !kMixed && kSkip ? 4 : 3) void wake_far_kernel(
-    WakeTask T, double *__restrict__ partials) {
+    WakeTask T, int first, int nb, double *__restrict__ partials) {
   __shared__ RowTable rt;
-  const int b = blockIdx.x, nb = gridDim.x;
+  const int b = first + (int)blockIdx.x;
   far_obs_block<kMixed, kTI, kSkip>(
       T, kSkip ? xcd_group<false>(b, nb, nb / T.P.mesh_zbins) : xcd_remap(b, nb), partials, rt);
 }
@@ -1291,6 +1292,20 @@ __global__ __launch_bounds__(kThreads) void wake_finalize_batched_kernel(
   finalize_point(tasks[j], i - tasks[j].obs0, g % kSumLanes, partials);
 }
 
+// Most workgroups of one launch, of 512 threads or fewer: a launch of 2^32
+// threads or more runs the remainder alone, with no error.  A large mesh by
+// phases takes several (1200 x 1200 points, four regions of 200 rows: 17
+// million workgroups), and a large batch (region 0 of 4096 tasks of a 17 x 17
+// mesh with 1500 columns: 25 million).
+constexpr int kMaxGrid = 1 << 22;
+
+// launch(first, grid) for each launch of `blocks` workgroups.
+template <typename F>
+void launch_blocks(int64_t blocks, const F &launch) {
+  for (int64_t at = 0; at < blocks; at += kMaxGrid)
+    launch((int)at, dim3((unsigned)(blocks - at < kMaxGrid ? blocks - at : kMaxGrid)));
+}
+
 // Workgroups of a launch of `per` threads per mesh point.
 unsigned point_grid(int M, int per) {
   return (unsigned)(((int64_t)M * per + kThreads - 1) / kThreads);
@@ -1386,12 +1401,6 @@ int make_task(const DfcsrHistory &H, const DfcsrLattice &L, const DfcsrWakeParam
 // The forms a batch's tasks take (DfcsrWakeBatch.forms): one launch each.
 enum { kFormPhases = 1, kFormLine1 = 2, kFormLine2 = 4 };
 
-// Most workgroups of one launch, of 512 threads or fewer: a launch of 2^32
-// threads or more runs the remainder alone, with no error.  A large batch takes
-// several (region 0 of 4096 tasks of a 17 x 17 mesh with 1500 columns: 25
-// million workgroups).
-constexpr int kMaxGrid = 1 << 22;
-
 // Most mesh points of a batch: kObsThreads or kSumLanes threads each, counted
 // in 32 bits.
 constexpr int64_t kMaxPoints = INT32_MAX / (kObsThreads > kSumLanes ? kObsThreads : kSumLanes);
@@ -1402,18 +1411,17 @@ void launch_regions(const WakeTask *dt, int k, int forms, int blocks, double *pa
   const double *lines = part;
   const int n1 = kNear ? LineSize<1>::kThreads : kThreads;
   const int n2 = kNear ? LineSize<2>::kThreads : kThreads;
-  for (int at = 0; at < blocks; at += kMaxGrid) {
-    const dim3 g(blocks - at < kMaxGrid ? blocks - at : kMaxGrid);
+  launch_blocks(blocks, [&](int first, dim3 g) {
     if (forms & kFormPhases)
       hipLaunchKernelGGL((wake_phase_batched_kernel<kMixed, kNear>), g, dim3(kThreads), 0, s, dt,
-                         k, at, part);
+                         k, first, part);
     if (forms & kFormLine1)
       hipLaunchKernelGGL((wake_line_batched_kernel<kMixed, kNear, 1>), g, dim3(n1), 0, s, dt, k,
-                         at, lines, part);
+                         first, lines, part);
     if (!kMixed && (forms & kFormLine2))
       hipLaunchKernelGGL((wake_line_batched_kernel<false, kNear, 2>), g, dim3(n2), 0, s, dt, k,
-                         at, lines, part);
-  }
+                         first, lines, part);
+  });
 }
 
 constexpr int64_t kTableAlign = 256;
@@ -1457,57 +1465,45 @@ extern "C" int dfcsr_wake_mesh(const DfcsrHistory *hist, const DfcsrLattice *lat
   double *part = static_cast<double *>(ws);
   hipStream_t s = as_stream(stream);
   const PhasePlan pl = make_plan(*p, T.cstride);
-  const dim3 ga((unsigned)far_blocks(pl, *p)), gb((unsigned)near_blocks(pl, *p));
+  const int64_t na = far_blocks(pl, *p), nb = near_blocks(pl, *p);
   const dim3 go(point_grid(T.M, pl.line ? kObsThreads : 1)), gf(point_grid(T.M, kSumLanes));
   hipLaunchKernelGGL(wake_observer_kernel, go, dim3(kThreads), 0, s, T, part);
-  if (pl.line) {
+  if (pl.line) {   // (one launch: a z line is 17 mesh points or more, so fewer than 2^21 workgroups)
     const bool mixed = precision == DFCSR_PREC_MIXED;
     auto far = mixed ? wake_far_line_kernel<true, 1>
                : (pl.S == 1 ? wake_far_line_kernel<false, 1> : wake_far_line_kernel<false, 2>);
     auto near = mixed ? wake_line_kernel<true, 1>
                 : (pl.S == 1 ? wake_line_kernel<false, 1> : wake_line_kernel<false, 2>);
-    hipLaunchKernelGGL(far, ga, dim3(kThreads), 0, s, T, part);
-    hipLaunchKernelGGL(near, gb, dim3(pl.S == 1 ? LineSize<1>::kThreads : LineSize<2>::kThreads),
-                       0, s, T, (const double *)part, part);
-  } else if (precision == DFCSR_PREC_MIXED) {
-    const bool ti_far = mixed_reads_ti(*hist, false);
-    const bool skip = far_skip(*hist, pl);
-    if (pl.obs_major && ti_far && skip)
-      hipLaunchKernelGGL((wake_far_kernel<true, true, true>), ga, dim3(kThreads), 0, s, T, part);
-    else if (pl.obs_major && ti_far)
-      hipLaunchKernelGGL((wake_far_kernel<true, true>), ga, dim3(kThreads), 0, s, T, part);
-    else if (pl.obs_major && skip)
-      hipLaunchKernelGGL((wake_far_kernel<true, false, true>), ga, dim3(kThreads), 0, s, T, part);
-    else if (pl.obs_major)
-      hipLaunchKernelGGL((wake_far_kernel<true, false>), ga, dim3(kThreads), 0, s, T, part);
-    else if (ti_far)
-      hipLaunchKernelGGL((wake_phase_kernel<true, false, true>), ga, dim3(kThreads), 0, s, T, part);
-    else
-      hipLaunchKernelGGL((wake_phase_kernel<true, false, false>), ga, dim3(kThreads), 0, s, T, part);
-    const bool ti = mixed_reads_ti(*hist, true);
-    if (mixed_cells(*hist) && cells32_ring32(*hist)) {
-      hipLaunchKernelGGL((wake_phase_kernel<true, true, false, kCellsRing32>), gb, dim3(kThreads),
-                         0, s, T, part);
-    } else if (mixed_cells(*hist)) {
-      hipLaunchKernelGGL((wake_phase_kernel<true, true, false, kCellsPlane>), gb, dim3(kThreads),
-                         0, s, T, part);
-    } else if (ti) {
-      hipLaunchKernelGGL((wake_phase_kernel<true, true, true>), gb, dim3(kThreads), 0, s, T, part);
-    } else {
-      hipLaunchKernelGGL((wake_phase_kernel<true, true, false>), gb, dim3(kThreads), 0, s, T, part);
-    }
+    hipLaunchKernelGGL(far, dim3((unsigned)na), dim3(kThreads), 0, s, T, part);
+    hipLaunchKernelGGL(near, dim3((unsigned)nb),
+                       dim3(pl.S == 1 ? LineSize<1>::kThreads : LineSize<2>::kThreads), 0, s, T,
+                       (const double *)part, part);
   } else {
-    if (pl.obs_major && far_skip(*hist, pl))
-      hipLaunchKernelGGL((wake_far_kernel<false, false, true>), ga, dim3(kThreads), 0, s, T, part);
-    else if (pl.obs_major)
-      hipLaunchKernelGGL((wake_far_kernel<false, false>), ga, dim3(kThreads), 0, s, T, part);
-    else
-      hipLaunchKernelGGL((wake_phase_kernel<false, false, false>), ga, dim3(kThreads), 0, s, T, part);
-    if (hist->cells) {
-      hipLaunchKernelGGL((wake_phase_kernel<false, true, false, kCellsPlane>), gb, dim3(kThreads),
-                         0, s, T, part);
+    const auto launch = [&](auto kernel, int64_t blocks) {
+      launch_blocks(blocks, [&](int first, dim3 g) {
+        hipLaunchKernelGGL(kernel, g, dim3(kThreads), 0, s, T, first, (int)blocks, part);
+      });
+    };
+    const bool skip = far_skip(*hist, pl);
+    if (precision == DFCSR_PREC_MIXED) {
+      const bool ti_far = mixed_reads_ti(*hist, false);
+      if (pl.obs_major && ti_far && skip) launch(wake_far_kernel<true, true, true>, na);
+      else if (pl.obs_major && ti_far) launch(wake_far_kernel<true, true>, na);
+      else if (pl.obs_major && skip) launch(wake_far_kernel<true, false, true>, na);
+      else if (pl.obs_major) launch(wake_far_kernel<true, false>, na);
+      else if (ti_far) launch(wake_phase_kernel<true, false, true>, na);
+      else launch(wake_phase_kernel<true, false, false>, na);
+      if (mixed_cells(*hist) && cells32_ring32(*hist))
+        launch(wake_phase_kernel<true, true, false, kCellsRing32>, nb);
+      else if (mixed_cells(*hist)) launch(wake_phase_kernel<true, true, false, kCellsPlane>, nb);
+      else if (mixed_reads_ti(*hist, true)) launch(wake_phase_kernel<true, true, true>, nb);
+      else launch(wake_phase_kernel<true, true, false>, nb);
     } else {
-      hipLaunchKernelGGL((wake_phase_kernel<false, true, false>), gb, dim3(kThreads), 0, s, T, part);
+      if (pl.obs_major && skip) launch(wake_far_kernel<false, false, true>, na);
+      else if (pl.obs_major) launch(wake_far_kernel<false, false>, na);
+      else launch(wake_phase_kernel<false, false, false>, na);
+      if (hist->cells) launch(wake_phase_kernel<false, true, false, kCellsPlane>, nb);
+      else launch(wake_phase_kernel<false, true, false>, nb);
     }
   }
   hipLaunchKernelGGL(wake_finalize_kernel, gf, dim3(kThreads), 0, s, T, (const double *)part);

@@ -386,3 +386,33 @@ def test_wake_batch_of_many_launches(K, ws):
         ref = torch.stack([w[n].flatten() for w in one])[torch.tensor(which, device=DEV)]
         assert torch.isfinite(ref).any()
         assert torch.equal(out[n].nan_to_num(nan=1e300), ref.nan_to_num(nan=1e300)), n
+
+
+@pytest.mark.parametrize("precision,tol", [(0, 1e-10), (1, 1e-8)])
+def test_wake_of_many_launches(K, ws, precision, tol):
+    """A mesh whose near regions by phases take more workgroups than a launch
+    holds (1200 x 1200 points, the chirp branch, 12 phases) against the same
+    points as explicit observers in small calls, float64 within 1e-10 of max|W|
+    and mixed within 1e-8 (the same float32 operations, float64 sums in another
+    order)."""
+    from pydfcsr_amd import _lib
+    from tests.gpu_util import DeviceHistory, DeviceLattice, wake_params
+    sx, sz, t, m, own = 50e-6, 50e-6, 0.33, 1200, _lib.Workspace(DEV)
+    T, lat = _History(t, sx, sz), O.LatticeTables(LAT_ELEMENTS)
+    beam = dict(sigma_x=sx, sigma_z=sz, slope=np.array([-1.7, 1e-6]), mean_x=0.0)
+    H = DeviceHistory(T, DEV, wrap=2, rings=("fp64", "fp32t", "cells", "cells32", "zspan"))
+    L, args = DeviceLattice(lat, DEV), (t, beam, 0.05, 4.0, 200, 3, 9.0)
+    P = wake_params(*args, (-sx, sx, m), (-sz, sz, m))
+    got = {k: v.flatten() for k, v in K.wake_mesh(H.desc, L.desc, P, precision, DEV, own).items()}
+    obs = torch.stack([got["zmesh"], got["xmesh"]], dim=1)
+    ref = {k: torch.empty_like(got[k]) for k in ("dE_dct", "x_kick")}
+    for a in range(0, m * m, m * m // 16):
+        o = obs[a:a + m * m // 16].contiguous()
+        Po = wake_params(*args, (0.0, 0.0, 1), (0.0, 0.0, len(o)), observers=o)
+        for k, v in K.wake_mesh(H.desc, L.desc, Po, precision, DEV, ws).items():
+            if k in ref:
+                ref[k][a:a + len(o)] = v.flatten()
+    for k, r in ref.items():
+        ok = torch.isfinite(r)
+        assert torch.equal(ok, torch.isfinite(got[k])) and ok.any()
+        assert (got[k] - r)[ok].abs().max() <= tol * r[ok].abs().max(), k
