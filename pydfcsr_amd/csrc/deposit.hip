@@ -57,8 +57,9 @@ __global__ __launch_bounds__(kThreads) void absmax_partial(const double *__restr
 
 // Fixed-point format of one grid.  A weight v is s = v 2^k = hi + r with
 // hi = rint(s), |r| <= 1/2, and lo = rint(r 2^d).  n max|w| 2^k < 2^62 keeps
-// the sum of n high words in 63 bits, n 2^(d-1) < 2^61 that of the low ones;
-// |s| < 2^50 and d <= 50 let the conversions add 1.5 2^52 and read the
+// the sum of n high words in 63 bits, n 2^(d-1) < 2^63 that of the low ones in
+// 64 (one bit less of d would be a coarser quantum from 2^30 particles on than
+// one word of 94 bits has); |s| < 2^50 and d <= 50 let the conversions add 1.5 2^52 and read the
 // integer from the mantissa (4 operations a word, against about 15 for a
 // float64 -> int64 conversion).
 struct FxScale {
@@ -73,7 +74,7 @@ __device__ inline FxScale fx_scale(double max_w, int64_t n) {
   if (max_w > 0.0) frexp(max_w, &e);     // max|w| < 2^e
   f.k = min(62 - e - en, 50 - e);
   f.k = max_w > 0.0 ? min(f.k, 900) : 0;
-  f.d = min(62 - en, 50);
+  f.d = min(64 - en, 50);
   f.up = ldexp(1.0, f.k);
   f.up_lo = ldexp(1.0, f.d);
   return f;
@@ -96,11 +97,28 @@ __device__ inline FxWords fx_words(double v, const FxScale &f) {
   return w;
 }
 
-// (hi + lo 2^-d) 2^-k with one rounding: hi's halves are exact float64s.
+// (hi + lo 2^-d) 2^-k.  The low word's whole units are carried into the high
+// one, so what is left of it is half a unit or less and nothing cancels: below
+// 2^53 units hi is exact and the sum is rounded once, past that it is within
+// 1.5 times that rounding.
 __device__ inline double fx_value(long long hi, long long lo, const FxScale &f) {
-  const double hh = (double)(hi >> 32) * 0x1p32, hl = (double)(hi & 0xffffffffll);
-  const double l = (double)lo * (1.0 / f.up_lo);
-  return (hh + (hl + l)) * (1.0 / f.up);
+  long long carry = lo >> f.d;
+  long long rest = lo - (carry << f.d);   // in [0, 2^d)
+  if (rest >> (f.d - 1)) {
+    ++carry;
+    rest -= 1ll << f.d;
+  }
+  return ((double)(hi + carry) + (double)rest * (1.0 / f.up_lo)) * (1.0 / f.up);
+}
+
+// The format that a deposition kernel left in hdr (k and d as doubles).
+__device__ inline FxScale fx_stored(const double *hdr) {
+  FxScale f;
+  f.k = (int)hdr[0];
+  f.d = (int)hdr[1];
+  f.up = ldexp(1.0, f.k);
+  f.up_lo = ldexp(1.0, f.d);
+  return f;
 }
 
 // Block reduction of the max|w| partials (0 without a weight).
@@ -207,9 +225,7 @@ __global__ __launch_bounds__(kThreads) void fx_to_double(const int64_t *__restri
                                                          double *__restrict__ outB) {
   double *out = blockIdx.y ? outB : outA;
   const int64_t *hi = acc + blockIdx.y * 2 * n, *lo = hi + n;
-  FxScale f;
-  f.up = ldexp(1.0, (int)hdr[2 * blockIdx.y]);
-  f.up_lo = ldexp(1.0, (int)hdr[2 * blockIdx.y + 1]);
+  const FxScale f = fx_stored(hdr + 2 * blockIdx.y);
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
     out[i] = fx_value(hi[i], lo[i], f);
@@ -461,9 +477,7 @@ __global__ __launch_bounds__(kThreads) void tile_sum_kernel(
   const int lr = cell / nb2, col = cell - lr * nb2;
   const int row = ((lr / G) * T + tile) * G + lr % G;
   if (row >= nb1) return;
-  FxScale f;
-  f.up = ldexp(1.0, (int)hdr[2 * grid]);
-  f.up_lo = ldexp(1.0, (int)hdr[2 * grid + 1]);
+  const FxScale f = fx_stored(hdr + 2 * grid);
   (grid ? outB : outA)[(int64_t)row * nb2 + col] = fx_value((long long)h, (long long)l, f);
 }
 

@@ -65,6 +65,60 @@ def test_deposit_forms(K, ws, bins, n):
         assert rel_max(v3.cpu(), O.histogram_cic_2d(x[ok], z[ok], bad[ok], *a)) <= 1e-13
 
 
+# whole grid in one tile, row tiles, and the direct form; few particles and
+# counts either side of a power of two
+@pytest.mark.parametrize("bins", [(16, 16), (256, 256), (1500, 1300)])
+@pytest.mark.parametrize("n", [200, 4096, 65535, 1 << 20])
+def test_deposit_relative(K, ws, bins, n):
+    """Each cell's own relative error, for weights of both signs over 2^-42 to 1
+    of the largest: every term (w S1) S2 is exact here (30 bits of weight, lower
+    corners at multiples of 1/8), so math.fsum of a cell's terms is its sum
+    rounded once.  The deposition may be off by two roundings, 2^-52 of the
+    value, and by half a quantum a term; the quantum is 2^-k with n max|w| 2^k <
+    2^94 or finer."""
+    import math
+    rng = np.random.default_rng(n + bins[0])
+    w = np.ldexp(rng.integers(1 << 29, 1 << 30, n) / 2.0 ** 30, rng.integers(-42, 1, n))
+    w *= rng.choice([-1.0, 1.0], n)
+    w[0] = 1.0
+    i, j = rng.integers(0, bins[0], n), rng.integers(0, bins[1], n)
+    i[n // 2:] %= 12   # half of them on few cells, half spread over the grid
+    j[n // 2:] %= 12
+    a, b = rng.integers(0, 8, n) / 8, rng.integers(0, 8, n) / 8
+    got = K.histogram_cic_2d(_t(i + a), _t(j + b), _t(w), bins[0], 0.0, float(bins[0]), bins[1],
+                             0.0, float(bins[1]), ws).cpu().numpy()
+    terms = {}
+    for di in (0, 1):
+        for dj in (0, 1):
+            t = w * ((1 - a) if di == 0 else a) * ((1 - b) if dj == 0 else b)
+            for c, r, v in zip(i + di, j + dj, t):
+                if c < bins[0] and r < bins[1]:
+                    terms.setdefault((c, r), []).append(v)
+    quantum = 2.0 ** -(94 - math.frexp(float(n))[1])
+    assert np.count_nonzero(got) <= len(terms)
+    for (c, r), v in terms.items():
+        ref = math.fsum(v)
+        assert abs(got[c, r] - ref) <= 2.0 ** -52 * abs(ref) + len(v) * quantum / 2, (c, r, ref)
+
+
+@pytest.mark.parametrize("n", [3, 10 ** 6, (1 << 29) + 1, (1 << 30) + 1])
+def test_deposit_quantum(K, ws, n):
+    """Weights far below the largest, each alone in a cell (the other particles
+    lie off the grid): the value to half a quantum of n max|w| 2^k < 2^94, and
+    two roundings, at the largest particle counts too."""
+    import math
+    x = torch.full((n,), -9.0, dtype=torch.float64, device=DEV)
+    w = torch.ones(n, dtype=torch.float64, device=DEV)
+    small = -(1 + 2.0 ** -20) * 2.0 ** -44
+    x[0], x[1], x[2] = 1.0, 3.0, 5.0
+    w[1], w[2] = small, -small / 64
+    h = K.histogram_cic_2d(x, x, w, 8, 0.0, 8.0, 8, 0.0, 8.0, ws).cpu()
+    quantum = 2.0 ** -(94 - math.frexp(float(n))[1])
+    for at, ref in ((1, 1.0), (3, small), (5, -small / 64)):
+        assert abs(float(h[at, at]) - ref) <= 2.0 ** -52 * abs(ref) + quantum / 2, (at, float(h[at, at]))
+    assert np.count_nonzero(h) == 3
+
+
 # one workgroup's pair tile (2048) less and more one, its last workgroup
 # holding one particle, and past one tile and two a workgroup of the full grid
 @pytest.mark.parametrize("n", [2, 3, 5, 2047, 2048, 2049, 4097, 524287, 524289, 1048577, 1572865])
