@@ -476,6 +476,16 @@ constexpr int kLineWgTarget = 4096;
 // 811 / 761 / 748 / 766 (as many as the observer-major form's: 2656, 491, 284,
 // 794).
 constexpr int kLineFarTarget = 6144;
+// Fewest workgroups of a line-form near launch, the share of lanes without an
+// observer taken off: below, a mesh of few z lines or an integration of few rows
+// goes by phases, which have a workgroup a mesh point and leave less of the chip
+// idle.  Measured on 4000 wakes of 17 to 300 x 1 to 128 points, 8 to 500 rows
+// and columns, how many are slower than by phases (over 3 %), and the worst:
+// float64 408 of 2002 and 7.6 times by lines alone, 17 and 1.37 times from 192 on (33 and 1.76 from
+// 160, 7 and 1.29 from 256, which gives more of the gain away); mixed 588 of 1998 and 6.7 times, 30
+// and 1.34 from 384 (77 and 1.59 from 256, 15 and 1.20 from 512).  20 z lines
+// of 20 x bins with 40 rows have 250 (float64), of 33 x bins 412.
+constexpr int kLineLeast = 192, kLineLeastMixed = 384;
 
 // Most near-region columns of a mesh by z lines: a thread of the observer
 // launch steps past the last by up to 15 x 2^24 (mesh points, check_params), and
@@ -543,19 +553,23 @@ __host__ __device__ inline PhasePlan make_plan(const DfcsrWakeParams &P, int cst
   pl.obg = pl.nog = pl.ng = 0;
   if (cstride && pl.obs_major && pl.nreg == 3 && pl.S <= (cstride == kColMixed ? 1 : 2) &&
       2 * (int64_t)P.Nz * P.mesh_zbins <= kMaxLineColumns) {
+    const int obg = pl.nob == 1 ? 1 : (pl.nob == 2 ? 2 : 4), nog = (pl.nob + obg - 1) / obg;
+    const int64_t lines = (int64_t)P.mesh_zbins * nog * 2;
+    const int64_t target = pl.S == 1 ? kLineWgTarget : kLineWgTarget / 2;
+    const int64_t most = (P.Nx + 2 * pl.S - 1) / (2 * pl.S);   // two passes of rows or more
+    int64_t ng = (target + lines - 1) / lines;
+    ng = ng > most ? most : ng;
+    // few lines or rows leave most of the chip idle
+    const int64_t least = cstride == kColMixed ? kLineLeastMixed : kLineLeast;
+    if (lines * ng * P.mesh_xbins < least * nog * obg * pl.W) return pl;
     pl.line = true;
     // region 0: a workgroup's four waves take columns of their own, S rows at a
     // time
     const int fl = P.mesh_zbins * pl.nob, fmost = (P.Nz + 3) / 4;
     const int fq = (kLineFarTarget + fl - 1) / fl;
     pl.nA = fq > fmost ? fmost : fq;
-    pl.obg = pl.nob == 1 ? 1 : (pl.nob == 2 ? 2 : 4);
-    pl.nog = (pl.nob + pl.obg - 1) / pl.obg;
-    const int64_t lines = (int64_t)P.mesh_zbins * pl.nog * 2;
-    const int64_t target = pl.S == 1 ? kLineWgTarget : kLineWgTarget / 2;
-    const int64_t most = (P.Nx + 2 * pl.S - 1) / (2 * pl.S);   // two passes of rows or more
-    int64_t ng = (target + lines - 1) / lines;
-    ng = ng > most ? most : ng;
+    pl.obg = obg;
+    pl.nog = nog;
     // row groups that leave the workspace at the size of the phases', unless
     // that would halve them
     const int64_t M = (int64_t)P.mesh_xbins * P.mesh_zbins;

@@ -264,7 +264,7 @@ def test_wake_batch_limits():
         rc, msg, _ = pack(8, 4096, 4096, 1, 1, prec)
         assert rc == -3 and b"mesh points" in msg
         # 4096 workgroups and more of region 0 a task
-        rc, msg, batch = pack(4096, 33, 33, 2, 1500, prec)
+        rc, msg, batch = pack(4096, 33, 33, 32, 1500, prec)
         assert rc == 0 and batch.blocks_far * 256 >= 1 << 32, msg
         assert batch.forms & 2
         # 1.18e9 columns of 2 x 500000 x 1184: by phases
@@ -272,6 +272,44 @@ def test_wake_batch_limits():
         assert rc == 0 and batch.forms == 2, msg
         rc, msg, batch = pack(1, 33, 500000, 1, 1184, prec)
         assert rc == 0 and batch.forms == 1, msg
+
+
+def _forms(xb, zb, Nx, Nz, prec):
+    """The form (DfcsrWakeBatch.forms) a mesh off the chirp branch packs to."""
+    import ctypes
+    lib = _lib.load()
+    h = _lib.History(1, 2, 3, None, None, 8, 0, 5, 16, 16, 0, 0, 0, 1, 1, 1)
+    h.cells, h.cells32, h.dcells32 = 7, 8, 9
+    p = _params(0.3)
+    p.Nx, p.Nz, p.mesh_xbins, p.mesh_zbins = Nx, Nz, xb, zb
+    out, batch = (_lib.c_dp * 1)(8), _lib.WakeBatch()
+    nb = int(lib.dfcsr_wake_task_table_bytes(1))
+    assert lib.dfcsr_wake_tasks_pack(
+        1, (_lib.History * 1)(h), (_lib.Lattice * 1)(_lib.Lattice(3, 100, 1, 0.0, 0.01, 4, 5)),
+        (_lib.WakeParams * 1)(p), prec, out, out, ctypes.create_string_buffer(nb), nb,
+        ctypes.byref(batch)) == 0, lib.dfcsr_last_error()
+    return batch.forms
+
+
+def test_wake_forms_by_size():
+    """Z lines (2: 33 or more x bins, 4: 17 to 32, float64) need 192 workgroups
+    of the near regions, the lanes without an observer taken off: a workgroup
+    takes a z line, one of two regions and two passes of rows or more (a row a
+    pass, with 17 to 32 x bins two).  Mixed precision needs 384, and 33 x bins.
+    Fewer go by phases (1)."""
+    F, M = _lib.DFCSR_PREC_FP64, _lib.DFCSR_PREC_MIXED
+    for prec in (F, M):
+        assert _forms(16, 64, 200, 200, prec) == 1
+        assert _forms(33, 20, 40, 200, prec) == 2    # 20 x 2 x 20, 33 lanes of 64
+        assert _forms(300, 2, 33, 500, prec) == 1
+        assert _forms(130, 4, 16, 500, prec) == 1
+    assert _forms(20, 20, 40, 100, F) == 4 and _forms(20, 20, 40, 100, M) == 1
+    assert _forms(17, 1, 200, 200, F) == 1
+    assert _forms(32, 12, 32, 100, F) == 4 and _forms(32, 12, 28, 100, F) == 1   # 24 x 8, 24 x 7
+    assert _forms(64, 8, 24, 100, F) == 2 and _forms(64, 8, 22, 100, F) == 1     # 16 x 12, 16 x 11
+    assert _forms(64, 8, 48, 100, M) == 2 and _forms(64, 8, 46, 100, M) == 1     # 16 x 24, 16 x 23
+    assert _forms(256, 4, 48, 100, F) == 2 and _forms(256, 4, 46, 100, F) == 1   # 8 x 24, 8 x 23
+    assert _forms(129, 20, 33, 500, M) == 1 and _forms(192, 20, 33, 500, M) == 2   # 40 x 17
 
 
 def test_bench_workload_lattices():

@@ -348,6 +348,65 @@ def test_wake_line_form(K, ws, mesh, nxz, sx, sz, t):
         assert 0 < n[1] <= n[0]
 
 
+# the same edges with z lines and rows enough that the line form is taken: one
+# and two observers past a quarter, half and whole wave, several blocks, an odd
+# last pass of rows, tiled windows, columns past 256, the mesh past the lattice
+@pytest.mark.parametrize("mesh,nxz,sx,sz,t", [
+    ((17, 46), (13, 9), 20e-6, 80e-6, 0.33), ((32, 24), (24, 31), 50e-6, 50e-6, 0.33),
+    ((33, 34), (22, 40), 300e-6, 30e-6, 0.33), ((64, 10), (41, 33), 20e-6, 80e-6, 0.5),
+    ((65, 76), (9, 17), 50e-6, 50e-6, 0.33), ((129, 48), (16, 16), 300e-6, 30e-6, 0.5),
+    ((300, 28), (11, 12), 50e-6, 50e-6, 0.33), ((20, 52), (10, 300), 20e-6, 80e-6, 0.33),
+    ((35, 9), (79, 257), 20e-6, 80e-6, 0.33), ((34, 61), (12, 15), 50e-6, 50e-6, 1.1)])
+def test_wake_line_form_taken(K, ws, mesh, nxz, sx, sz, t):
+    """The wake by z lines on meshes that the rule of sizes gives to them (in
+    mixed precision from 33 x bins on) against the same wake by phases (explicit
+    observers), float64 within 1e-10 of max|W| and mixed within 1e-8; the oracle's
+    C integral within 1e-10 (mixed 1e-4) of max|dE_dct|, the size of the terms
+    that x_kick's sums cancel; batched bit for bit; the span table changes no bit
+    and evaluates no more points."""
+    from oracle import csr_ref_c as C
+    from tests.gpu_util import DeviceHistory, DeviceLattice, wake_params
+    from tests.test_abi import _forms
+    assert _forms(*mesh, *nxz, 0) == (4 if mesh[0] < 33 else 2)
+    assert _forms(*mesh, *nxz, 1) == (1 if mesh[0] < 33 else 2)
+    T, lat = _History(t, sx, sz), O.LatticeTables(LAT_ELEMENTS)
+    beam = dict(sigma_x=sx, sigma_z=sz, slope=np.array([0.3, 1e-6]), mean_x=0.0)
+    xa, za = (-5 * sx, 5 * sx, mesh[0]), (-5 * sz, 5 * sz, mesh[1])
+    L, args, M = DeviceLattice(lat, DEV), (t, beam, 0.05, 4.0, *nxz, 9.0), mesh[0] * mesh[1]
+    P = wake_params(*args, xa, za)
+    rings = ("fp64", "fp32t", "cells", "cells32")
+    H, Hz = (DeviceHistory(T, DEV, wrap=2, rings=r) for r in (rings, rings + ("zspan",)))
+    keep, ref = C._Keep(), None
+    for p, tol, oracle in ((0, 1e-10, 1e-10), (1, 1e-8, 1e-4)):
+        line = K.wake_mesh(H.desc, L.desc, P, p, DEV, ws)
+        obs = torch.stack([line["zmesh"].flatten(), line["xmesh"].flatten()], dim=1).contiguous()
+        Po = wake_params(*args, (0.0, 0.0, 1), (0.0, 0.0, M), observers=obs)
+        ph = K.wake_mesh(H.desc, L.desc, Po, p, DEV, ws)
+        if ref is None:
+            ref = C.wake(C.hist_from_tracker(T, keep), C.lat_from_tables(lat, keep), t, beam, 0.05,
+                         4.0, *nxz, 9.0, obs.cpu().numpy())
+        top = np.nanmax(np.abs(ref[0]))
+        for k, r in zip(("dE_dct", "x_kick"), ref):
+            a, b = line[k].cpu().numpy().ravel(), ph[k].cpu().numpy().ravel()
+            assert np.array_equal(np.isnan(a), np.isnan(b)), (p, k)
+            assert np.array_equal(np.isnan(a), np.isnan(r)), (p, k)
+            ok = np.isfinite(r)
+            assert ok.any() and np.abs(r[ok]).max() > 0
+            straight = k == "x_kick" and np.abs(r[ok]).max() < 1e-9 * top
+            assert np.abs(a - b)[ok].max() <= tol * (top if straight else np.abs(r[ok]).max()), (p, k)
+            assert np.abs(a - r)[ok].max() <= oracle * top, (p, k)
+        z = K.wake_mesh(Hz.desc, L.desc, P, p, DEV, ws)
+        o = [{k: torch.empty(M, dtype=torch.float64, device=DEV) for k in ("dE_dct", "x_kick")}
+             for _ in range(2)]
+        K.wake_mesh_batched([H.desc, Hz.desc], [L.desc] * 2, [P] * 2, p, o, DEV, ws)
+        for k in ("dE_dct", "x_kick"):
+            for v in (z[k], o[0][k], o[1][k]):
+                assert np.array_equal(line[k].cpu().numpy().ravel(), v.cpu().numpy().ravel(),
+                                      equal_nan=True), (p, k)
+        n = [K.wake_points_evaluated(h.desc, L.desc, P, p, DEV, ws) for h in (H, Hz)]
+        assert 0 < n[1] <= n[0]
+
+
 # s' columns in one to five groups of 64, dealt a wave each, shared by two or
 # four waves, or each to all waves; the chirp branch (four regions) and not
 @pytest.mark.parametrize("nz", [5, 64, 65, 128, 150, 200, 256, 257])
@@ -416,6 +475,41 @@ def test_wake_batch_forms_unset(K, ws, forms):
                 assert np.array_equal(w[n].cpu().numpy(), v[n].cpu().numpy(), equal_nan=True), (p, n)
 
 
+@pytest.mark.parametrize("forms", [0, -1, 8])
+def test_wake_batch_all_forms_unset(K, ws, forms):
+    """As test_wake_batch_forms_unset, with z lines enough for every form."""
+    import ctypes
+    from pydfcsr_amd import _lib
+    from tests.gpu_util import DeviceHistory, DeviceLattice, wake_params
+    sx, sz, t = 50e-6, 50e-6, 0.33
+    T, lat = _History(t, sx, sz), O.LatticeTables(LAT_ELEMENTS)
+    beam = dict(sigma_x=sx, sigma_z=sz, slope=np.array([0.3, 1e-6]), mean_x=0.0)
+    H = DeviceHistory(T, DEV, wrap=2, rings=("fp64", "fp32t", "cells", "cells32", "zspan"))
+    L, lib = DeviceLattice(lat, DEV), _lib.load()
+    Ps = [wake_params(t, beam, 0.05, 4.0, 70, 65, 9.0, (-sx, sx, m), (-sz, sz, 16))
+          for m in (5, 20, 33)]
+    k = len(Ps)
+    for p in (0, 1):
+        one = [K.wake_mesh(H.desc, L.desc, P, p, DEV, ws) for P in Ps]
+        o = [{n: torch.full_like(w[n], 7.0) for n in ("dE_dct", "x_kick")} for w in one]
+        host = torch.empty(lib.dfcsr_wake_task_table_bytes(k), dtype=torch.uint8)
+        batch = _lib.WakeBatch()
+        _lib.check(lib.dfcsr_wake_tasks_pack(
+            k, (_lib.History * k)(*[H.desc] * k), (_lib.Lattice * k)(*[L.desc] * k),
+            (_lib.WakeParams * k)(*Ps), p, (_lib.c_dp * k)(*[v["dE_dct"].data_ptr() for v in o]),
+            (_lib.c_dp * k)(*[v["x_kick"].data_ptr() for v in o]), host.data_ptr(), host.numel(),
+            ctypes.byref(batch)), "pack")
+        batch.forms = forms
+        dev = host.to(DEV)
+        part = torch.empty(int(batch.partial_bytes), dtype=torch.uint8, device=DEV)
+        _lib.check(lib.dfcsr_wake_batched_launch(
+            dev.data_ptr(), ctypes.byref(batch), p, part.data_ptr(), part.numel(),
+            torch.cuda.current_stream().cuda_stream), "launch")
+        for w, v in zip(one, o):
+            for n in v:
+                assert np.array_equal(w[n].cpu().numpy(), v[n].cpu().numpy(), equal_nan=True), (p, n)
+
+
 def test_wake_batch_of_many_launches(K, ws):
     """A batch whose region 0 takes more workgroups than a launch holds (4096
     tasks of 17 x 17 points, 1500 columns by z lines, a chirp-branch task among
@@ -427,13 +521,13 @@ def test_wake_batch_of_many_launches(K, ws):
     H = DeviceHistory(T, DEV, wrap=2, rings=("fp64", "cells", "zspan"))
     L = DeviceLattice(lat, DEV)
     P = [wake_params(t, dict(sigma_x=sx, sigma_z=sz, slope=np.array([s, 1e-6]), mean_x=0.0), 0.05,
-                     4.0, 3, 1500, 9.0, (-sx, sx, 17), (-sz, sz, 17)) for s in (0.3, -0.4, -1.7)]
+                     4.0, 48, 1500, 9.0, (-sx, sx, 17), (-sz, sz, 17)) for s in (0.3, -0.4, -1.7)]
     one = [K.wake_mesh(H.desc, L.desc, p, 0, DEV, ws) for p in P]
     which = [2 if j == 2000 else j % 2 for j in range(k)]
     out = {n: torch.full((k, 17 * 17), 7.0, dtype=torch.float64, device=DEV)
            for n in ("dE_dct", "x_kick")}
     o = [{n: v[j] for n, v in out.items()} for j in range(k)]
-    # (its 27 GB go with this workspace)
+    # (its 29 GB go with this workspace)
     K.wake_mesh_batched([H.desc] * k, [L.desc] * k, [P[w] for w in which], 0, o, DEV,
                         _lib.Workspace(DEV))
     for n in out:
