@@ -181,7 +181,8 @@ __global__ __launch_bounds__(kThreads) void zero_i32(int32_t *__restrict__ a, in
 }
 
 // ---- direct form: global atomics ---------------------------------------------
-// For grids whose row tiles do not suit LDS (tile_plan).  blockIdx.y: the
+// For grids whose row tiles do not suit LDS (tile_plan), and few particles on
+// many tiles (few_on_many).  blockIdx.y: the
 // grid (0: weights wA, 1: weights wB; null: unit weights).
 __global__ __launch_bounds__(kThreads) void cic_kernel(
     const double *__restrict__ q1, const double *__restrict__ q2,
@@ -286,6 +287,20 @@ TilePlan tile_plan(int nb1, int nb2) {
     }
   }
   return p;
+}
+
+// Few particles on a grid of many tiles, or of many rows (each workgroup makes a
+// map of them): zeroing and storing the tiles' LDS takes longer than the direct
+// form's atomics.  Measured, both grids, tiles / direct, us: 640 x 640 (45
+// tiles a grid) at 100 particles 27 / 16, at 1e4 33 / 21, at 3e4 34 / 35; 400 x
+// 400 (17) 19 / 16, 25 / 20, 30 / 37; 20000 x 3 25 / 16, 28 / 20, 34 / 31; 300 x
+// 300 (10) 16 / 17, 21 / 20, 28 / 40; one grid of 400 x 400 16 / 18, 20 / 19.
+// Either way the sums, and so the grids, are the same.
+constexpr int64_t kFewParticles = 10240;
+constexpr int kManyTiles = 24, kManyRows = 8192;
+
+bool few_on_many(const TilePlan &p, int ngrid, int nb1, int64_t n) {
+  return n <= kFewParticles && (p.T * ngrid >= kManyTiles || nb1 >= kManyRows);
 }
 
 // Chunks of the particles per tile and grid: at most kMaxWg workgroups.
@@ -519,7 +534,7 @@ int deposit_impl(const char *who, const double *q1, const double *q2, const doub
   const double *wmax = wB ? wB : wA;   // the non-unit weight, if any
   if (wmax) hipLaunchKernelGGL(absmax_partial, dim3(nb), dim3(kThreads), 0, s, wmax, n, hdr + 8);
   const TilePlan t = tile_plan(nb1, nb2);
-  if (t.T) {
+  if (t.T && !few_on_many(t, ngrid, nb1, n)) {
     int chunks = tile_chunks(t, ngrid, n);
     const int64_t per = n > 0 ? (n + chunks - 1) / chunks : 1;
     auto kernel = t.T > 2 ? cic_tile_kernel<true> : cic_tile_kernel<false>;

@@ -65,6 +65,25 @@ def test_deposit_forms(K, ws, bins, n):
         assert rel_max(v3.cpu(), O.histogram_cic_2d(x[ok], z[ok], bad[ok], *a)) <= 1e-13
 
 
+# grids of many tiles or rows at either side of the line between few particles
+# (direct) and more (tiles)
+@pytest.mark.parametrize("bins", [(400, 401), (700, 690), (9000, 5), (41, 4001)])
+@pytest.mark.parametrize("n", [1, 10240, 10241])
+def test_deposit_few_on_many(K, ws, bins, n):
+    """As test_deposit_forms; and the same sums bit for bit with particles off
+    the grid beside them, up to a count that takes the tiles (8192 to 16383
+    particles share one scale)."""
+    test_deposit_forms(K, ws, bins, n)
+    n = max(n, 8192)
+    rng = np.random.default_rng(n)
+    x, z, px = rng.normal(0.0, 1.0, n), rng.normal(0.0, 1.0, n), rng.normal(0.0, 1e-3, n)
+    a, off = (bins[0], -2.5, 2.5, bins[1], -2.0, 2.25), 16383 - n
+    d, v = (t.clone() for t in K.deposit_density_vx(_t(x), _t(z), _t(px), *a, ws))
+    e, w = K.deposit_density_vx(*(_t(np.append(t, np.full(off, c)))
+                                  for t, c in ((x, 9.0), (z, 9.0), (px, 0.0))), *a, ws)
+    assert torch.equal(d, e) and torch.equal(v, w)
+
+
 # whole grid in one tile, row tiles, and the direct form; few particles and
 # counts either side of a power of two
 @pytest.mark.parametrize("bins", [(16, 16), (256, 256), (1500, 1300)])
