@@ -33,6 +33,11 @@ constexpr int kLdsBytes = 160 * 1024;
 // 4e5 8 / 12, at 1e6 21 / 19; 256 x 256 at 1e6 28 / 25.  dE alone: 64 x 64 at
 // 2e6 19 / 19, at 3e6 27 / 25; 128 x 128 at 3e6 28 / 29, at 8e6 83 / 60.
 constexpr int64_t kLdsFromTwo = 1250000, kLdsFromOne = 4000000;
+// ... on meshes of at most this many times the points that LDS holds: past it
+// too few particles are in the middle.  Both kicks: 512 x 512 (26 times) at
+// 2e6 42 / 38, at 1e7 262 / 205; 850 x 850 (71) 46 / 49, 285 / 259; 1024 x 1024
+// (102) 49 / 53, 294 / 277; 2048 x 2048 96 / 105, 475 / 491.
+constexpr int64_t kLdsMeshes = 64;
 
 // A linspace axis with its step formed once: the interval of v as
 // rgi_interval finds it (its guess may come from the reciprocal of the step,
@@ -225,8 +230,9 @@ extern "C" int dfcsr_apply_wakes(double *px, double *pz, const double *x, const 
   const MeshAxis ax = make_axis(xr0, xr1, xbins), az = make_axis(zr0, zr1, zbins);
   hipStream_t s = as_stream(stream);
   // (a mesh one point wide has no cells: no particle is kicked)
-  if (n >= (transverse_on ? kLdsFromTwo : kLdsFromOne) && xbins >= 2 && zbins >= 2) {
-    const int value = transverse_on ? 16 : 8;
+  const int value = transverse_on ? 16 : 8;
+  if (n >= (transverse_on ? kLdsFromTwo : kLdsFromOne) && xbins >= 2 && zbins >= 2 &&
+      (int64_t)xbins * zbins <= kLdsMeshes * (kLdsBytes / value)) {
     const MeshPart part = middle(xbins, zbins, kLdsBytes / value);
     const int64_t bytes = (int64_t)part.ni * part.nj * value;
     int64_t b = (n + kLdsThreads - 1) / kLdsThreads;

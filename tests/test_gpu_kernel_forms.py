@@ -280,6 +280,14 @@ def test_kick_thin_meshes(K, nx, nz, two):
     test_kick_forms(K, nx, nz, two)
 
 
+# the largest meshes of which the middle is held, and the next
+@pytest.mark.parametrize("nx,nz,two", [(1024, 640, 1), (1024, 641, 1), (2048, 640, 0),
+                                       (2048, 641, 0)])
+def test_kick_large_meshes(K, nx, nz, two):
+    """As test_kick_forms."""
+    test_kick_forms(K, nx, nz, two)
+
+
 LAT_ELEMENTS = [dict(type="drift", L=0.1, nsep=1), dict(type="dipole", L=0.3, angle=0.05, nsep=1),
                 dict(type="drift", L=0.4, nsep=2), dict(type="dipole", L=0.3, angle=-0.05, nsep=1)]
 
