@@ -24,20 +24,26 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kMaxJobs = 4096;
 
-// Jobs of one launch, as a kernel argument: no copy of them on the stream.
-constexpr int kJobs = 16;
+// Jobs of one launch, as a kernel argument: no copy of them on the stream.  A
+// step has one or two; a whole history's go 64 a launch (3 KB of the 4 KB that
+// arguments may take), or a small grid's launches would be all its time: 64
+// slices onto 37 x 70 52 us with 16 a launch, 31 with 64.
+constexpr int kJobs = 16, kManyJobs = 64;
+template <int kN>
 struct RegridJobs {
-  DfcsrRegridJob j[kJobs];
+  DfcsrRegridJob j[kN];
 };
+static_assert(sizeof(RegridJobs<kManyJobs>) <= 3072, "kernel arguments");
 
 // per-job mean of the raw vx_x field (np.mean(vx_x), deposit.py:332, 384):
 // one workgroup a job, wide enough that a 100 x 100 slice is ten loads in
 // flight a thread (12 us as 256 threads, 5 us now)
 constexpr int kMeanThreads = 1024;
 
+template <int kN>
 __global__ __launch_bounds__(kMeanThreads) void vxx_mean_kernel(const double *__restrict__ src,
                                                                 int64_t slot_stride,
-                                                                RegridJobs jobs,
+                                                                RegridJobs<kN> jobs,
                                                                 double *__restrict__ means) {
   __shared__ double red[kMeanThreads / 64];
   const DfcsrRegridJob &J = jobs.j[blockIdx.x];
@@ -77,8 +83,9 @@ __device__ inline AxisAt axis_at(double q, double g0, double g1, int n) {
 // lane per record evaluating its four corners), into the float32 ones 19 (25).
 constexpr int kTX = 8, kTZ = 32, kNodeX = kTX + 1, kNodeZ = kTZ + 1;
 
+template <int kN>
 __global__ __launch_bounds__(kThreads) void regrid_kernel(
-    const double *__restrict__ src, int64_t slot_stride, RegridJobs jobs,
+    const double *__restrict__ src, int64_t slot_stride, RegridJobs<kN> jobs,
     const double *__restrict__ means, double *__restrict__ h64, float *__restrict__ h32,
     float *__restrict__ h32t, double *__restrict__ c64, float *__restrict__ c32, int Xi, int Zi,
     int cap, double xi0, double xi1, double zi0, double zi1) {
@@ -346,16 +353,20 @@ extern "C" int dfcsr_regrid(const double *src, int64_t src_slot_stride, const Df
   hipStream_t s = as_stream(stream);
   double *means = static_cast<double *>(ws);
   const int gx = ((Xi + kTX - 1) / kTX) * ((Zi + kTZ - 1) / kTZ);
-  for (int k = 0; k < njobs; k += kJobs) {
-    const int m = njobs - k < kJobs ? njobs - k : kJobs;
-    RegridJobs J = {};
-    for (int i = 0; i < m; ++i) J.j[i] = jobs[k + i];
-    hipLaunchKernelGGL(vxx_mean_kernel, dim3(m), dim3(kMeanThreads), 0, s, src, src_slot_stride, J,
-                       means + k);
-    hipLaunchKernelGGL(regrid_kernel, dim3(gx, m), dim3(kThreads), 0, s, src, src_slot_stride, J,
-                       (const double *)(means + k), hist64, hist32, hist32t, cells, cells32, Xi, Zi,
-                       cap, xi0, xi1, zi0, zi1);
-  }
+  const auto launch = [&](auto J) {
+    constexpr int N = sizeof(J.j) / sizeof(J.j[0]);
+    for (int k = 0; k < njobs; k += N) {
+      const int m = njobs - k < N ? njobs - k : N;
+      for (int i = 0; i < m; ++i) J.j[i] = jobs[k + i];
+      hipLaunchKernelGGL(vxx_mean_kernel<N>, dim3(m), dim3(kMeanThreads), 0, s, src,
+                         src_slot_stride, J, means + k);
+      hipLaunchKernelGGL(regrid_kernel<N>, dim3(gx, m), dim3(kThreads), 0, s, src,
+                         src_slot_stride, J, (const double *)(means + k), hist64, hist32, hist32t,
+                         cells, cells32, Xi, Zi, cap, xi0, xi1, zi0, zi1);
+    }
+  };
+  if (njobs > kJobs) launch(RegridJobs<kManyJobs>{});
+  else launch(RegridJobs<kJobs>{});
   DFCSR_LAUNCH_CHECK("regrid");
   return DFCSR_OK;
 }

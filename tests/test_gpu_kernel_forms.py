@@ -227,6 +227,30 @@ def test_df_forms(K, ws, nx, nz, window, order):
         assert np.array_equal(g.cpu().numpy(), h.cpu().numpy(), equal_nan=True)
 
 
+@pytest.mark.parametrize("jobs", [16, 17, 64, 65, 131])
+def test_regrid_many_jobs(K, ws, jobs):
+    """Slices re-gridded in one call, whose jobs go 16 or 64 a launch, against
+    the same slices in calls of one: every ring bit for bit."""
+    rng = np.random.default_rng(jobs)
+    nb, Xi, Zi, cap = (7, 9), 11, 35, jobs + 2
+    src = _t(rng.normal(0.0, 1.0, (jobs, 5, *nb)))
+    J = [(j, (3 * j) % cap if cap % 3 else j, *nb, -1.0 - 0.01 * j, 1.2, -1.0, 1.0 + 0.02 * j)
+         for j in range(jobs)]
+
+    def rings(calls):
+        f64, f32 = (dict(dtype=d, device=DEV) for d in (torch.float64, torch.float32))
+        h64, h32t = torch.zeros((Xi, Zi, cap, 20), **f64), torch.zeros((Xi, Zi, cap, 20), **f32)
+        h32 = torch.zeros((Xi, cap, 5, Zi, 4), **f32)
+        c, c32 = torch.zeros((cap, Xi, Zi + 1, 5), **f64), torch.zeros((cap, Xi, Zi + 1, 5), **f32)
+        for k in calls:
+            K.regrid(src, 5 * nb[0] * nb[1], k, h64, h32, Xi, Zi, -1.1, 1.1, -1.05, 1.5, ws, h32t,
+                     c, c32)
+        return h64, h32, h32t, c, c32
+
+    for a, b in zip(rings([J]), rings([[j] for j in J])):
+        assert a.any() and torch.equal(a, b)
+
+
 # the smallest mesh, one that is no mesh, odd ones, the largest two wakes and
 # the largest one wake that fit the LDS whole, and meshes of which the middle is
 # held: one row too many, thin ones
