@@ -723,14 +723,6 @@ __host__ __device__ inline int64_t line_at(const WakeTask &T, int zl) {
   return T.line + (int64_t)zl * (kLineHead + 2 * (int64_t)T.P.Nz * T.cstride);
 }
 
-// x' (r in region 0 .. 2) and s' axes of region r for mesh point i.
-__device__ inline const double *xaxis_at(const WakeTask &T, const double *ws, int i, int r) {
-  return T.line ? ws + line_at(T, i % T.P.mesh_zbins) + 4 * r : ws + obs_at(T, i) + 16 + 4 * r;
-}
-__device__ inline const double *saxis_at(const WakeTask &T, const double *ws, int i, int r) {
-  return T.line ? ws + line_at(T, i % T.P.mesh_zbins) + 12 + 4 * r : ws + obs_at(T, i) + 32 + 4 * r;
-}
-
 // Integrates phase ph of the mesh point whose observer data is od; every
 // thread returns the block sums of wz_k wx_j (I_z, I_x) over the phase.
 // kTI (mixed only): read the time-innermost FP32 ring.  kCells (a
@@ -929,8 +921,9 @@ __device__ inline void run_phase_block(const WakeTask &T, int l, double *__restr
 // w integrates, for observer ol of the block, column block (4 g + w) S + sub
 // over every row of region 0 inside the history; the workgroup's 4 S column
 // blocks are added in order into one partial sum per observer (NaN where the
-// reference's integrand is 0/0 over the region, as wake_phase).  Summation: per column over the rows in order, weighted sums
-// over the block's columns in order.  kSkip: lookups the history's span
+// reference's integrand is 0/0 over the region, as wake_phase).  Summation:
+// per column over the rows in order, weighted sums over the block's columns in
+// order.  kSkip: lookups the history's span
 // table shows to gather zero density and gradients are skipped (an integrand
 // of exactly 0, as in the near regions); every entry is read from the table
 // itself (zrow = the table, zt0 = nt: no LDS copy of the newest slices).
@@ -939,7 +932,7 @@ __device__ void far_obs_block(const WakeTask &T, int l, double *__restrict__ par
                               RowTable &rt) {
   const DfcsrHistory &H = T.H;
   const DfcsrLattice &L = T.L;
-  const PhasePlan pl = make_plan(T.P, T.cstride);
+  const PhasePlan pl = make_plan(T.P, 0);
   const int xb = T.P.mesh_xbins, zb = T.P.mesh_zbins;
   const int per_line = pl.nob * pl.nA;
   const int zl = l / per_line, rem = l - zl * per_line;
@@ -959,8 +952,8 @@ __device__ void far_obs_block(const WakeTask &T, int l, double *__restrict__ par
   const double inv_ds = 1.0 / L.ds;
   // the z line's x' rows (the same for every observer of the line) and this
   // observer's s' columns (the same too, off the chirp branch)
-  const LinAxis xa = load_axis(xaxis_at(T, partials, ob * pl.W * zb + zl, 0));
-  const LinAxis sa = load_axis(saxis_at(T, partials, i, 0));
+  const LinAxis xa = load_axis(partials + obs_at(T, ob * pl.W * zb + zl) + 16);
+  const LinAxis sa = load_axis(od + 32);
   double *out = partials + T.part + ((int64_t)i * (pl.nA + pl.nB) + g) * 2;
   const bool writer = wave == 0 && sub == 0 && valid;
   if (xa.n < 2 || sa.n < 2) {   // trapz over a single sample (uniform)
@@ -1474,7 +1467,8 @@ extern "C" int dfcsr_wake_mesh(const DfcsrHistory *hist, const DfcsrLattice *lat
     return set_error(DFCSR_ENOWS, "wake_mesh: workspace of %lld bytes, %lld needed",
                      (long long)ws_bytes, (long long)least);
   WakeTask T;
-  if ((rc = make_task(*hist, *lat, *p, precision, ws_bytes / (int64_t)sizeof(double), dE_dct, x_kick, xmesh, zmesh, T, "wake_mesh")))
+  if ((rc = make_task(*hist, *lat, *p, precision, ws_bytes / (int64_t)sizeof(double), dE_dct,
+                      x_kick, xmesh, zmesh, T, "wake_mesh")))
     return rc;
   double *part = static_cast<double *>(ws);
   hipStream_t s = as_stream(stream);
