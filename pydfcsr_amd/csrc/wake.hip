@@ -1099,14 +1099,14 @@ __host__ __device__ inline bool cells32_ring32(const DfcsrHistory &H) {
 
 // Workgroups per CU the register allocation must allow: the near phases on
 // the cell-major ring 4 (128 registers), the others 2.  The launch's
-// workgroups are those from `first` on of the nb (launch_blocks).
+// workgroups are those from `first` on (launch_blocks).
 template <bool kMixed, bool kNear, bool kTI, int kCells = kRings>
 __global__ __launch_bounds__(kThreads, kCells ? 4 : DFCSR_WAKE_MINBLOCKS) void wake_phase_kernel(
-    WakeTask T, int first, int nb, double *__restrict__ partials) {
+    WakeTask T, int first, double *__restrict__ partials) {
   __shared__ double red[kThreads / 64];
-  const int b = first + (int)blockIdx.x;
+  const int b = blockIdx.x, nb = gridDim.x;
   run_phase_block<kMixed, kNear, kTI, kCells>(
-      T, kNear ? xcd_group<true>(b, nb, kNearGroup) : xcd_remap(b, nb), partials, red);
+      T, first + (kNear ? xcd_group<true>(b, nb, kNearGroup) : xcd_remap(b, nb)), partials, red);
 }
 
 // The observer-major region-0 launch.  kSkip: the span-table skip (far_skip,
@@ -1119,11 +1119,11 @@ __global__ __launch_bounds__(kThreads, kCells ? 4 : DFCSR_WAKE_MINBLOCKS) void w
 // the whole wake).
 template <bool kMixed, bool kTI, bool kSkip = false>
 __global__ __launch_bounds__(kThreads, !kMixed && kSkip ? 4 : 3) void wake_far_kernel(
-    WakeTask T, int first, int nb, double *__restrict__ partials) {
+    WakeTask T, int first, double *__restrict__ partials) {
   __shared__ RowTable rt;
-  const int b = first + (int)blockIdx.x;
+  const int b = blockIdx.x, nb = gridDim.x, per_line = max(nb / T.P.mesh_zbins, 1);
   far_obs_block<kMixed, kTI, kSkip>(
-      T, kSkip ? xcd_group<false>(b, nb, nb / T.P.mesh_zbins) : xcd_remap(b, nb), partials, rt);
+      T, first + (kSkip ? xcd_group<false>(b, nb, per_line) : xcd_remap(b, nb)), partials, rt);
 }
 
 // Whether a wake's observer-major region 0 skips lookups on the span table:
@@ -1489,7 +1489,7 @@ extern "C" int dfcsr_wake_mesh(const DfcsrHistory *hist, const DfcsrLattice *lat
   } else {
     const auto launch = [&](auto kernel, int64_t blocks) {
       launch_blocks(blocks, [&](int first, dim3 g) {
-        hipLaunchKernelGGL(kernel, g, dim3(kThreads), 0, s, T, first, (int)blocks, part);
+        hipLaunchKernelGGL(kernel, g, dim3(kThreads), 0, s, T, first, part);
       });
     };
     const bool skip = far_skip(*hist, pl);
