@@ -2,7 +2,7 @@
 //
 // Replaces CSR2D.get_CSR_mesh / calculate_2D_CSR / get_CSR_wake /
 // get_CSR_integrand (CSR.py:361-782).  Off the chirp branch, with cell-major
-// rings and enough x bins (make_plan), a mesh is integrated by z lines
+// rings and enough x bins (by_lines), a mesh is integrated by z lines
 // (wake_line.h); what follows is the form of every other wake.  A mesh
 // point's integral over its regions (3 without chirp, 4 with) is split into
 // phases: one phase is one region and one chunk of its x' rows, over all s'
@@ -476,21 +476,6 @@ constexpr int kLineWgTarget = 4096;
 // 811 / 761 / 748 / 766 (as many as the observer-major form's: 2656, 491, 284,
 // 794).
 constexpr int kLineFarTarget = 6144;
-// Fewest workgroups of a line-form near launch, the share of lanes without an
-// observer taken off: below, a mesh of few z lines or an integration of few rows
-// goes by phases, which have a workgroup a mesh point and leave less of the chip
-// idle.  Measured on 4000 wakes of 17 to 300 x 1 to 128 points, 8 to 500 rows
-// and columns, how many are slower than by phases (over 3 %), and the worst:
-// float64 408 of 2002 and 7.6 times by lines alone, 17 and 1.37 times from 192 on (33 and 1.76 from
-// 160, 7 and 1.29 from 256, which gives more of the gain away); mixed 588 of 1998 and 6.7 times, 30
-// and 1.34 from 384 (77 and 1.59 from 256, 15 and 1.20 from 512).  20 z lines
-// of 20 x bins with 40 rows have 250 (float64), of 33 x bins 412.
-constexpr int kLineLeast = 192, kLineLeastMixed = 384;
-
-// Most near-region columns of a mesh by z lines: a thread of the observer
-// launch steps past the last by up to 15 x 2^24 (mesh points, check_params), and
-// that fits an int.
-constexpr int64_t kMaxLineColumns = (int64_t)1 << 30;
 
 // Doubles per mesh point of a wake by phases: partial sums and observer data.
 __host__ __device__ inline int64_t point_doubles(const PhasePlan &pl) {
@@ -507,8 +492,27 @@ __host__ __device__ inline int64_t point_doubles(const PhasePlan &pl) {
 // 1387 / 1346 / 1351).
 constexpr int kFarWaveTarget = 8192;
 
-// cstride: doubles per column of the line form, 0 when the history lacks the
-// rings it reads (line_stride).
+// Line form: observer blocks per workgroup of the near launch, groups of them per
+// z line, and the most row groups per region.
+struct LineGroups {
+  int obg, nog;
+  int64_t ng;
+};
+
+__host__ __device__ inline LineGroups line_groups(const PhasePlan &pl, const DfcsrWakeParams &P) {
+  LineGroups g;
+  g.obg = pl.nob == 1 ? 1 : (pl.nob == 2 ? 2 : 4);
+  g.nog = (pl.nob + g.obg - 1) / g.obg;
+  const int64_t lines = (int64_t)P.mesh_zbins * g.nog * 2;
+  const int64_t target = pl.S == 1 ? kLineWgTarget : kLineWgTarget / 2;
+  const int64_t most = (P.Nx + 2 * pl.S - 1) / (2 * pl.S);   // two passes of rows or more
+  g.ng = (target + lines - 1) / lines;
+  g.ng = g.ng > most ? most : g.ng;
+  return g;
+}
+
+// cstride: doubles per column of the line form, 0 for a wake by phases
+// (line_stride decides).
 __host__ __device__ inline PhasePlan make_plan(const DfcsrWakeParams &P, int cstride) {
   PhasePlan pl;
   pl.nreg = (fabs(P.slope0) <= 1) ? 3 : 4;   // the branch test of make_regions
@@ -542,41 +546,24 @@ __host__ __device__ inline PhasePlan make_plan(const DfcsrWakeParams &P, int cst
     pl.W = pl.S = pl.nob = pl.q = 0;
     pl.nA = pl.ch0;
   }
-  // By z lines: off the chirp branch (all observers of a line then share rows
-  // and columns), from more than a quarter wave of observers (float64) or half
-  // a wave (mixed: the phases' cells are half as large and cached).  Measured,
-  // lines / phases, us, mesh x bins by 32, 200 x 200 points: float64 17: 480 /
-  // 620, 32: 500 / 749, 48: 671 / 1125 (16 by phases 470); mixed 17: 496 / 382,
-  // 32: 494 / 484, 33: 623 / 639, 48: 628 / 733.
-  // A launch's threads count a mesh's columns in 32 bits (kMaxLineColumns).
-  pl.line = false;
+  pl.line = cstride != 0;
   pl.obg = pl.nog = pl.ng = 0;
-  if (cstride && pl.obs_major && pl.nreg == 3 && pl.S <= (cstride == kColMixed ? 1 : 2) &&
-      2 * (int64_t)P.Nz * P.mesh_zbins <= kMaxLineColumns) {
-    const int obg = pl.nob == 1 ? 1 : (pl.nob == 2 ? 2 : 4), nog = (pl.nob + obg - 1) / obg;
-    const int64_t lines = (int64_t)P.mesh_zbins * nog * 2;
-    const int64_t target = pl.S == 1 ? kLineWgTarget : kLineWgTarget / 2;
-    const int64_t most = (P.Nx + 2 * pl.S - 1) / (2 * pl.S);   // two passes of rows or more
-    int64_t ng = (target + lines - 1) / lines;
-    ng = ng > most ? most : ng;
-    // few lines or rows leave most of the chip idle
-    const int64_t least = cstride == kColMixed ? kLineLeastMixed : kLineLeast;
-    if (lines * ng * P.mesh_xbins < least * nog * obg * pl.W) return pl;
-    pl.line = true;
+  if (pl.line) {
+    const LineGroups g = line_groups(pl, P);
+    pl.obg = g.obg;
+    pl.nog = g.nog;
     // region 0: a workgroup's four waves take columns of their own, S rows at a
     // time
     const int fl = P.mesh_zbins * pl.nob, fmost = (P.Nz + 3) / 4;
     const int fq = (kLineFarTarget + fl - 1) / fl;
     pl.nA = fq > fmost ? fmost : fq;
-    pl.obg = obg;
-    pl.nog = nog;
     // row groups that leave the workspace at the size of the phases', unless
     // that would halve them
     const int64_t M = (int64_t)P.mesh_xbins * P.mesh_zbins;
     const int64_t room = (point_doubles(pl) - kObsLine - 2 * pl.nA) * M -
                          (int64_t)P.mesh_zbins * (kLineHead + 2 * (int64_t)P.Nz * cstride);
     const int64_t fit = room / (4 * M);
-    pl.ng = (int)(fit < ng && 2 * fit >= ng ? fit : ng);
+    pl.ng = (int)(fit < g.ng && 2 * fit >= g.ng ? fit : g.ng);
     pl.nB = 2 * pl.ng;
   }
   return pl;
@@ -1346,11 +1333,43 @@ int check_rings(const DfcsrHistory &H, int precision, const char *who) {
   return DFCSR_OK;
 }
 
-// Doubles per column of the line form of this precision, 0 when the history
-// lacks the cell-major rings it reads.
-int line_stride(const DfcsrHistory &H, int precision) {
-  if (precision == DFCSR_PREC_FP64) return H.cells ? kColFp64 : 0;
-  return mixed_cells(H) ? kColMixed : 0;
+// Most near-region columns of a mesh by z lines: a thread of the observer
+// launch steps past the last by up to 15 x 2^24 (mesh points, check_params), and
+// that fits an int.
+constexpr int64_t kMaxLineColumns = (int64_t)1 << 30;
+
+// Fewest workgroups of a line-form near launch, the share of lanes without an
+// observer taken off: below, a mesh of few z lines or an integration of few rows
+// goes by phases, which have a workgroup a mesh point and leave less of the chip
+// idle.  Measured on 4000 wakes of 17 to 300 x 1 to 128 points, 8 to 500 rows
+// and columns, how many are slower than by phases (over 3 %), and the worst:
+// float64 408 of 2002 and 7.6 times by lines alone, 17 and 1.37 times from 192 on (33 and 1.76 from
+// 160, 7 and 1.29 from 256, which gives more of the gain away); mixed 588 of 1998 and 6.7 times, 30
+// and 1.34 from 384 (77 and 1.59 from 256, 15 and 1.20 from 512).  20 z lines
+// of 20 x bins with 40 rows have 250 (float64), of 33 x bins 412.
+constexpr int kLineLeast = 192, kLineLeastMixed = 384;
+
+// Whether a wake goes by z lines, where its history has the rings: off the
+// chirp branch (all observers of a line then share rows and columns), from more
+// than a quarter wave of observers (float64) or half a wave (mixed: the phases'
+// cells are half as large and cached), with workgroups and columns as above.
+// Measured, lines / phases, us, mesh x bins by 32, 200 x 200 points: float64
+// 17: 480 / 620, 32: 500 / 749, 48: 671 / 1125 (16 by phases 470); mixed 17:
+// 496 / 382, 32: 494 / 484, 33: 623 / 639, 48: 628 / 733.
+bool by_lines(const DfcsrWakeParams &P, bool mixed) {
+  const PhasePlan pl = make_plan(P, 0);
+  if (!pl.obs_major || pl.nreg != 3 || pl.S > (mixed ? 1 : 2)) return false;
+  if (2 * (int64_t)P.Nz * P.mesh_zbins > kMaxLineColumns) return false;
+  const LineGroups g = line_groups(pl, P);
+  const int64_t near = 2 * (int64_t)P.mesh_zbins * g.nog * g.ng;   // (two regions)
+  return near * P.mesh_xbins >= (int64_t)(mixed ? kLineLeastMixed : kLineLeast) * g.nog * g.obg * pl.W;
+}
+
+// Doubles per column of a wake by z lines, 0 for one by phases.
+int line_stride(const DfcsrHistory &H, const DfcsrWakeParams &P, int precision) {
+  const bool mixed = precision == DFCSR_PREC_MIXED;
+  if (!(mixed ? mixed_cells(H) : H.cells != nullptr) || !by_lines(P, mixed)) return 0;
+  return mixed ? kColMixed : kColFp64;
 }
 
 // check_params without setting the error message (for the size queries).
@@ -1367,9 +1386,10 @@ int64_t phase_doubles(const DfcsrWakeParams &p) {
 
 int64_t partial_doubles(const DfcsrWakeParams &p) {
   int64_t n = phase_doubles(p);
-  for (int cs : {kColFp64, kColMixed}) {
-    const PhasePlan pl = make_plan(p, cs);
-    const int64_t m = pl.line ? line_doubles(pl, p, cs) : 0;
+  for (bool mixed : {false, true}) {
+    if (!by_lines(p, mixed)) continue;
+    const int cs = mixed ? kColMixed : kColFp64;
+    const int64_t m = line_doubles(make_plan(p, cs), p, cs);
     n = m > n ? m : n;
   }
   return n;
@@ -1380,8 +1400,9 @@ int64_t partial_doubles(const DfcsrWakeParams &p) {
 int make_task(const DfcsrHistory &H, const DfcsrLattice &L, const DfcsrWakeParams &P,
               int precision, int64_t room, double *dE, double *xk, double *xmesh, double *zmesh,
               WakeTask &T, const char *who) {
-  PhasePlan pl = make_plan(P, line_stride(H, precision));
-  if (pl.line && line_doubles(pl, P, line_stride(H, precision)) > room) pl = make_plan(P, 0);
+  int cstride = line_stride(H, P, precision);
+  if (cstride && line_doubles(make_plan(P, cstride), P, cstride) > room) cstride = 0;
+  const PhasePlan pl = make_plan(P, cstride);
   T.H = H;
   T.L = L;
   T.P = P;
@@ -1394,7 +1415,7 @@ int make_task(const DfcsrHistory &H, const DfcsrLattice &L, const DfcsrWakeParam
   T.obs = (int64_t)T.M * (pl.nA + pl.nB) * 2;
   T.ostride = pl.line ? kObsLine : kObsStride;
   T.line = pl.line ? T.obs + (int64_t)T.M * kObsLine : 0;   // > 0 in line form
-  T.cstride = pl.line ? line_stride(H, precision) : 0;
+  T.cstride = cstride;
   T.nA = pl.nA;
   T.nB = pl.nB;
   T.blockA0 = T.blockB0 = T.obs0 = 0;

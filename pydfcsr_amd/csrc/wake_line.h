@@ -18,7 +18,7 @@
 //     in flight over the points of the current ones.
 // z lines are dealt round the XCDs and rows round the workgroups, since those
 // near the bunch have most of the work (contiguous ranges per XCD: 1.3x
-// slower at 128 x 128).  The rule is make_plan's.
+// slower at 128 x 128).  The rule is by_lines.
 // Bound: vector ALU issue, about 95 (float64) and 125 (mixed) instructions a
 // point; near regions 86 % of the issue cycles.  Measured, the phase and
 // observer-major forms and this one: float64 128 x 128 mesh, 355 slices (near
