@@ -566,7 +566,10 @@ def main():
                                "wake_line_kernel for the near regions -- on the chirp branch "
                                "wake_far_kernel and wake_phase_kernel -- wake_finalize_kernel; "
                                "one stream, timed together)",
+                     # by z lines some of these are shared between observers: an
+                     # equivalent rate, not the share of the ALUs in use
                      "flops_per_point": FLOPS_PER_POINT,
+                     "flops": "reference formula, per evaluated point",
                      "points": "evaluated",
                      "nominal_equivalent_frac": round(achieved / frac_eval / peak, 4)},
         "init_s": round(t0 - t_init, 2),

@@ -213,7 +213,8 @@ int dfcsr_regrid(const double *src, int64_t src_slot_stride, const DfcsrRegridJo
  * z) everywhere.  With them the near-region phases of
  * a wake read cells (FP64 wakes: cells, mixed: cells32), whose neighbouring
  * z lie in neighbouring cells.  Off the chirp branch a mesh of 17 or more x
- * bins (mixed: 33 or more) is then integrated by z lines, from these rings
+ * bins (mixed: 33 or more), with z lines and rows enough to fill the GPU (20 z
+ * lines and 40 rows are), is then integrated by z lines, from these rings
  * alone: the results
  * differ from the phases' by rounding (float64 sums in another order; FP64
  * also interpolates along x first).  Otherwise they are identical with or

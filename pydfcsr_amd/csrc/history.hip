@@ -37,7 +37,7 @@ static_assert(sizeof(RegridJobs<kManyJobs>) <= 3072, "kernel arguments");
 
 // per-job mean of the raw vx_x field (np.mean(vx_x), deposit.py:332, 384):
 // one workgroup a job, wide enough that a 100 x 100 slice is ten loads in
-// flight a thread (12 us as 256 threads, 5 us now)
+// flight a thread (12 us as 256 threads, 4 us now)
 constexpr int kMeanThreads = 1024;
 
 template <int kN>

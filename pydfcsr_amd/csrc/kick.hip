@@ -12,9 +12,9 @@
 // time (512 cycles for the eight corners), so the wakes are held in LDS,
 // scaled once per mesh point: all of them, or the middle of the mesh that
 // fits, around which a bunch gathers, and the few particles outside read
-// global memory.  3e6 particles, both kicks of a
-// 128 x 128 mesh, MI355X: 38 us, 3.8 TB/s (67 from global memory, every corner
-// divided by the beam energy for each particle).
+// global memory.  3e6 particles, both kicks of a 128 x 128 mesh, MI355X: 33.5
+// us, 4.3 TB/s (58 from global memory, every corner divided by the beam energy
+// for each particle).
 #include <algorithm>
 
 #include "common.h"
