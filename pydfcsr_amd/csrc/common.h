@@ -31,6 +31,16 @@ int set_error(int code, const char *fmt, ...);
                                 hipGetErrorString(_e));                          \
   } while (0)
 
+// launch(first, n) for each launch of `blocks` workgroups of `threads`: a launch
+// of 2^32 threads or more (along x) runs the remainder alone, with no error, so
+// they are cut at 2^31.
+template <typename F>
+void launch_blocks(int64_t blocks, int threads, const F &launch) {
+  const int64_t most = ((int64_t)1 << 31) / threads;
+  for (int64_t at = 0; at < blocks; at += most)
+    launch((int)at, (unsigned)(blocks - at < most ? blocks - at : most));
+}
+
 // np.linspace(start, stop, num)[i]: y = i*step + start with step =
 // (stop - start)/(num - 1), two roundings (no fused multiply-add), and the
 // last point pinned to stop.  num == 1 gives start.

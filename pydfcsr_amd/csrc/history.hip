@@ -85,7 +85,7 @@ constexpr int kTX = 8, kTZ = 32, kNodeX = kTX + 1, kNodeZ = kTZ + 1;
 
 template <int kN>
 __global__ __launch_bounds__(kThreads) void regrid_kernel(
-    const double *__restrict__ src, int64_t slot_stride, RegridJobs<kN> jobs,
+    const double *__restrict__ src, int64_t slot_stride, RegridJobs<kN> jobs, int first,
     const double *__restrict__ means, double *__restrict__ h64, float *__restrict__ h32,
     float *__restrict__ h32t, double *__restrict__ c64, float *__restrict__ c32, int Xi, int Zi,
     int cap, double xi0, double xi1, double zi0, double zi1) {
@@ -94,7 +94,8 @@ __global__ __launch_bounds__(kThreads) void regrid_kernel(
   __shared__ double v[kNodeX * kNodeZ * 5];
   const DfcsrRegridJob &J = jobs.j[blockIdx.y];
   const int across = (Zi + kTZ - 1) / kTZ;
-  const int x0 = (int)blockIdx.x / across * kTX, z0 = (int)blockIdx.x % across * kTZ;
+  const int tile = first + (int)blockIdx.x;
+  const int x0 = tile / across * kTX, z0 = tile % across * kTZ;
   const int rows = min(kTX, Xi - x0), cols = min(kTZ, Zi - z0);
   const int t = threadIdx.x;
   if (t < kNodeX)
@@ -223,9 +224,9 @@ template <typename T>
 __global__ __launch_bounds__(kSpanThreads) void zspan_kernel(const T *__restrict__ cells,
                                                          uint32_t *__restrict__ zspan, int Xi,
                                                          int Zi, int cap, int head, int nt,
-                                                         int first) {
+                                                         int first, int block0) {
   __shared__ int lo_s[2][kSpanRows + 1], hi_s[2][kSpanRows + 1];
-  const int xb = blockIdx.x * kSpanRows;
+  const int xb = (block0 + (int)blockIdx.x) * kSpanRows;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwave = kSpanThreads / 64;
   const int nrow = min(kSpanRows + 1, Xi - xb);   // rows xb .. xb + nrow - 1 (x + 1 clamped)
   const int64_t plane = (int64_t)Xi * DFCSR_CELL_ROW(Zi) * DFCSR_CELL;
@@ -288,12 +289,14 @@ extern "C" int dfcsr_history_zspan(const double *cells, const float *cells32, ui
   int gy = nt - first;
   if (gy > 1024) gy = 1024;
   hipStream_t s = as_stream(stream);
-  if (cells)
-    hipLaunchKernelGGL(zspan_kernel<double>, dim3(gx, gy), dim3(kSpanThreads), 0, s, cells, zspan,
-                       Xi, Zi, cap, head, nt, first);
-  else
-    hipLaunchKernelGGL(zspan_kernel<float>, dim3(gx, gy), dim3(kSpanThreads), 0, s, cells32, zspan,
-                       Xi, Zi, cap, head, nt, first);
+  launch_blocks(gx, kSpanThreads, [&](int at, unsigned g) {
+    if (cells)
+      hipLaunchKernelGGL(zspan_kernel<double>, dim3(g, gy), dim3(kSpanThreads), 0, s, cells, zspan,
+                         Xi, Zi, cap, head, nt, first, at);
+    else
+      hipLaunchKernelGGL(zspan_kernel<float>, dim3(g, gy), dim3(kSpanThreads), 0, s, cells32,
+                         zspan, Xi, Zi, cap, head, nt, first, at);
+  });
   DFCSR_LAUNCH_CHECK("history_zspan");
   return DFCSR_OK;
 }
@@ -352,7 +355,7 @@ extern "C" int dfcsr_regrid(const double *src, int64_t src_slot_stride, const Df
   }
   hipStream_t s = as_stream(stream);
   double *means = static_cast<double *>(ws);
-  const int gx = ((Xi + kTX - 1) / kTX) * ((Zi + kTZ - 1) / kTZ);
+  const int64_t tiles = (int64_t)((Xi + kTX - 1) / kTX) * ((Zi + kTZ - 1) / kTZ);
   const auto launch = [&](auto J) {
     constexpr int N = sizeof(J.j) / sizeof(J.j[0]);
     for (int k = 0; k < njobs; k += N) {
@@ -360,9 +363,11 @@ extern "C" int dfcsr_regrid(const double *src, int64_t src_slot_stride, const Df
       for (int i = 0; i < m; ++i) J.j[i] = jobs[k + i];
       hipLaunchKernelGGL(vxx_mean_kernel<N>, dim3(m), dim3(kMeanThreads), 0, s, src,
                          src_slot_stride, J, means + k);
-      hipLaunchKernelGGL(regrid_kernel<N>, dim3(gx, m), dim3(kThreads), 0, s, src,
-                         src_slot_stride, J, (const double *)(means + k), hist64, hist32, hist32t,
-                         cells, cells32, Xi, Zi, cap, xi0, xi1, zi0, zi1);
+      launch_blocks(tiles, kThreads, [&](int first, unsigned g) {
+        hipLaunchKernelGGL(regrid_kernel<N>, dim3(g, m), dim3(kThreads), 0, s, src,
+                           src_slot_stride, J, first, (const double *)(means + k), hist64, hist32,
+                           hist32t, cells, cells32, Xi, Zi, cap, xi0, xi1, zi0, zi1);
+      });
     }
   };
   if (njobs > kJobs) launch(RegridJobs<kManyJobs>{});

@@ -1286,20 +1286,6 @@ __global__ __launch_bounds__(kThreads) void wake_finalize_batched_kernel(
   finalize_point(tasks[j], i - tasks[j].obs0, g % kSumLanes, partials);
 }
 
-// Most workgroups of one launch, of 512 threads or fewer: a launch of 2^32
-// threads or more runs the remainder alone, with no error.  A large mesh by
-// phases takes several (1200 x 1200 points, four regions of 200 rows: 17
-// million workgroups), and a large batch (region 0 of 4096 tasks of a 17 x 17
-// mesh with 1500 columns: 25 million).
-constexpr int kMaxGrid = 1 << 22;
-
-// launch(first, grid) for each launch of `blocks` workgroups.
-template <typename F>
-void launch_blocks(int64_t blocks, const F &launch) {
-  for (int64_t at = 0; at < blocks; at += kMaxGrid)
-    launch((int)at, dim3((unsigned)(blocks - at < kMaxGrid ? blocks - at : kMaxGrid)));
-}
-
 // Workgroups of a launch of `per` threads per mesh point.
 unsigned point_grid(int M, int per) {
   return (unsigned)(((int64_t)M * per + kThreads - 1) / kThreads);
@@ -1433,21 +1419,24 @@ enum { kFormPhases = 1, kFormLine1 = 2, kFormLine2 = 4 };
 // in 32 bits.
 constexpr int64_t kMaxPoints = INT32_MAX / (kObsThreads > kSumLanes ? kObsThreads : kSumLanes);
 
+// The launches of one region group of a batch.  A large one takes several each
+// (region 0 of 4096 tasks of a 17 x 17 mesh with 48 rows and 1500 columns: 25
+// million workgroups).
 template <bool kMixed, bool kNear>
 void launch_regions(const WakeTask *dt, int k, int forms, int blocks, double *part,
                     hipStream_t s) {
   const double *lines = part;
   const int n1 = kNear ? LineSize<1>::kThreads : kThreads;
   const int n2 = kNear ? LineSize<2>::kThreads : kThreads;
-  launch_blocks(blocks, [&](int first, dim3 g) {
+  launch_blocks(blocks, n2 > n1 ? n2 : n1, [&](int first, unsigned g) {
     if (forms & kFormPhases)
-      hipLaunchKernelGGL((wake_phase_batched_kernel<kMixed, kNear>), g, dim3(kThreads), 0, s, dt,
+      hipLaunchKernelGGL((wake_phase_batched_kernel<kMixed, kNear>), dim3(g), dim3(kThreads), 0, s, dt,
                          k, first, part);
     if (forms & kFormLine1)
-      hipLaunchKernelGGL((wake_line_batched_kernel<kMixed, kNear, 1>), g, dim3(n1), 0, s, dt, k,
+      hipLaunchKernelGGL((wake_line_batched_kernel<kMixed, kNear, 1>), dim3(g), dim3(n1), 0, s, dt, k,
                          first, lines, part);
     if (!kMixed && (forms & kFormLine2))
-      hipLaunchKernelGGL((wake_line_batched_kernel<false, kNear, 2>), g, dim3(n2), 0, s, dt, k,
+      hipLaunchKernelGGL((wake_line_batched_kernel<false, kNear, 2>), dim3(g), dim3(n2), 0, s, dt, k,
                          first, lines, part);
   });
 }
@@ -1509,8 +1498,8 @@ extern "C" int dfcsr_wake_mesh(const DfcsrHistory *hist, const DfcsrLattice *lat
                        (const double *)part, part);
   } else {
     const auto launch = [&](auto kernel, int64_t blocks) {
-      launch_blocks(blocks, [&](int first, dim3 g) {
-        hipLaunchKernelGGL(kernel, g, dim3(kThreads), 0, s, T, first, part);
+      launch_blocks(blocks, kThreads, [&](int first, unsigned g) {
+        hipLaunchKernelGGL(kernel, dim3(g), dim3(kThreads), 0, s, T, first, part);
       });
     };
     const bool skip = far_skip(*hist, pl);

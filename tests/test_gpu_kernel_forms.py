@@ -251,6 +251,37 @@ def test_regrid_many_jobs(K, ws, jobs):
         assert a.any() and torch.equal(a, b)
 
 
+def test_grids_of_many_launches(K, ws):
+    """An interp grid of more tiles (re-grid) and rows (span table) than one
+    launch's threads can hold: a slice of two by two points, whose fields are
+    bilinear, on 140 million x rows, within three float32 roundings; spans of
+    rows at either end, and none between."""
+    from pydfcsr_amd import _lib
+    lib, Xi, Zi = _lib.load(), 140_000_000, 2
+    f = np.random.default_rng(0).normal(0.0, 1.0, (5, 2, 2))
+    cells = torch.zeros((1, Xi, Zi + 1, 5), dtype=torch.float32, device=DEV)
+    K.regrid(_t(f), 20, [(0, 0, 2, 2, -1.0, 1.0, -1.0, 1.0)], None, None, Xi, Zi, -1.0, 1.0, -1.0,
+             1.0, ws, cells32=cells)
+    for a in (0, 5_000_001, 5_782_280, 69_999_999, 134_217_728, Xi - 9):   # nine rows from a
+        y = (np.arange(a, a + 9) / (Xi - 1))[:, None]
+        for z in range(3):
+            ref = (1 - y) * f[:, 0, min(z, 1)] + y * f[:, 1, min(z, 1)]
+            got = cells[0, a:a + 9, z].cpu().numpy()
+            assert np.abs(got - ref).max() <= 3 * 2.0 ** -24 * np.abs(f).max(), (a, z)
+    Xi = 20_000_000
+    cells = cells.view(-1)[:Xi * 15].view(1, Xi, 3, 5).zero_()
+    hot = [0, 7, 3_222_784, 16_777_215, Xi - 1]
+    for k, x in enumerate(hot):
+        cells[0, x, k % 2, 0] = 1.0
+    span = torch.full((Xi, 1), 7, dtype=torch.int32, device=DEV)
+    _lib.check(lib.dfcsr_history_zspan(None, cells.data_ptr(), span.data_ptr(), Xi, Zi, 1, 0, 1, 0,
+                                       torch.cuda.current_stream().cuda_stream), "zspan")
+    ref = torch.full((Xi, 1), 0xFFFF, dtype=torch.int32, device=DEV)
+    for k, x in enumerate(hot):   # an entry joins rows x and x + 1
+        ref[max(x - 1, 0):x + 1] = (k % 2) | (k % 2) << 16
+    assert torch.equal(span, ref)
+
+
 # the smallest mesh, one that is no mesh, odd ones, the largest two wakes and
 # the largest one wake that fit the LDS whole, and meshes of which the middle is
 # held: one row too many, thin ones
